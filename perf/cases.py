@@ -1,0 +1,523 @@
+"""Timing cases of the public entry points, with inputs made from a seed and 64-bit reference results.
+
+A case is a dict of plain values; `kind` says which entry points a pass goes through:
+
+  points   one bosonic frequency of the (omega, q) loop: set_local_omega, run_points over a batch of q
+           points, get_sigma (without the EOM for a q path, as the loop runs there)
+  loop     run_loop over every omega and q of the workload
+  tangent  the same as points in tangent-linear mode, three directions (t, t', U)
+  onep     the routines around the loop: get_giw, get_nfock, get_sigma_g_loc, get_ndga
+  inverse  inverse_matrix, the drop-in for lapack_module's inverse
+  lambda   the lambda correction of a final susceptibility, from the host array to the corrected one
+
+`exact` forms the same quantities in torch's complex128 from the formulas: G by batched inverses, the
+k sums by FFT, eta by the fixed-point iteration eta <- (1 + gamma)(1 - A) + eta (1 - A), which converges
+because the vertices here keep 1 - A contracting (no value is given where it does not), and the
+derivatives by forward-mode differentiation of all that.
+"""
+from __future__ import annotations
+
+import dataclasses
+import math
+
+import numpy as np
+import torch
+
+from adga_amd import api, synth
+
+DEV = "cuda"
+
+
+# ---------------------------------------------------------------------------------------------- cases
+def _points(name, n, nk, iwf, iwb, omega, npts, precision, box=0, vq=0.0, bubble_range=0, extra=0, path=False,
+            kind="points"):
+    c = {"kind": kind, "n": n, "nkx": nk[0], "nky": nk[1], "nkz": nk[2], "iwf": iwf, "iwb": iwb, "omega": omega,
+         "npts": npts, "precision": precision, "box": box, "vq": vq, "bubble_range": bubble_range, "extra": extra,
+         "path": path}
+    if name:
+        c["name"] = name
+    return c
+
+
+def listed():
+    return [
+        # the smallest call: the 1-orbital workload's BSE matrix (N = 40) through the drop-in inverse, which
+        # a caller with main.F90 unchanged makes twice per point; latency only
+        {"name": "inverse_n40", "kind": "inverse", "n": 40},
+        # the same at the 3-orbital workload's size: one matrix at a time
+        {"name": "inverse_n1080", "kind": "inverse", "n": 1080},
+        # the whole loop of the 1-orbital 8^3 workload, N = 40: 5632 points, eleven omega, small matrices
+        {"name": "loop_n1_k8_fp64", "kind": "loop", "n": 1, "nkx": 8, "nky": 8, "nkz": 8, "iwf": 20, "iwb": 5,
+         "precision": "fp64"},
+        # odd grid and box, a part of the q list, V(q) and the large bubble range with its tail: N = 136
+        _points("ragged_n2_vq_refined", 2, (11, 9, 7), 17, 3, 1, 301, "refined", vq=0.4, bubble_range=2, extra=13),
+        # the reference's published run: susceptibility along a 41-point q path of a 20^3 grid, N = 540
+        _points("qpath_n540_fp64", 3, (20, 20, 20), 30, 0, 0, 41, "fp64", path=True),
+        # the main path: 3 orbitals, 20^3 k, N = 1080, a batch of q points at one omega, both precisions
+        _points("t2g_n1080_refined", 3, (20, 20, 20), 60, 15, 2, 1500, "refined"),
+        _points("t2g_n1080_fp64", 3, (20, 20, 20), 60, 15, -7, 700, "fp64"),
+        # the shrinking box of the 5-orbital workload: its largest matrices and its smallest
+        _points("d5_n4000_refined", 5, (16, 16, 16), 80, 20, 0, 48, "refined"),
+        _points("d5_n2000_fp64", 5, (16, 16, 16), 80, 20, 20, 64, "fp64", box=40),
+        # derivatives in t, t', U on the 12^3 grid, N = 720
+        _points("tangent_n720", 3, (12, 12, 12), 40, 10, 0, 500, "fp64", kind="tangent"),
+        # one-particle routines on the 20^3 grid with the published run's 2000 frequencies
+        {"name": "onep_k20_iw2000", "kind": "onep", "n": 3, "nkx": 20, "nky": 20, "nkz": 20, "iwmax": 2000, "iwf": 60},
+        # lambda correction over every (omega, q) of the 12^3 grid with 21 omega
+        {"name": "lambda_k12", "kind": "lambda", "n": 3, "nqp": 1728, "iwb": 10},
+    ]
+
+
+def _log_int(rng, lo, hi):
+    return int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+
+
+def draw(rng):
+    kind = rng.choice(["points"] * 6 + ["path", "loop", "tangent", "onep", "inverse", "inverse", "lambda"])
+    if kind == "inverse":
+        return {"kind": "inverse", "n": _log_int(rng, 8, 1400)}
+    if kind == "lambda":
+        return {"kind": "lambda", "n": rng.randint(1, 4), "nqp": _log_int(rng, 60, 3000), "iwb": rng.randint(1, 10)}
+    if kind == "onep":
+        nk = [rng.randint(4, 20) for _ in range(3)]
+        return {"kind": "onep", "n": rng.randint(1, 5), "nkx": nk[0], "nky": nk[1], "nkz": nk[2],
+                "iwmax": _log_int(rng, 60, 1500), "iwf": rng.randint(3, 40)}
+    if kind == "loop":
+        return {"kind": "loop", "n": rng.randint(1, 2), "nkx": rng.randint(3, 8), "nky": rng.randint(3, 8),
+                "nkz": rng.randint(1, 8), "iwf": rng.randint(4, 22), "iwb": rng.randint(1, 5),
+                "precision": rng.choice(["fp64", "refined"])}
+    n = rng.choice([1, 2, 3, 3, 3, 4, 5])
+    size = _log_int(rng, 30, 720 if kind == "tangent" else 2400)          # BSE size, about
+    iwf = max(2, min(80, int(round(size / (2 * n * n)))))
+    if kind == "path":
+        e = 2 * rng.randint(2, 10)
+        return _points("", n, (e, e, e), iwf, rng.randint(0, 2), 0, len(synth.q_path((e, e, e))),
+                       rng.choice(["fp64", "refined"]), path=True)
+    top = 12 if n >= 4 else 20
+    nk = tuple(rng.randint(3, top) for _ in range(3))
+    iwb = rng.randint(0, 12)
+    size = 2 * n * n * iwf
+    most = int(min(nk[0] * nk[1] * nk[2], 4e12 / (2 * 8 / 3 * size ** 3 + 1e6), 40e9 / (32.0 * size ** 2)))
+    npts = _log_int(rng, 1, max(1, min(most, 2000)))
+    if kind == "tangent":
+        return _points("", n, nk, iwf, iwb, rng.randint(-iwb, iwb), npts, "fp64", kind="tangent")
+    box = rng.randint(max(1, iwf // 2), iwf) if rng.random() < 0.3 else 0
+    br = rng.choice([0, 0, 0, 1, 2])
+    return _points("", n, nk, iwf, iwb, rng.randint(-iwb, iwb), npts, rng.choice(["refined", "refined", "fp64"]),
+                   box=box, vq=0.4 if rng.random() < 0.25 else 0.0, bubble_range=br,
+                   extra=rng.randint(4, 30) if br else 0)
+
+
+# ---------------------------------------------------------------------------------------------- inputs
+def _workload(case, seed):
+    """The case's synthetic workload; hopping and U vary by a few percent with the seed."""
+    r = np.random.default_rng([seed, 77])
+    n = case["n"]
+    a, b = 1.0 + 0.05 * r.uniform(-1, 1, 2)
+    par = {1: dict(model="sc1", U=2.0 * b, J=0.0, t=0.25 * a),
+           3: dict(model="t2g", U=5.0 * b, J=0.75, t=-0.26 * a, tp=-0.08 * a)}.get(
+               n, dict(model="rand5", U=4.0 * b, J=0.6, t=0.15 * a))
+    iwf, iwb = case["iwf"], case.get("iwb", 0)
+    return synth.Workload(name="case", n=n, nk=(case["nkx"], case["nky"], case["nkz"]), iwfmax_small=iwf,
+                          iwbmax_small=iwb, beta=10.0, seed=seed % (1 << 31), iwmax=iwf + iwb + case.get("extra", 0),
+                          q_list="path" if case.get("path") else "vol", vq=case.get("vq", 0.0),
+                          bubble_range=case.get("bubble_range", 0), **par)
+
+
+def _chi_loc(inp, iwb, box, seed):
+    """chi_loc of both channels (N, N): the local bubble on the diagonal plus Hermitian noise, as
+    synth.chi_loc forms it, for a box of its own and with the noise drawn on the GPU."""
+    n = inp.n
+    N, off = 2 * box * n * n, inp.iwmax
+    w = np.arange(-box, box) + off
+    diag = (-inp.beta * inp.giw[w][:, :, None] * inp.giw[w - iwb][:, None, :]).reshape(-1)
+    out = []
+    for ch in range(2):
+        g = torch.Generator(device=DEV)
+        g.manual_seed((seed * 2 + ch) * 64 + iwb + 32)
+        x = torch.randn(N, N, dtype=torch.complex128, device=DEV, generator=g) * (math.sqrt(2.0) * 0.5e-3)
+        x += x.mH.clone()
+        x.diagonal().add_(torch.from_numpy(diag).to(DEV))
+        out.append(x.T.contiguous().cpu().numpy().T)  # Fortran order
+    return out
+
+
+def _dchi_loc(inp, tan, iwb, box, seed):
+    """d chi_loc / d(t, t', U), (N, N, 3): the local bubble's derivative and a symmetric one of the vertex."""
+    d = synth.dchi_loc(inp, tan, iwb, box)
+    x = np.random.default_rng([seed, 13]).standard_normal(d.shape[:2] + (1,)) * 1e-3
+    return d + (x + x.transpose(1, 0, 2)) * np.array([1.0, -0.5, 0.2])
+
+
+def _iq(case, nqp):
+    """The first npts positions of the q list, 1-based."""
+    return np.arange(1, min(case["npts"], nqp) + 1, dtype=np.int32)
+
+
+def _inverse_input(case, seed):
+    n = case["n"]
+    r = np.random.default_rng([seed, n])
+    x = r.normal(size=(n, n)) + 1j * r.normal(size=(n, n))
+    # a BSE matrix: the identity plus a vertex part of moderate norm
+    return np.asfortranarray(np.eye(n) + 0.35 / math.sqrt(n) * x)
+
+
+def _onep_input(case, seed):
+    """The workload's one-particle data with a Hubbard-I-like self-energy over case["iwmax"] frequencies;
+    giw is a placeholder that get_giw fills."""
+    wl = dataclasses.replace(_workload(dict(case, iwb=0), seed), iwmax=case["iwf"])
+    inp = synth.build_inputs(wl)
+    r = np.random.default_rng([seed, 5])
+    m, n = case["iwmax"], case["n"]
+    m = max(m, case["iwf"])
+    nu = math.pi * (2 * np.arange(-m, m) + 1) / wl.beta
+    h, s, e = (wl.U * (0.5 + 0.02 * r.normal(size=n)), wl.U * (0.5 + 0.02 * r.normal(size=n)),
+               0.05 * wl.U * r.normal(size=n))
+    siw = np.asfortranarray(h + s ** 2 / (1j * nu[:, None] - e))
+    return dataclasses.replace(inp, siw=siw, giw=np.ones_like(siw), wl=dataclasses.replace(wl, iwmax=m))
+
+
+def _lambda_input(case, seed):
+    r = np.random.default_rng([seed, 9])
+    n, nqp, nw = case["n"], case["nqp"], 2 * case["iwb"] + 1
+    n2 = n * n
+    w = np.abs(np.arange(nw) - case["iwb"])
+    size = (0.4 + 0.6 * r.random((nqp * nw))) / (1.0 + np.repeat(w, nqp) ** 2)
+    chi = 0.02 * (r.standard_normal((nqp * nw, n2, n2)) + 1j * r.standard_normal((nqp * nw, n2, n2)))
+    chi *= size[:, None, None]
+    d = np.arange(n) * (n + 1)
+    chi[:, d, d] += size[:, None]
+    loc = np.zeros((nw, n2, n2), dtype=np.complex128)
+    loc[:, d, d] = (0.55 / (1.0 + w ** 2))[:, None]
+    return chi.transpose(2, 1, 0), loc.transpose(2, 1, 0), 10.0
+
+
+def prepare(case, seed):
+    kind = case["kind"]
+    if kind == "inverse":
+        return {"kind": kind, "m": _inverse_input(case, seed)}
+    if kind == "lambda":
+        chi, loc, beta = _lambda_input(case, seed)
+        return {"kind": kind, "chi": chi, "loc": loc, "beta": beta, "nqp": case["nqp"]}
+    if kind == "onep":
+        inp = _onep_input(case, seed)
+        ctx = api.Context(inp)
+        inp = dataclasses.replace(inp, giw=ctx.get_giw())
+        box = max(1, case["iwf"] // 4)
+        ctx.set_local_omega(0, *_chi_loc(inp, 0, box, seed), box)
+        ctx.run_points(np.array([inp.wl.nqp // 2 + 1], dtype=np.int32), "fp64")  # a self-energy to sum over
+        return {"kind": kind, "ctx": ctx}
+    wl = _workload(case, seed)
+    inp = synth.build_inputs(wl)
+    if kind == "loop":
+        pts = [(w, q) for w in range(-wl.iwbmax_small, wl.iwbmax_small + 1) for q in range(wl.nqp)]
+        chi = {w: _chi_loc(inp, w, wl.iwfmax_small, seed) for w in range(-wl.iwbmax_small, wl.iwbmax_small + 1)}
+        return {"kind": kind, "ctx": api.Context(inp, batch=wl.nqp), "points": pts, "chi": chi,
+                "precision": case["precision"]}
+    iq = _iq(case, wl.nqp)
+    box = case["box"] or wl.iwfmax_small
+    ctx = api.Context(inp, batch=len(iq))
+    st = {"kind": kind, "ctx": ctx, "iq": iq, "omega": case["omega"], "box": box, "precision": case["precision"],
+          "eom": wl.do_eom, "chi": _chi_loc(inp, case["omega"], box, seed)}
+    if kind == "tangent":
+        tan = synth.tangents(inp)
+        ctx.set_tangents(tan)
+        st["dchi"] = np.asfortranarray(_dchi_loc(inp, tan, case["omega"], box, seed))
+    return st
+
+
+def run(s):
+    kind = s["kind"]
+    if kind == "inverse":
+        return api.inverse_matrix(s["m"])[0]
+    if kind == "lambda":
+        with api.Lambda(s["chi"], s["loc"], s["beta"], s["nqp"]) as lam:
+            target = lam.target()
+            value, _ = lam.solve()
+            return {"target": target, "lambda": value, "chi": lam.chi(value)}
+    ctx = s["ctx"]
+    if kind == "onep":
+        giw, nf = ctx.get_giw(), ctx.get_nfock()
+        sl, gl = ctx.get_sigma_g_loc()
+        ndk, nd = ctx.get_ndga()
+        return {"giw": giw, "n_fock": nf, "sigma_loc": sl, "gloc": gl, "n_dga_k": ndk, "n_dga": nd}
+    ctx.reset_sigma()
+    if kind == "loop":
+        out = api.run_loop(ctx, s["points"], lambda w, c: s["chi"][w][0 if c == "dens" else 1], s["precision"])
+        loc = {k: np.stack([out[k][w] for w in sorted(s["chi"])]) for k in ("chi_loc_d", "chi_loc_m", "bubble_loc")}
+        return {**{k: out[k] for k in ("chi_d", "chi_m", "bubble_nl", "status", "sigma_nl", "sigma_dmft")}, **loc}
+    res = {}
+    res["chi_loc_d"], res["chi_loc_m"], res["bubble_loc"] = ctx.set_local_omega(s["omega"], *s["chi"], s["box"])
+    if kind == "tangent":
+        t = ctx.set_local_omega_tangent(s["dchi"], s["dchi"])
+        res["dchi_loc_d"], res["dchi_loc_m"], res["dbubble_loc"] = t
+        res.update(ctx.run_points_tangent(s["iq"]))
+    else:
+        r = ctx.run_points(s["iq"], s["precision"])
+        res.update({k: r[k] for k in ("chi_d", "chi_m", "bubble_nl", "status")})
+    if s["eom"]:
+        res["sigma_nl"], res["sigma_dmft"], res["sigma_hf"] = ctx.get_sigma()
+    if kind == "tangent":
+        res["dsigma_nl"] = ctx.get_sigma_tangent()
+    return res
+
+
+def work(case):
+    kind, n = case["kind"], case["n"]
+    n2 = n * n
+    if kind == "inverse":
+        return {"bytes": 32 * n2, "flops": 8 * n ** 3}
+    if kind == "lambda":
+        p = case["nqp"] * (2 * case["iwb"] + 1)
+        return {"bytes": 16 * p * (n2 * n2 + 1), "flops": 200 * p}
+    nkp = case["nkx"] * case["nky"] * case["nkz"]
+    if kind == "onep":
+        sig = 16 * n2 * 2 * case["iwf"] * nkp
+        inv = 4 * nkp * max(case["iwmax"], case["iwf"])
+        return {"bytes": 2 * sig + 16 * nkp * n2 * 3 + 16 * case["iwmax"] * (2 * n + 2 * n2), "flops": inv * 20 * n ** 3}
+    N = 2 * n2 * (case.get("box") or case["iwf"])
+    if kind == "loop":
+        nw, npts, chans = 2 * case["iwb"] + 1, nkp * (2 * case["iwb"] + 1), 1
+    else:
+        nw, npts, chans = 1, case["npts"], 4 if kind == "tangent" else 1
+    sig = 0 if case.get("path") else 16 * n2 * 2 * case["iwf"] * nkp * chans
+    bse = 2 * npts * (8 / 3 * N ** 3 + chans * 8 * N * N * n2)
+    return {"bytes": nw * 32 * N * N + 16 * n2 * nkp + 48 * npts * n2 * n2 * chans + sig, "flops": bse}
+
+
+# ---------------------------------------------------------------------------------------------- 64-bit results
+def _t(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).to(DEV)
+
+
+def _g(p, a, iws):
+    """G(k, nu) for the frequencies iws as (nw, nkx, nky, nkz, n, n)."""
+    n = p["n"]
+    nu = math.pi * (2 * torch.tensor(list(iws), dtype=torch.float64, device=DEV) + 1) / p["beta"]
+    s = a["siw"][torch.tensor([w + p["iwmax"] for w in iws], device=DEV)]
+    diag = 1j * nu[:, None] + a["mu"] - a["dc"] - s
+    m = torch.diag_embed(diag)[:, None] - a["hk"].permute(2, 0, 1)[None]
+    return torch.linalg.inv(m).reshape(len(iws), *p["nk"], n, n)
+
+
+def _back(x):
+    """x(-R) on the three grid axes."""
+    return torch.roll(torch.flip(x, (0, 1, 2)), (1, 1, 1), (0, 1, 2))
+
+
+def _bubble_fields(p, ga, gb):
+    """-beta/nkp sum_k ga(k)_il gb(k - q)_k'j for every q: (nkp, n2, n2) in the compound indices (ij), (lk')."""
+    n, n2 = p["n"], p["n"] ** 2
+    A, B = torch.fft.fftn(ga, dim=(0, 1, 2)), _back(torch.fft.fftn(gb, dim=(0, 1, 2)))
+    c = torch.einsum("xyzil,xyzkj->xyzijlk", A, B)
+    return torch.fft.ifftn(c, dim=(0, 1, 2)).reshape(-1, n2, n2) * (-p["beta"] / p["nkp"])
+
+
+def _omega(p, a):
+    """Every output of one omega, as tensors in the entry points' layouts; None where the iteration stalls."""
+    n, n2, box, iwb = p["n"], p["n"] ** 2, p["box"], p["omega"]
+    beta, nf = p["beta"], 2 * p["box"]
+    N, npts = n2 * nf, len(p["iq"])
+    ws = range(-box, box)
+    at = lambda w: torch.tensor([v + p["iwmax"] for v in w], device=DEV)  # noqa: E731
+    loc = lambda w: -beta * (a["giw"][at(w)][:, :, None] * a["giw"][at(w) - iwb][:, None, :]).reshape(len(w), n2)  # noqa: E731
+    w0 = loc(ws)
+    wi = 1.0 / w0
+    eye = torch.eye(n2, dtype=torch.complex128, device=DEV)
+    q = torch.tensor([int(p["q0"][i - 1]) for i in p["iq"]], device=DEV)
+    chi0 = torch.stack([_bubble_fields(p, _g(p, a, [w])[0], _g(p, a, [w - iwb])[0])[q] for w in ws], 1)
+    big, outer = w0.sum(0), None
+    if p["range"]:
+        lo = [w for w in range(-p["K"], p["K"]) if not -box <= w < box]
+        big = loc(range(-p["K"], p["K"])).sum(0)
+        outer = 0
+        for w in lo:
+            outer = outer + _bubble_fields(p, _g(p, a, [w])[0], _g(p, a, [w - iwb])[0])[q]
+    bloc = torch.diag(big) / beta ** 2
+    bsum = chi0.sum(1) if outer is None else chi0.sum(1) + outer
+    out = {"bubble_loc": bloc if p["range"] != 2 else None, "bubble_nl": (bsum / beta ** 2 - bloc).permute(1, 2, 0)}
+    S = chi0 * wi[None, :, None, :] - eye
+    chiw = torch.diag_embed(w0)
+    dot = lambda x, y: torch.einsum("...sdi,...dit->...st", x, y) / beta ** 2  # noqa: E731
+    eta, gamq = {}, None
+    for r in "dm":
+        x = a["x" + r]
+        C = 0.5 * (x + x.T) * wi.reshape(-1)[None, :]
+        C = C - torch.eye(N, dtype=torch.complex128, device=DEV)
+        gam = C.reshape(nf, n2, N).sum(0)
+        opg = gam + eye.repeat(1, nf)
+        W = None
+        if r == "d" and a["vq"] is not None:
+            W = (2.0 / beta ** 2) * (chi0 @ a["vq"][torch.tensor(p["iq"] - 1, device=DEV).long()][:, None])
+
+        def left(y):  # y (1 - A) for y (npts, n2, N)
+            y = y.reshape(-1, n2, nf, n2)
+            z = torch.einsum("psdi,pdij->psdj", y, S).reshape(npts, n2, N) @ C
+            return z if W is None else z + torch.einsum("psdi,pdij->psj", y, W) @ opg
+
+        b = left(opg.expand(npts, n2, N).contiguous())
+        e, last = b, None
+        for _ in range(400):
+            new = b + left(e)
+            step = float((new - e).detach().abs().max() / new.detach().abs().max())
+            e = new
+            if not step < 1e3:
+                return None
+            if last is not None and step < 1e-14 and step > 0.5 * last or step == 0.0:
+                break
+            last = step
+        else:
+            return None
+        eta[r] = e
+        g4 = gam.reshape(n2, nf, n2)
+        out["chi_loc_" + r] = dot(g4, chiw)
+        out["chi_" + r] = (dot(g4, chi0 - chiw) + dot(e.reshape(npts, n2, nf, n2), chi0)).permute(1, 2, 0)
+        if r == "d":
+            gd = gam
+            gamq = S.permute(0, 2, 1, 3).reshape(npts, n2, N) @ C
+    if not p["eom"]:
+        return out
+    f = 1.0 / (beta * p["nqp"])
+    u, ut = a["u"], a["ut"]
+    uw = u - 0.5 * ut
+    m = 1.5 * f * (ut @ eta["m"]) + f * (u @ gamq) - f * (uw @ eta["d"])
+    if a["vq"] is not None:
+        v = a["vq"][torch.tensor(p["iq"] - 1, device=DEV).long()]
+        m = m - f * (v @ eta["d"]) - f * (v @ gd)
+    m = m.reshape(npts, n, n, nf, n, n)  # (i j)(nu l k')
+    half = []
+    for w in range(box):
+        grid = torch.zeros(p["nkp"], n ** 4, dtype=torch.complex128, device=DEV)
+        grid = grid.index_copy(0, q, m[:, :, :, box + w].reshape(npts, -1)).reshape(*p["nk"], n, n, n, n)
+        F = torch.fft.fftn(grid, dim=(0, 1, 2))
+        G = torch.fft.fftn(_g(p, a, [w - iwb])[0], dim=(0, 1, 2))
+        half.append(torch.fft.ifftn(torch.einsum("xyzijlk,xyzjk->xyzil", F, G), dim=(0, 1, 2)).reshape(-1, n, n))
+    z = torch.zeros_like(half[0])
+    half = half + [z] * (p["iwf"] - box)
+    pos = torch.stack(half, 0)                                   # (nu, k, i, l)
+    sig = torch.cat([pos.flip(0).mH, pos], 0).permute(2, 3, 0, 1)
+    out["sigma_nl"] = sig
+    dm = torch.zeros(p["iwf"], n, n, dtype=torch.complex128, device=DEV)
+    if 1 in p["iq"]:
+        md = (-1.0 / beta) * (u @ gd).reshape(n, n, nf, n, n)[:, :, box:]
+        gl = a["giw"][at(range(box)) - iwb]
+        dm = torch.cat([torch.einsum("ikdlk,dk->dil", md, gl), dm[: p["iwf"] - box]], 0)
+        both = torch.cat([dm.flip(0).mH, dm], 0)
+        if iwb == 0:
+            u4 = u.reshape(n, n, n, n)
+            h = torch.einsum("iijj,j->i", 2.0 * u4, a["ndmft"]) - torch.einsum("ijij,j->i", u4, a["ndmft"])
+            # added before the negative frequencies are filled from the positive ones
+            both = both + torch.cat([torch.diag(h.conj()).expand(p["iwf"], n, n),
+                                     torch.diag(h).expand(p["iwf"], n, n)], 0)
+    else:
+        both = torch.cat([dm, dm], 0)
+    out["sigma_dmft"] = both.permute(1, 2, 0)
+    return out
+
+
+def _arrays(inp, chi):
+    a = {"hk": _t(inp.hk), "siw": _t(inp.siw), "giw": _t(inp.giw), "dc": _t(inp.dc[0]),
+         "mu": torch.tensor(complex(inp.mu), dtype=torch.complex128, device=DEV), "u": _t(inp.u), "ut": _t(inp.u_tilde),
+         "ndmft": _t(inp.n_dmft), "xd": _t(chi[0]), "xm": _t(chi[1]),
+         "vq": None if inp.v_q is None else _t(inp.v_q.transpose(2, 0, 1))}
+    return a
+
+
+def _par(inp, omega, box, iq):
+    wl = inp.wl
+    return {"n": wl.n, "nk": wl.nk, "nkp": wl.nkp, "beta": inp.beta, "iwmax": inp.iwmax, "iwf": wl.iwfmax_small,
+            "box": box, "omega": omega, "iq": iq, "q0": inp.q_data - 1, "nqp": wl.nqp, "eom": wl.do_eom,
+            "range": wl.bubble_range, "K": inp.iwmax - wl.iwbmax_small}
+
+
+def _host(out):
+    return {k: None if v is None else v.detach().resolve_conj().cpu().numpy() for k, v in out.items()}
+
+
+def exact(case, seed):
+    kind = case["kind"]
+    if kind == "inverse":
+        return np.linalg.inv(_inverse_input(case, seed))
+    if kind == "lambda":
+        chi, loc, beta = _lambda_input(case, seed)
+        d = np.arange(case["n"]) * (case["n"] + 1)
+        phys = chi[np.ix_(d, d)].sum(axis=(0, 1))
+        target = float(loc[np.ix_(d, d)].sum(axis=(0, 1)).sum().real / beta)
+        f = lambda x: float((phys / (1 + x * phys)).sum().real) / (beta * case["nqp"]) - target  # noqa: E731
+        pole = -1.0 / phys[case["iwb"] * case["nqp"]:(case["iwb"] + 1) * case["nqp"]].real.max()
+        lo, hi = pole + 1e-9, 1.0
+        while f(hi) > 0:
+            hi *= 2
+        for _ in range(200):
+            mid = 0.5 * (lo + hi)
+            lo, hi = (mid, hi) if f(mid) > 0 else (lo, mid)
+        x = 0.5 * (lo + hi)
+        return {"target": target, "lambda": x, "chi": phys / (1 + x * phys)}
+    if kind == "onep":
+        return _exact_onep(case, seed)
+    wl = _workload(case, seed)
+    inp = synth.build_inputs(wl)
+    if kind == "loop":
+        per = []
+        for w in range(-wl.iwbmax_small, wl.iwbmax_small + 1):
+            iq = np.arange(1, wl.nqp + 1)
+            per.append(_omega(_par(inp, w, wl.iwfmax_small, iq), _arrays(inp, _chi_loc(inp, w, wl.iwfmax_small, seed))))
+            if per[-1] is None:
+                return None
+        per = [_host(o) for o in per]
+        out = {k: np.concatenate([o[k] for o in per], axis=2) for k in ("chi_d", "chi_m", "bubble_nl")}
+        out.update({k: sum(o[k] for o in per) for k in ("sigma_nl", "sigma_dmft")})
+        out.update({k: np.stack([o[k] for o in per]) for k in ("chi_loc_d", "chi_loc_m", "bubble_loc")})
+        return {**out, "status": None}
+    iq = _iq(case, wl.nqp)
+    box = case["box"] or wl.iwfmax_small
+    chi = _chi_loc(inp, case["omega"], box, seed)
+    p, a = _par(inp, case["omega"], box, iq), _arrays(inp, chi)
+    if kind == "points":
+        out = _omega(p, a)
+        if out is None:
+            return None
+        out = {**_host(out), "status": None}
+        if wl.do_eom:
+            zero = np.zeros((wl.n, wl.n, wl.nkp), dtype=np.complex128)
+            out["sigma_hf"] = None if case["vq"] and case["omega"] == 0 else zero
+        return out
+    tan = synth.tangents(inp)
+    dchi = _t(_dchi_loc(inp, tan, case["omega"], box, seed))
+    keys = ("hk", "siw", "giw", "mu", "u", "ut", "xd", "xm")
+    grads, out = [], None
+    import torch.autograd.forward_ad as fwd
+    for d in range(3):
+        da = {"hk": _t(tan.dhk[..., d]), "siw": _t(tan.dsiw[..., d]), "giw": _t(tan.dgiw[..., d]),
+              "mu": torch.tensor(complex(tan.dmu[d]), dtype=torch.complex128, device=DEV), "u": _t(tan.du[..., d]),
+              "ut": _t(tan.du_tilde[..., d]), "xd": dchi[..., d].contiguous(), "xm": dchi[..., d].contiguous()}
+        with fwd.dual_level():
+            o = _omega(p, {**a, **{k: fwd.make_dual(a[k], da[k]) for k in keys}})
+            if o is None:
+                return None
+            pair = {k: fwd.unpack_dual(v) for k, v in o.items()}
+            out = {k: v.primal for k, v in pair.items()}
+            grads.append({k: v.tangent for k, v in pair.items()})
+    res = _host(out)
+    for k in ("chi_d", "chi_m", "bubble_nl", "chi_loc_d", "chi_loc_m", "bubble_loc", "sigma_nl"):
+        res["d" + k] = torch.stack([g[k] for g in grads], -1).resolve_conj().cpu().numpy()
+    return {**res, "status": None, "sigma_hf": np.zeros((wl.n, wl.n, wl.nkp), dtype=np.complex128)}
+
+
+def _exact_onep(case, seed):
+    """k and frequency sums of G; what depends on the self-energy the context has accumulated has no value."""
+    inp = _onep_input(case, seed)
+    p, a = _par(inp, 0, 1, np.ones(1, dtype=int)), _arrays(inp, (np.zeros((1, 1)), np.zeros((1, 1))))
+    n, m, nkp = case["n"], inp.iwmax, inp.wl.nkp
+    giw = torch.zeros(2 * m, n, dtype=torch.complex128, device=DEV)
+    occ = torch.zeros(nkp, n, n, dtype=torch.float64, device=DEV)
+    step = max(1, 1_000_000 // nkp)
+    for w in range(0, m, step):
+        ws = range(w, min(m, w + step))
+        g = _g(p, a, ws).reshape(len(ws), nkp, n, n)
+        giw[m + w:m + w + len(ws)] = torch.diagonal(g, dim1=2, dim2=3).mean(1)
+        occ += g.real.sum(0)
+    giw[:m] = giw[m:].flip(0).conj()
+    occ = occ * (2.0 / inp.beta) + 0.5 * torch.eye(n, dtype=torch.float64, device=DEV)
+    return {"giw": giw.cpu().numpy(), "n_fock": occ.to(torch.complex128).cpu().numpy(), "sigma_loc": None, "gloc": None,
+            "n_dga_k": None, "n_dga": None}
