@@ -75,7 +75,7 @@ def _log_int(rng, lo, hi):
 def _noise(rng):
     """Scale of the vertex: the repository's workloads' in two of three draws, else up to strong ones (1 - A is
     about 1e-3 at 1e-3 and of order one at 1)."""
-    return 1e-3 if rng.random() < 0.66 else math.exp(rng.uniform(math.log(1e-3), 0.0)))
+    return 1e-3 if rng.random() < 0.66 else math.exp(rng.uniform(math.log(1e-3), 0.0))
 
 
 def draw(rng):
