@@ -45,7 +45,7 @@ def _dptr(a):
 
 class Context:
     def __init__(self, inp, batch=None, refine_tol=None, refine_maxit=None, bubble=None, eom=None, lu_streams=None,
-                 do_eom=None, fallback=None, bubble_range=None):
+                 do_eom=None, fallback=None, bubble_range=None, series=None):
         wl = inp.wl
         self.n = wl.n
         self.n2 = wl.n * wl.n
@@ -77,7 +77,7 @@ class Context:
             bubble_range = getattr(wl, "bubble_range", 0) or None  # the debug option "Bubble" (+ the tail)
         for key, v in (("batch", batch), ("refine_tol", refine_tol), ("refine_maxit", refine_maxit),
                        ("bubble", bubble), ("eom", eom), ("lu_streams", lu_streams), ("do_eom", int(bool(do_eom))),
-                       ("fallback", fallback), ("bubble_range", bubble_range)):
+                       ("fallback", fallback), ("bubble_range", bubble_range), ("series", series)):
             if v is not None:
                 self._check(lib.adga_set_option(self.h, key.encode(), float(v)))
 

@@ -22,9 +22,11 @@ void launch_local(const Geom& g, int iwb, const z64* giw, const z64* xd, const z
 void launch_bubble(const Geom& g, int iwb, int npts, const int* qidx, const z64* gt, z64* chi0q, hipStream_t s,
                    const z64* gt2 = nullptr, bool accumulate = false);
 // Out = C_ch^T Z_ch for the channels ch0 .. ch0 + nch - 1 (C row-major as the left operand, Z and Out in the
-// residual layouts), plus B - Y when B is given, plus Out itself when accumulate
+// residual layouts), plus B - Y when B is given, plus Out itself when accumulate; with rmax each matrix's
+// max |Out| as the bits of a double (atomic maximum: cleared by the caller)
 void resid_gemm(const Geom& g, int npts, int ch0, int nch, const z64* cd, const z64* cm, const z64* Z, z64* Out,
-                const z64* B, const z64* Y, hipStream_t s, bool accumulate = false);
+                const z64* B, const z64* Y, hipStream_t s, bool accumulate = false,
+                unsigned long long* rmax = nullptr);
 void launch_smat(const Geom& g, int npts, const z64* chi0q, const z64* winv, z64* S, hipStream_t s);
 template <typename T>
 void launch_build(const Geom& g, int npts, int ldm, const z64* S, const z64* cd, const z64* cm, cplx<T>* M,
@@ -33,12 +35,14 @@ void launch_gamq(const Geom& g, int npts, const z64* S, const z64* cd, z64* Z, z
 // the right operand of gamma^q_d's product (S of each point in the residual product's layout)
 void launch_gamq_z(const Geom& g, int npts, const z64* S, z64* Z, hipStream_t s);
 size_t lu_inv_elems(int N);
+bool lu_supported(int N);  // whether N is in the LU's range
 std::vector<int> lu_ops_factor(int N, int W);
 // factor + forward elimination of the right-hand-side columns [N, W) only (no backward substitution)
 std::vector<int> lu_ops_factor_fwd(int N, int W);
 // the same list as lu_ops_factor written into buf (at most cap ints); returns the number of ints the list needs
 size_t lu_ops_factor_into(int N, int W, int* buf, size_t cap);
-// Events around the launches of the largest GEMM tile shape (the factorisation's dominant kernel):
+// Events around the launches of the BSE solve's dominant kernel (the factorisation's largest GEMM tile shape,
+// or the iteration's residual product):
 // mark() records one event; collect() (after the stream has completed) returns the summed
 // milliseconds of the bracketed launches and resets.
 struct LuTimer {
@@ -89,8 +93,18 @@ struct VqTerm {
 };
 void launch_rhs(const Geom& g, int npts, const z64* S, const z64* cd, const z64* cm, const z64* opgd,
                 const z64* opgm, z64* Z, z64* B, hipStream_t s, const VqTerm* vq = nullptr);
-void launch_residual(const Geom& g, int npts, const z64* S, const z64* cd, const z64* cm, const z64* B,
-                     const z64* Y, z64* Z, z64* R, double* rel, hipStream_t s, const VqTerm* vq = nullptr);
+// per-matrix norms of a batch: rel = max|R| / max|B|; bmax and rmax hold the maxima as the bits of doubles
+struct ResidNorm {
+  double* rel;
+  unsigned long long *bmax, *rmax;
+};
+// max|B| of each matrix into nrm.bmax, nrm.rmax cleared: once per right-hand side, before its residuals
+void launch_absmax_rhs(const Geom& g, int npts, const z64* B, const ResidNorm& nrm, hipStream_t s);
+void launch_add(long n, const z64* R, z64* Y, hipStream_t s);  // Y += R
+enum ResidMode { RESID_OF = 0, RESID_STEP = 1, RESID_START = 2 };
+void launch_residual(const Geom& g, int npts, const z64* S, const z64* cd, const z64* cm, const z64* B, z64* Y,
+                     z64* Z, z64* R, const ResidNorm& nrm, hipStream_t s, const VqTerm* vq = nullptr,
+                     ResidMode mode = RESID_OF, LuTimer* timer = nullptr);
 // V(q) (vq.hip): W of a batch (qpos: 0-based q list positions, vq: (n2, n2, nqp)); the density matrices'
 // term; Out_{2b} += (1 + gamma^w_d)^T (W^T X) with X = (1 + gamma^w_d)^T (Y null) or the density solution Y
 void launch_vq_w(const Geom& g, int npts, const int* qpos, const z64* vq, const z64* chi0q, z64* W, hipStream_t s);

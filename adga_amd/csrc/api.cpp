@@ -10,16 +10,31 @@ using namespace adga_host;
 
 namespace {
 
+void free_norm(adga::ResidNorm& n) {
+  dfree(n.rel); dfree(n.bmax); dfree(n.rmax);
+}
+
+void alloc_norm(adga::ResidNorm& n, size_t nmat) {
+  dalloc(&n.rel, nmat);
+  dalloc(&n.bmax, nmat);
+  dalloc(&n.rmax, nmat);
+}
+
 void free_batch(adga_ctx* c) {
   dfree(c->chi0q); dfree(c->S); dfree(c->gamq); dfree(c->Bp); dfree(c->Y); dfree(c->Z); dfree(c->R);
-  dfree(c->mt); dfree(c->chi_out); dfree(c->bub_out); dfree(c->M); dfree(c->inv); dfree(c->rel);
-  dfree(c->piv); dfree(c->info); dfree(c->qidx); dfree(c->act); dfree(c->keep);
+  dfree(c->mt); dfree(c->chi_out); dfree(c->bub_out); free_norm(c->nrm);
+  dfree(c->qidx); dfree(c->keep);
   c->cap = 0;
+}
+
+void free_lu(adga_ctx* c) {
+  dfree(c->M); dfree(c->inv); dfree(c->piv); dfree(c->info); dfree(c->act);
+  c->lu_cap = 0;
 }
 
 void free_fallback(adga_ctx* c) {
   FallbackBufs& f = c->fb;
-  dfree(f.S); dfree(f.B); dfree(f.Y); dfree(f.Z); dfree(f.R); dfree(f.M); dfree(f.inv); dfree(f.rel);
+  dfree(f.S); dfree(f.B); dfree(f.Y); dfree(f.Z); dfree(f.R); dfree(f.M); dfree(f.inv); free_norm(f.nrm);
   dfree(f.W); dfree(f.Q);
   dfree(f.piv); dfree(f.info); dfree(f.sel);
   f.cap = 0;
@@ -41,15 +56,25 @@ void ensure_batch(adga_ctx* c, int nb) {
   dalloc(&c->mt, nb * pmat);
   dalloc(&c->chi_out, 2 * nb * (size_t)g.n4);
   dalloc(&c->bub_out, nb * (size_t)g.n4);
-  dalloc((char**)&c->M, 2 * nb * (size_t)g.N * c->ldm * sizeof(z64));
-  dalloc((char**)&c->inv, 2 * nb * adga::lu_inv_elems(g.N) * sizeof(z64));
-  dalloc(&c->rel, 2 * nb);
-  dalloc(&c->piv, 2 * nb * (size_t)g.N);
-  dalloc(&c->info, 2 * nb);
+  alloc_norm(c->nrm, 2 * nb);
   dalloc(&c->qidx, nb);
-  dalloc(&c->act, 2 * nb);
   dalloc(&c->keep, nb);
   c->cap = nb;
+}
+
+// LU workspace of a batch of nb points (sized for complex128 and the largest box), apart from the rest: a
+// context whose batches all converge by fixed-point iteration never holds it
+void ensure_lu(adga_ctx* c, int nb) {
+  if (nb <= c->lu_cap) return;
+  free_lu(c);
+  nb = std::max(nb, c->cap);
+  const Geom& g = c->g;
+  dalloc((char**)&c->M, 2 * nb * (size_t)g.N * c->ldm * sizeof(z64));
+  dalloc((char**)&c->inv, 2 * nb * adga::lu_inv_elems(g.N) * sizeof(z64));
+  dalloc(&c->piv, 2 * nb * (size_t)g.N);
+  dalloc(&c->info, 2 * nb);
+  dalloc(&c->act, 2 * nb);
+  c->lu_cap = nb;
 }
 
 // V(q) workspace of a batch of nb points
@@ -208,7 +233,10 @@ const std::vector<int>& ensure_ops_rhs(adga_ctx* c, int prec) {
   return ops;
 }
 
-// FP64 re-solve of the points `pts` (batch positions) whose complex64 refinement did not converge:
+// Steps of the fixed-point iteration (series_solve) that cost about what the LU of the same batch does.
+int series_steps(const Geom& g) { return std::min(8 + g.N / (4 * g.n2), 2 + g.N / 8); }
+
+// FP64 LU solve of the points `pts` (batch positions) whose complex64 refinement or iteration did not converge:
 // their S and right-hand sides are gathered, the density and magnetic matrices rebuilt in complex128,
 // factored, solved and checked, and the solutions scattered back into the batch's Y.  Updates the
 // points' entries of relh / infoh and returns the number of matrices re-solved.
@@ -233,7 +261,7 @@ int fallback_fp64(adga_ctx* c, const std::vector<int>& pts, std::vector<double>&
     dalloc(&f.R, 2 * cap * pmat);
     dalloc(&f.M, 2 * cap * per_mat);
     dalloc(&f.inv, 2 * cap * adga::lu_inv_elems(G.N));
-    dalloc(&f.rel, 2 * cap);
+    alloc_norm(f.nrm, 2 * cap);
     dalloc(&f.piv, 2 * cap * (size_t)G.N);
     dalloc(&f.info, 2 * cap);
     dalloc(&f.sel, cap);
@@ -261,11 +289,12 @@ int fallback_fp64(adga_ctx* c, const std::vector<int>& pts, std::vector<double>&
     if (!adga::launch_lu<double>(2 * k, g.N, g.N, c->ldm, ops64, f.M, f.piv, f.inv, f.info, s) ||
         !adga::launch_lu_solve<double>(2 * k, g.N, g.n2, c->ldm, f.M, f.piv, f.inv, f.B, f.Y, false, s))
       throw HipError{hipErrorInvalidValue, "FP64 re-solve: BSE size outside the LU kernel's range"};
-    adga::launch_residual(g, k, f.S, c->cd, c->cm, f.B, f.Y, f.Z, f.R, f.rel, s, c->vq ? &fv : nullptr);
+    adga::launch_absmax_rhs(g, k, f.B, f.nrm, s);
+    adga::launch_residual(g, k, f.S, c->cd, c->cm, f.B, f.Y, f.Z, f.R, f.nrm, s, c->vq ? &fv : nullptr);
     adga::launch_gather(k, blen, f.sel, f.Y, c->Y, true, s);
     r.resize(2 * k);
     inf.resize(2 * k);
-    CK(hipMemcpyAsync(r.data(), f.rel, sizeof(double) * 2 * k, hipMemcpyDeviceToHost, s));
+    CK(hipMemcpyAsync(r.data(), f.nrm.rel, sizeof(double) * 2 * k, hipMemcpyDeviceToHost, s));
     CK(hipMemcpyAsync(inf.data(), f.info, sizeof(int) * 2 * k, hipMemcpyDeviceToHost, s));
     CK(hipStreamSynchronize(s));
     for (int j = 0; j < k; ++j)
@@ -297,9 +326,10 @@ int refine(adga_ctx* c, int nb, std::vector<double>& relh, std::vector<int>& inf
   std::vector<double> prev(nmat, INFINITY);
   int iters = 0;
   const adga::VqTerm vt{c->W, c->opgd, c->vqQ};
+  adga::launch_absmax_rhs(g, nb, c->Bp, c->nrm, s);
   for (int it = 0;; ++it) {
-    adga::launch_residual(g, nb, c->S, c->cd, c->cm, c->Bp, c->Y, c->Z, c->R, c->rel, s, c->vq ? &vt : nullptr);
-    CK(hipMemcpyAsync(relh.data(), c->rel, sizeof(double) * nmat, hipMemcpyDeviceToHost, s));
+    adga::launch_residual(g, nb, c->S, c->cd, c->cm, c->Bp, c->Y, c->Z, c->R, c->nrm, s, c->vq ? &vt : nullptr);
+    CK(hipMemcpyAsync(relh.data(), c->nrm.rel, sizeof(double) * nmat, hipMemcpyDeviceToHost, s));
     CK(hipStreamSynchronize(s));
     int nact = 0;
     for (int m = 0; m < nmat; ++m) {
@@ -334,6 +364,95 @@ int refine(adga_ctx* c, int nb, std::vector<double>& relh, std::vector<int>& inf
 }  // namespace
 
 namespace adga_host {
+// M Y = B (M = 1 - T, T Y = C^T (blockdiag(S)^T Y), with V(q) its rank-n^2 term) for the 2 nb matrices of a
+// batch by the fixed-point iteration Y <- B + T Y from Y = B, in FP64: each step is the residual R = B - M Y
+// and Y += R, so its cost is one residual product, 8 N^2 n^2 flops per matrix against 8/3 N^3 of an LU, and
+// the norm that stops it is the residual itself.  It converges where T contracts (the BSE far from an
+// instability).
+//
+// The rule: the residuals' ratio gives each matrix's contraction rho (the first one, |T B| / |B|, and the
+// later |r'| / |r| where those are worse), hence the steps ln(tol / r) / ln(rho) it still needs; the LU is
+// taken (false, Y undefined) as soon as more than one point in eight needs over series_steps() of them in
+// all - for a large batch from three products on its first 8 points, so that a batch that does not contract
+// costs next to nothing, and for a small one from its first one or two.  The steps predicted are queued
+// together: a few waits per batch.  They go on to `tol`, or until the residual stops falling; a matrix whose
+// residual then is above `accept` puts its point into `left`.  `steps`: those taken.
+bool series_solve(adga_ctx* c, int nb, double tol, double accept, const z64* B, z64* Y, std::vector<double>& relh,
+                  std::vector<int>& left, int* steps) {
+  const Geom& g = c->gw;
+  hipStream_t s = c->stream;
+  const int kmax = series_steps(g);
+  const adga::VqTerm vt{c->W, c->opgd, c->vqQ};
+  const adga::VqTerm* vtp = c->vq ? &vt : nullptr;
+  std::vector<double> rho(2 * nb, 0.0), prev;
+  std::vector<int> need(2 * nb);
+  int done = 0;  // residuals of the present batch
+  // the residuals of the first k points after `mode`, `count` - 1 more steps, and each matrix's rho and need
+  // (0: converged, or not falling; kmax + 1: not contracting)
+  auto advance = [&](int k, adga::ResidMode mode, int count) {
+    const bool start = mode == adga::RESID_START;
+    if (start) done = 0;
+    prev.assign(relh.begin(), relh.begin() + 2 * k);
+    for (int j = 0; j < count; ++j)
+      adga::launch_residual(g, k, c->S, c->cd, c->cm, B, Y, c->Z, c->R, c->nrm, s, vtp,
+                            j == 0 ? mode : adga::RESID_STEP, k == nb && !(start && j == 0) ? &c->lut : nullptr);
+    CK(hipMemcpyAsync(relh.data(), c->nrm.rel, sizeof(double) * 2 * k, hipMemcpyDeviceToHost, s));
+    CK(hipStreamSynchronize(s));
+    done += count;
+    for (int m = 0; m < 2 * k; ++m) {
+      const double r = relh[m], fell = start ? r : std::pow(r / prev[m], 1.0 / count);
+      if (start) rho[m] = fell;
+      need[m] = 0;
+      if (r <= tol) continue;
+      if (!start && r <= 8 * accept && !(fell < 0.5)) continue;  // at round-off
+      rho[m] = std::max(rho[m], fell);
+      const double n = rho[m] < 1.0 && std::isfinite(r) ? std::ceil(std::log(tol / r) / std::log(rho[m])) : INFINITY;
+      need[m] = (int)std::min(n, (double)kmax + 1);
+    }
+  };
+  auto slow = [&](int k) {  // points among the first k that need more than kmax steps in all
+    int n = 0;
+    for (int b = 0; b < k; ++b) n += done + std::max(need[2 * b], need[2 * b + 1]) > kmax;
+    return n;
+  };
+  left.clear();
+  if (steps) *steps = 0;
+  adga::launch_absmax_rhs(g, nb, B, c->nrm, s);
+  constexpr int LOOK = 8;
+  if (nb >= 8 * LOOK) {
+    advance(LOOK, adga::RESID_START, 1);
+    for (int k = 0; k < 2 && 2 * slow(LOOK) <= LOOK; ++k) advance(LOOK, adga::RESID_STEP, 1);
+    if (2 * slow(LOOK) > LOOK) return false;
+  }
+  advance(nb, adga::RESID_START, 1);
+  for (;;) {
+    if (8 * slow(nb) > nb) return false;
+    int k = 0;
+    for (int m = 0; m < 2 * nb; ++m)
+      if (done + need[m] <= kmax) k = std::max(k, need[m]);
+    if (k == 0) break;
+    if (done == 1 && nb < 8 * LOOK) k = std::min(k, 1);  // a second look at the contraction first
+    advance(nb, adga::RESID_STEP, k);
+    if (steps) *steps = done - 1;
+  }
+  for (int b = 0; b < nb; ++b)
+    if (!(relh[2 * b] <= accept && relh[2 * b + 1] <= accept)) left.push_back(b);
+  if (8 * left.size() > (size_t)nb) return false;
+  // the last residual is at hand: one more step, whose residual is below the one tested by the contraction
+  adga::launch_add(2L * nb * g.N * g.n2, c->R, Y, s);
+  return true;
+}
+
+bool factor_fp64(adga_ctx* c, int nb) {
+  const Geom& g = c->gw;
+  ensure_lu(c, nb);
+  const adga::VqTerm vt{c->W, c->opgd, c->vqQ};
+  adga::launch_build<double>(g, nb, c->ldm, c->S, c->cd, c->cm, (z64*)c->M, c->stream);
+  if (c->vq) adga::launch_vq_build<double>(g, nb, c->ldm, vt, (z64*)c->M, c->stream);
+  return adga::launch_lu<double>(2 * nb, g.N, g.N, c->ldm, ensure_ops(c, 0), (z64*)c->M, c->piv, (z64*)c->inv,
+                                 c->info, c->stream);
+}
+
 void conv_tables(adga_ctx* c) { ensure_conv(c); }
 void flush_eom(adga_ctx* c) { eom_flush(c); }
 }  // namespace adga_host
@@ -475,6 +594,11 @@ int adga_set_option(adga_ctx* c, const char* key, double v) {
       return ADGA_OK;
     });
   }
+  if (!strcmp(key, "series")) {
+    if (!(v == 0 || v == 1)) return fail(c, ADGA_E_ARG, "series must be 0 (LU always) or 1");
+    c->series = v == 1;
+    return ADGA_OK;
+  }
   if (!strcmp(key, "fallback")) {
     if (!(v == 0 || v == 1)) return fail(c, ADGA_E_ARG, "fallback must be 0 or 1");
     c->fallback = v == 1;
@@ -581,7 +705,7 @@ int run_points_impl(adga_ctx* c, int npts, const int* iq, int precision, double*
     c->lut.flops = 0.0;
     int worst = ADGA_OK;
     hipEvent_t* ev = c->ev;
-    std::vector<int> qh, qp, infoh, st, keep, resolved;
+    std::vector<int> qh, qp, infoh, st, keep, resolved, left;
     std::vector<double> relh;
     std::vector<z64> chih, bubh;
     for (int p0 = 0; p0 < npts; p0 += c->batch) {
@@ -646,50 +770,73 @@ int run_points_impl(adga_ctx* c, int npts, const int* iq, int precision, double*
       CK(hipEventRecord(ev[2], s));
       int iters = 0;
       double maxrel = 0.0;
-      bool lu_ok;
+      bool lu_ok = adga::lu_supported(g.N), factored = false;
       const int prec = precision == ADGA_PREC_FP64 ? 0 : 1;
-      const bool rhs = carry_rhs(c, prec);
-      const std::vector<int>& ops = rhs ? ensure_ops_rhs(c, prec) : ensure_ops(c, prec);
-      const int W = rhs ? g.N + n2 : g.N;
-      adga::LuLanes lanes = c->lanes;
-      lanes.n = pick_lanes(c, prec, g.N, nmat);
       relh.assign(nmat, 0.0);
       infoh.assign(nmat, 0);
       resolved.assign(nmat, 0);
-      if (precision == ADGA_PREC_FP64) {
-        adga::launch_build<double>(g, nb, c->ldm, c->S, c->cd, c->cm, (z64*)c->M, s);
-        if (vtp) adga::launch_vq_build<double>(g, nb, c->ldm, vt, (z64*)c->M, s);
-        if (rhs) adga::launch_rhs_into_m<double>(nmat, g.N, n2, c->ldm, c->Bp, (z64*)c->M, s);
+      // the iteration's tolerance: the refined mode's own, but no looser than a complex64 solve's residual
+      // (4e-7 at N = 1080); one below the round-off of a residual is left to the LU and its limits
+      const double tol = prec == 0 ? SERIES_TOL64 : std::min(c->refine_tol, 1e-6);
+      int steps = 0;
+      bool series = lu_ok && c->series && tol >= SERIES_TOL64 && series_solve(c, nb, tol, prec == 0 ? SERIES_ACCEPT64 : tol, c->Bp, c->Y, relh, left,
+                                             &steps);
+      if (series && !left.empty() && (tan || !c->fallback)) series = false;  // these need every point's factors
+      if (series) {
         CK(hipEventRecord(ev[3], s));
-        CK(hipEventRecord(c->ev_lu[0], s));
-        lu_ok = adga::launch_lu<double>(nmat, g.N, W, c->ldm, ops, (z64*)c->M, c->piv, (z64*)c->inv, c->info, s,
-                                        &c->lut, &lanes);
-        CK(hipEventRecord(c->ev_lu[1], s));
-        if (lu_ok)
-          lu_ok = adga::launch_lu_solve<double>(nmat, g.N, n2, c->ldm, (const z64*)c->M, c->piv, (const z64*)c->inv,
-                                                rhs ? nullptr : c->Bp, c->Y, false, s, nullptr, rhs);
-        if (lu_ok) {
-          // one FP64 residual of the solution: reports the achieved accuracy and non-finite solves
-          adga::launch_residual(g, nb, c->S, c->cd, c->cm, c->Bp, c->Y, c->Z, c->R, c->rel, s, vtp);
-          CK(hipMemcpyAsync(relh.data(), c->rel, sizeof(double) * nmat, hipMemcpyDeviceToHost, s));
-          CK(hipMemcpyAsync(infoh.data(), c->info, sizeof(int) * nmat, hipMemcpyDeviceToHost, s));
-          CK(hipStreamSynchronize(s));
+        for (int b : left) resolved[2 * b] = resolved[2 * b + 1] = 1;
+        const int again = fallback_fp64(c, left, relh, infoh);
+        if (prec == 1) {
+          c->stats[14] += again;
+          iters = std::max(0, steps - 1);  // the steps that correct Y = (1 + T) B
         }
-      } else {
-        adga::launch_build<float>(g, nb, c->ldm, c->S, c->cd, c->cm, (c32*)c->M, s);
-        if (vtp) adga::launch_vq_build<float>(g, nb, c->ldm, vt, (c32*)c->M, s);
-        if (rhs) adga::launch_rhs_into_m<float>(nmat, g.N, n2, c->ldm, c->Bp, (c32*)c->M, s);
-        CK(hipEventRecord(ev[3], s));
-        CK(hipEventRecord(c->ev_lu[0], s));
-        lu_ok = adga::launch_lu<float>(nmat, g.N, W, c->ldm, ops, (c32*)c->M, c->piv, (c32*)c->inv, c->info, s,
-                                       &c->lut, &lanes);
-        CK(hipEventRecord(c->ev_lu[1], s));
-        if (lu_ok)
-          lu_ok = adga::launch_lu_solve<float>(nmat, g.N, n2, c->ldm, (const c32*)c->M, c->piv, (const c32*)c->inv,
-                                               rhs ? nullptr : c->Bp, c->Y, false, s, nullptr, rhs);
-        if (lu_ok) {
-          CK(hipMemcpyAsync(infoh.data(), c->info, sizeof(int) * nmat, hipMemcpyDeviceToHost, s));
-          iters = refine(c, nb, relh, infoh, resolved);
+      } else if (lu_ok) {
+        factored = true;
+        ensure_lu(c, nb);
+        c->lut.used = 0;  // the timer brackets the factorisation's kernel, not an iteration given up
+        c->lut.flops = 0.0;
+        const bool rhs = carry_rhs(c, prec);
+        const std::vector<int>& ops = rhs ? ensure_ops_rhs(c, prec) : ensure_ops(c, prec);
+        const int W = rhs ? g.N + n2 : g.N;
+        adga::LuLanes lanes = c->lanes;
+        lanes.n = pick_lanes(c, prec, g.N, nmat);
+        relh.assign(nmat, 0.0);
+        if (precision == ADGA_PREC_FP64) {
+          adga::launch_build<double>(g, nb, c->ldm, c->S, c->cd, c->cm, (z64*)c->M, s);
+          if (vtp) adga::launch_vq_build<double>(g, nb, c->ldm, vt, (z64*)c->M, s);
+          if (rhs) adga::launch_rhs_into_m<double>(nmat, g.N, n2, c->ldm, c->Bp, (z64*)c->M, s);
+          CK(hipEventRecord(ev[3], s));
+          CK(hipEventRecord(c->ev_lu[0], s));
+          lu_ok = adga::launch_lu<double>(nmat, g.N, W, c->ldm, ops, (z64*)c->M, c->piv, (z64*)c->inv, c->info, s,
+                                          &c->lut, &lanes);
+          CK(hipEventRecord(c->ev_lu[1], s));
+          if (lu_ok)
+            lu_ok = adga::launch_lu_solve<double>(nmat, g.N, n2, c->ldm, (const z64*)c->M, c->piv, (const z64*)c->inv,
+                                                  rhs ? nullptr : c->Bp, c->Y, false, s, nullptr, rhs);
+          if (lu_ok) {
+            // one FP64 residual of the solution: reports the achieved accuracy and non-finite solves
+            adga::launch_absmax_rhs(g, nb, c->Bp, c->nrm, s);
+            adga::launch_residual(g, nb, c->S, c->cd, c->cm, c->Bp, c->Y, c->Z, c->R, c->nrm, s, vtp);
+            CK(hipMemcpyAsync(relh.data(), c->nrm.rel, sizeof(double) * nmat, hipMemcpyDeviceToHost, s));
+            CK(hipMemcpyAsync(infoh.data(), c->info, sizeof(int) * nmat, hipMemcpyDeviceToHost, s));
+            CK(hipStreamSynchronize(s));
+          }
+        } else {
+          adga::launch_build<float>(g, nb, c->ldm, c->S, c->cd, c->cm, (c32*)c->M, s);
+          if (vtp) adga::launch_vq_build<float>(g, nb, c->ldm, vt, (c32*)c->M, s);
+          if (rhs) adga::launch_rhs_into_m<float>(nmat, g.N, n2, c->ldm, c->Bp, (c32*)c->M, s);
+          CK(hipEventRecord(ev[3], s));
+          CK(hipEventRecord(c->ev_lu[0], s));
+          lu_ok = adga::launch_lu<float>(nmat, g.N, W, c->ldm, ops, (c32*)c->M, c->piv, (c32*)c->inv, c->info, s,
+                                         &c->lut, &lanes);
+          CK(hipEventRecord(c->ev_lu[1], s));
+          if (lu_ok)
+            lu_ok = adga::launch_lu_solve<float>(nmat, g.N, n2, c->ldm, (const c32*)c->M, c->piv, (const c32*)c->inv,
+                                                 rhs ? nullptr : c->Bp, c->Y, false, s, nullptr, rhs);
+          if (lu_ok) {
+            CK(hipMemcpyAsync(infoh.data(), c->info, sizeof(int) * nmat, hipMemcpyDeviceToHost, s));
+            iters = refine(c, nb, relh, infoh, resolved);
+          }
         }
       }
       if (!lu_ok) return fail(c, ADGA_E_ARG, "BSE size outside the supported range of the LU kernel");
@@ -758,7 +905,7 @@ int run_points_impl(adga_ctx* c, int npts, const int* iq, int precision, double*
       }
       CK(hipEventRecord(ev[6], s));
       CK(hipGetLastError());
-      if (tan) tangent_batch(c, nb, p0, npts, keep, nfailed, *tan);
+      if (tan) tangent_batch(c, nb, p0, npts, keep, nfailed, *tan, factored);
       chih.resize((size_t)2 * nb * g.n4);
       bubh.resize((size_t)nb * g.n4);
       CK(hipMemcpyAsync(chih.data(), c->chi_out, sizeof(z64) * chih.size(), hipMemcpyDeviceToHost, s));
@@ -772,11 +919,13 @@ int run_points_impl(adga_ctx* c, int npts, const int* iq, int precision, double*
       c->stats[2 + 3] += ms[3];            // Inversion (LU, solve, refinement, FP64 re-solves)
       c->stats[2 + 6] += ms[4];            // Chi (eta + contraction)
       c->stats[2 + 5] += ms[5];            // EOM
-      float lums = 0.f;
-      CK(hipEventElapsedTime(&lums, c->ev_lu[0], c->ev_lu[1]));
-      lane_store(c, lums);
-      c->stats[9] += lums;                 // the batched LU kernel alone
-      c->stats[10] += 1;                   // its launches
+      if (factored) {
+        float lums = 0.f;
+        CK(hipEventElapsedTime(&lums, c->ev_lu[0], c->ev_lu[1]));
+        lane_store(c, lums);
+        c->stats[9] += lums;               // the batched LU kernel alone
+        c->stats[10] += 1;                 // its launches
+      }
       c->stats[11] += c->lut.collect();    // the dominant GEMM kernel: milliseconds,
       c->stats[12] += c->lut.flops;        // algorithmic flops,
       c->stats[13] += c->lut.launches;     // launches
@@ -961,6 +1110,7 @@ int adga_ctx_destroy(adga_ctx* c) {
   if (!c) return ADGA_OK;
   lane_store(c, INFINITY);  // a lane trial left pending by a failed batch counts as the slowest
   free_batch(c);
+  free_lu(c);
   free_fallback(c);
   dfree(c->hk); dfree(c->siw); dfree(c->giw); dfree(c->dc); dfree(c->u); dfree(c->ut); dfree(c->ndmft);
   dfree(c->gt); dfree(c->keom);

@@ -54,12 +54,14 @@ void free_tangent(adga_ctx* c) {
 }
 
 void tangent_batch(adga_ctx* c, int nb, int p0, int npts, const std::vector<int>& keep, int nfailed,
-                   const TangentOut& out) {
+                   const TangentOut& out, bool factored) {
   const Geom& g = c->gw;
   const Geom& G = c->g;
   hipStream_t s = c->stream;
   ensure_tangent_batch(c, nb);
   const int nmat = 2 * nb;
+  std::vector<double> relh;
+  std::vector<int> left;
   const size_t tab = (size_t)G.nw * G.nkp * G.n2, loc = (size_t)G.n2 * G.nf, cc = (size_t)G.N * G.N,
                pm = (size_t)G.n2 * G.N, nsig = (size_t)G.n2 * G.nf * G.nkp_eom;
   for (int dir = 0; dir < c->ndir; ++dir) {
@@ -93,10 +95,18 @@ void tangent_batch(adga_ctx* c, int nb, int p0, int npts, const std::vector<int>
       adga::launch_bubble(g, c->iwb, nb, c->qidx, c->gt, c->t_dchi0q, s, dgt, true);
     }
     adga::launch_dsmat(g, nb, c->chi0q, c->t_dchi0q, c->winv, dwinv, c->t_dS, s);
-    // d eta: M d eta^T = C^T Z1 + dC^T Z2, solved with the complex128 factors of the forward solve
+    // d eta: M d eta^T = C^T Z1 + dC^T Z2, by the forward solve's iteration or with its complex128 factors
     adga::launch_tangent_rhs(g, nb, c->S, c->t_dS, c->cd, c->cm, dcd, dcm, c->opgd, c->opgm, dgamd, dgamm, c->Y,
                              c->t_Z1, c->t_Z2, c->t_B, s);
-    if (!adga::launch_lu_solve<double>(nmat, g.N, g.n2, c->ldm, (const z64*)c->M, c->piv, (const z64*)c->inv, c->t_B,
+    if (!factored) {
+      relh.assign(nmat, 0.0);
+      if (!series_solve(c, nb, SERIES_TOL64, SERIES_ACCEPT64, c->t_B, c->t_dY, relh, left) || !left.empty()) {
+        if (!factor_fp64(c, nb)) throw HipError{hipErrorInvalidValue, "tangent solve: BSE size outside the LU's range"};
+        factored = true;
+      }
+    }
+    if (factored &&
+        !adga::launch_lu_solve<double>(nmat, g.N, g.n2, c->ldm, (const z64*)c->M, c->piv, (const z64*)c->inv, c->t_B,
                                        c->t_dY, false, s))
       throw HipError{hipErrorInvalidValue, "tangent solve: BSE size outside the solve kernel's range"};
     adga::launch_dchi(g, nb, c->chi0q, c->t_dchi0q, c->chi0w, dw, c->gamd, c->gamm, dgamd, dgamm, c->Y, c->t_dY,

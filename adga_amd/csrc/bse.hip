@@ -237,118 +237,244 @@ template void launch_build<double>(const Geom&, int, int, const z64*, const z64*
 // The residual products take their right operand row-major, one N x (npts n2) plane per channel:
 // Z_ch[x][b*n2 + s] = sum_c' S_b[d][c'][i'] V[2b + ch][d*n2 + c'][s]  (x = d*n2 + i'), i.e.
 // Z = blockdiag(S)^T V with the points side by side, V = Y (a solution) or, when Y is null,
-// V = (1 + gamma^w_ch)^T.  Threads run over one matrix m = 2b + ch at a time (x, then s fastest),
-// so the reads of S_b and V_m stay local; the writes land in runs of n2 values.
-__global__ void k_resid_z(Geom g, int npts, const z64* __restrict__ S, const z64* __restrict__ Y,
-                          const z64* __restrict__ opg_d, const z64* __restrict__ opg_m, z64* __restrict__ Z) {
-  const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  const long ncol = (long)npts * g.n2;
-  if (idx >= 2 * g.N * ncol) return;
-  const int s = (int)(idx % g.n2);
-  const long mx = idx / g.n2;
-  const int x = (int)(mx % g.N), m = (int)(mx / g.N);
-  const int b = m / 2, ch = m % 2;
-  const int d = x / g.n2, ip = x % g.n2;
-  const z64* Sd = S + ((long)b * g.nf + d) * g.n4;
-  z64 acc = mk(0.0, 0.0);
-  if (Y) {
-    const z64* Ym = Y + (long)m * g.N * g.n2;
-    for (int cp = 0; cp < g.n2; ++cp) acc = cfma(Sd[cp * g.n2 + ip], Ym[(long)(d * g.n2 + cp) * g.n2 + s], acc);
-  } else {
-    const z64* opg = ch == 0 ? opg_d : opg_m;
-    for (int cp = 0; cp < g.n2; ++cp) acc = cfma(Sd[cp * g.n2 + ip], opg[s + (long)(d * g.n2 + cp) * g.n2], acc);
-  }
-  Z[((long)ch * g.N + x) * ncol + (long)b * g.n2 + s] = acc;
+// V = (1 + gamma^w_ch)^T (k_resid_zt).
+// |re| + |im| as an order-preserving integer: a NaN is above every number, so a maximum keeps it
+__device__ __forceinline__ unsigned long long abs_bits(z64 v) {
+  return (unsigned long long)__double_as_longlong(cabs1(v)) & 0x7fffffffffffffffull;
+}
+__device__ __forceinline__ unsigned long long umax64(unsigned long long a, unsigned long long b) {
+  return a > b ? a : b;
 }
 
 // Out[(2b + ch) N + r][s] = sum_x C_ch(x, r) Z_ch[x][b*n2 + s], plus (B - Y) at the same position
-// when B is given (the residual): the FP64 products on the 3M tile (128 x 64, eight waves), C read
-// row-major as A(r, x) = C[r N + x], the output in the point-major layout of Y.  Workgroups are
-// dealt round-robin to the 8 XCDs; the decode puts all row tiles of one column tile on one XCD,
-// adjacent in time, so that the column block of Z (N x 64) is shared through its L2.
-constexpr int RG_TM = 128, RG_TN = 64, RG_WR = 4, RG_WC = 2, RG_KC = 16;
-__global__ void __launch_bounds__(RG_WR * RG_WC * 64)
-k_resid_gemm(Geom g, int npts, int ch0, const z64* __restrict__ cd, const z64* __restrict__ cm,
-             const z64* __restrict__ Z, z64* Out, const z64* __restrict__ B,
-             const z64* __restrict__ Y, int accumulate) {
-  __shared__ __attribute__((aligned(16))) unsigned char lds[G3Cfg<double, RG_TM, RG_TN, RG_WR, RG_WC, RG_KC>::LDS];
-  const int ch = ch0 + (int)blockIdx.y;
-  const z64* C = ch == 0 ? cd : cm;
+// when B is given (the residual): complex FP64 products by the 3M method (X = Ar Br, Y = Ai Bi,
+// Z = (Ar + Ai)(Br + Bi), as gemm3m_tile), C read row-major as A(r, x) = C[r N + x], the output in the
+// point-major layout of Y.  With rmax, each matrix's max |Out| goes there from the output registers
+// (abs_bits, combined per column in LDS), instead of a second pass over Out.
+//
+// Bound by the FP64 matrix cores: four waves per workgroup, K staged through two LDS buffers in chunks of
+// RG_KC, one barrier per chunk, the next k's fragments loaded ahead of each k's MFMAs, and two (64 x 64 tile,
+// 32 x 32 per wave) to four (32 x 32 tile, 16 x 16 per wave) workgroups per CU, so that one's barriers and
+// staging run under another's MFMAs.  An eight-wave 128 x 64 tile, alone on its CU, took 3.83 ms against 3.21
+// (49 against 59 TFLOP/s issued; an MFMA loop alone reaches 77) at N = 1080, 27000 columns.
+// Workgroup b runs on XCD b % 8; each XCD takes a contiguous eighth of the tiles in an order of RG_GC columns
+// by all rows, so that the 64 or 128 resident workgroups of an XCD share their C and Z panels through its L2
+// and no XCD holds more than one tile more than another (whole columns per XCD: N = 4000, 1200 columns 5.25
+// against 4.26 ms, N = 540, 369 columns 64 against 50 us).
+constexpr int RG_KC = 16, RG_GC = 8;
+template <int TM, int TN>
+__global__ void __launch_bounds__(256, TM == 64 ? 2 : 4)
+k_resid_gemm(Geom g, int npts, int ch0, int nch, const z64* __restrict__ cd, const z64* __restrict__ cm,
+             const z64* __restrict__ Zall, z64* Out, const z64* __restrict__ B, const z64* __restrict__ Y,
+             int accumulate, unsigned long long* __restrict__ rmax) {
+  using V = f64x4;
+  constexpr int KC = RG_KC, WR = 2, WC = 2, RB = TM / WR / 16, CB = TN / WC / 16;
+  constexpr int LDA = KC + 1, LDB = TN + 8, BUF = TM * LDA + KC * LDB;  // strides without bank conflicts
+  constexpr int PA = TM * KC / 256, PB = KC * TN / 256;
+  __shared__ __attribute__((aligned(16))) z64 lds[2 * BUF];
   const int N = g.N, n2 = g.n2, ncol = npts * n2;
-  const int ntr = (N + RG_TM - 1) / RG_TM, ntc = (ncol + RG_TN - 1) / RG_TN;
-  const int L = (int)blockIdx.x, xcd = L & 7, j = L >> 3;
-  const int tc = (j / ntr) * 8 + xcd, tr = j % ntr;
-  if (tc >= ntc) return;
-  const int rt = tr * RG_TM, ct = tc * RG_TN;
-  auto at = [=](int r, int col) {
-    const int b = col / n2, sq = col - b * n2;
-    return ((long)(2 * b + ch) * N + r) * n2 + sq;
+  const int ntr = (N + TM - 1) / TM, ntc = (ncol + TN - 1) / TN, per = ntr * ntc, tot = nch * per;
+  const int share = (tot + 7) / 8, slot = (int)blockIdx.x >> 3, id = ((int)blockIdx.x & 7) * share + slot;
+  if (slot >= share || id >= tot) return;
+  const int ch = ch0 + id / per, e0 = id % per, full = ntc / RG_GC * RG_GC;
+  const int gw = e0 < full * ntr ? RG_GC : ntc - full;  // columns of this tile's group
+  const int gc = e0 < full * ntr ? e0 / (RG_GC * ntr) * RG_GC : full, ge = e0 - gc * ntr;
+  const int rt = ge / gw * TM, ct = (gc + ge % gw) * TN;
+  const z64* A = ch == 0 ? cd : cm;
+  const z64* Z = Zall + (long)ch * N * ncol;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int wr = (wave / WC) * (TM / WR), wc = (wave % WC) * (TN / WC), li = lane & 15, lg = lane >> 4;
+  const bool inside = rt + TM <= N && ct + TN <= ncol;
+  V x[RB][CB], y[RB][CB], z[RB][CB];
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb) x[rb][cb] = y[rb][cb] = z[rb][cb] = V{0, 0, 0, 0};
+  z64 pa[PA], pb[PB];
+  auto fetch = [&](int kb) {
+    const bool whole = inside && kb + KC <= N;
+#pragma unroll
+    for (int i = 0; i < PA; ++i) {
+      const int e = t + i * 256, row = rt + e / KC, k = kb + e % KC;
+      pa[i] = whole || (row < N && k < N) ? A[(long)row * N + k] : mk(0.0, 0.0);
+    }
+#pragma unroll
+    for (int i = 0; i < PB; ++i) {
+      const int e = t + i * 256, k = kb + e / TN, col = ct + e % TN;
+      pb[i] = whole || (k < N && col < ncol) ? Z[(long)k * ncol + col] : mk(0.0, 0.0);
+    }
   };
-  gemm3m_tile<double, RG_TM, RG_TN, RG_WR, RG_WC, RG_KC>(
-      C, N, Z + (long)ch * N * ncol, ncol,
-      [=](int r, int col) {
-        const long i = at(r, col);
-        return B ? csub(B[i], Y[i]) : Out[i];
-      },
-      [=](int r, int col, z64 v) { Out[at(r, col)] = v; }, N, ncol, N, B == nullptr && !accumulate, false, rt, ct,
-      lds);
-}
-
-// Out = C_ch^T Z_ch (+ B - Y when B is given, + Out itself when accumulate)
-void resid_gemm(const Geom& g, int npts, int ch0, int nch, const z64* cd, const z64* cm, const z64* Z, z64* Out,
-                const z64* B, const z64* Y, hipStream_t s, bool accumulate) {
-  const int ntr = (g.N + RG_TM - 1) / RG_TM, ntc = (npts * g.n2 + RG_TN - 1) / RG_TN;
-  const int nwg = ntr * ((ntc + 7) / 8) * 8;
-  hipLaunchKernelGGL(k_resid_gemm, dim3(nwg, nch), dim3(RG_WR * RG_WC * 64), 0, s, g, npts, ch0, cd, cm, Z, Out, B,
-                     Y, accumulate ? 1 : 0);
-}
-
-// Per-matrix max |R| / max |B| (|.| = |re|+|im|), one workgroup per matrix; a zero right-hand
-// side counts as converged when the residual is zero too.
-__global__ void __launch_bounds__(256) k_resid_norm(Geom g, const z64* __restrict__ R, const z64* __restrict__ B,
-                                                    double* __restrict__ rel) {
-  __shared__ double sr[256], sb[256];
-  const int m = blockIdx.x, t = threadIdx.x;
-  const long tot = (long)g.N * g.n2;
-  double mr = 0.0, mb = 0.0;
-  for (long e = t; e < tot; e += 256) {
-    mr = fmax(mr, cabs1(R[(long)m * tot + e]));
-    mb = fmax(mb, cabs1(B[(long)m * tot + e]));
-    double v = R[(long)m * tot + e].re + R[(long)m * tot + e].im;
-    if (!isfinite(v)) mr = INFINITY;
-  }
-  sr[t] = mr;
-  sb[t] = mb;
+  auto stage = [&](int b) {
+    z64* As = lds + b * BUF;
+    z64* Bs = As + TM * LDA;
+#pragma unroll
+    for (int i = 0; i < PA; ++i) {
+      const int e = t + i * 256;
+      As[(e / KC) * LDA + e % KC] = pa[i];
+    }
+#pragma unroll
+    for (int i = 0; i < PB; ++i) {
+      const int e = t + i * 256;
+      Bs[(e / TN) * LDB + e % TN] = pb[i];
+    }
+  };
+  auto compute = [&](int b, int kend) {  // k in [kend, KC) of a last, partial chunk are staged zeros
+    const z64* Ap = lds + b * BUF + (wr + li) * LDA + lg;
+    const z64* Bp = lds + b * BUF + TM * LDA + lg * LDB + wc + li;
+    z64 a[2][RB], v[2][CB];
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) a[0][rb] = Ap[rb * 16 * LDA];
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb) v[0][cb] = Bp[cb * 16];
+#pragma unroll
+    for (int kk = 0; kk < KC; kk += 4) {
+      const int p = (kk >> 2) & 1;
+      if (kk + 4 < KC) {
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) a[p ^ 1][rb] = Ap[rb * 16 * LDA + kk + 4];
+#pragma unroll
+        for (int cb = 0; cb < CB; ++cb) v[p ^ 1][cb] = Bp[(kk + 4) * LDB + cb * 16];
+      }
+      if (kk >= kend) continue;
+      double as[RB], vs[CB];
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) as[rb] = a[p][rb].re + a[p][rb].im;
+#pragma unroll
+      for (int cb = 0; cb < CB; ++cb) vs[cb] = v[p][cb].re + v[p][cb].im;
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+        for (int cb = 0; cb < CB; ++cb) {
+          x[rb][cb] = Mfma<double>::op(a[p][rb].re, v[p][cb].re, x[rb][cb]);
+          y[rb][cb] = Mfma<double>::op(a[p][rb].im, v[p][cb].im, y[rb][cb]);
+          z[rb][cb] = Mfma<double>::op(as[rb], vs[cb], z[rb][cb]);
+        }
+    }
+  };
+  fetch(0);
+  stage(0);
+  if (KC < N) fetch(KC);
   __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
-    if (t < o) { sr[t] = fmax(sr[t], sr[t + o]); sb[t] = fmax(sb[t], sb[t + o]); }
+  int b = 0, kb = 0;
+  for (; kb + KC < N; kb += KC) {
+    compute(b, KC);
+    stage(b ^ 1);  // last read in the previous chunk, before the barrier that ended it
+    if (kb + 2 * KC < N) fetch(kb + 2 * KC);
     __syncthreads();
+    b ^= 1;
   }
-  if (t == 0) rel[m] = sb[0] > 0.0 ? sr[0] / sb[0] : (sr[0] > 0.0 ? INFINITY : 0.0);
+  auto at = [&](int r, int col) {
+    const int pt = col / n2;
+    return ((long)(2 * pt + ch) * N + r) * n2 + (col - pt * n2);
+  };
+  // what is added to the product is loaded beside the last chunk's MFMAs
+  const bool add = B != nullptr || accumulate;
+  z64 cin[RB][CB][4];
+  if (add) {
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+      for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int row = rt + wr + rb * 16 + Mfma<double>::row(lg, v), col = ct + wc + cb * 16 + li;
+          z64 c = mk(0.0, 0.0);
+          if (row < N && col < ncol) {
+            const long i = at(row, col);
+            c = B ? csub(B[i], Y[i]) : Out[i];
+          }
+          cin[rb][cb][v] = c;
+        }
+  }
+  compute(b, N - kb);
+  unsigned long long mx[CB] = {};
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int row = rt + wr + rb * 16 + Mfma<double>::row(lg, v), col = ct + wc + cb * 16 + li;
+        if (row < N && col < ncol) {
+          z64 o = mk(x[rb][cb][v] - y[rb][cb][v], (z[rb][cb][v] - x[rb][cb][v]) - y[rb][cb][v]);
+          if (add) o = cadd(cin[rb][cb][v], o);
+          Out[at(row, col)] = o;
+          mx[cb] = umax64(mx[cb], abs_bits(o));
+        }
+      }
+  if (rmax) {
+    __syncthreads();  // the tile's LDS reads are done
+    unsigned long long* sm = reinterpret_cast<unsigned long long*>(lds);
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb) {
+      unsigned long long v = mx[cb];
+      v = umax64(v, __shfl_xor(v, 16));
+      v = umax64(v, __shfl_xor(v, 32));
+      if (lane < 16) sm[(wave / WC) * TN + wc + cb * 16 + lane] = v;
+    }
+    __syncthreads();
+    if (t < TN && ct + t < ncol) atomicMax(&rmax[2 * ((ct + t) / n2) + ch], umax64(sm[t], sm[TN + t]));
+  }
 }
 
-// Zg[d*n2 + i'][b*n2 + s] = S_b[d][s][i'] (the channel-0 plane of the residual product's right
-// operand), so that C^T Zg (k_resid_gemm) is
-// gamma^q_d(s, r) = sum_d sum_i' S_b[d][s][i'] C_d(d*n2 + i', r) = sum_nu chi0^{nl,q} F^w_d
-// (main.F90:693-700, the accumulation of rectanglework over nu).
-__global__ void k_gamq_z(Geom g, int npts, const z64* __restrict__ S, z64* __restrict__ Z) {
-  const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  const long ncol = (long)npts * g.n2;
-  if (idx >= g.N * ncol) return;
-  const int col = (int)(idx % ncol), x = (int)(idx / ncol);
-  const int b = col / g.n2, s = col - b * g.n2;
-  const int d = x / g.n2, ip = x % g.n2;
-  Z[idx] = S[((long)b * g.nf + d) * g.n4 + s * g.n2 + ip];
+// Out = C_ch^T Z_ch (+ B - Y when B is given, + Out itself when accumulate).  64 x 64 tiles from four rounds
+// of the chip's 512 such workgroups on; below, 32 x 32 tiles lose less to the last round and to few
+// workgroups (64 x 64 against 32 x 32: N = 1080, 27000 columns 3.21 / 3.50 ms; N = 4000, 2400 columns
+// 4.26 / 4.40; N = 2000, 3200 columns 1.44 / 1.39; N = 540, 738 columns 89 / 50 us; N = 40, 1024 columns 15 / 8).
+void resid_gemm(const Geom& g, int npts, int ch0, int nch, const z64* cd, const z64* cm, const z64* Z, z64* Out,
+                const z64* B, const z64* Y, hipStream_t s, bool accumulate, unsigned long long* rmax) {
+  auto tiles = [&](int tile) {
+    return nch * ((long)(g.N + tile - 1) / tile) * (((long)npts * g.n2 + tile - 1) / tile);
+  };
+  auto grid = [](long n) { return dim3((unsigned)((n + 7) / 8 * 8)); };
+  if (tiles(64) >= 2048)
+    hipLaunchKernelGGL((k_resid_gemm<64, 64>), grid(tiles(64)), dim3(256), 0, s, g, npts, ch0, nch, cd, cm, Z, Out, B,
+                       Y, accumulate ? 1 : 0, rmax);
+  else
+    hipLaunchKernelGGL((k_resid_gemm<32, 32>), grid(tiles(32)), dim3(256), 0, s, g, npts, ch0, nch, cd, cm, Z, Out, B,
+                       Y, accumulate ? 1 : 0, rmax);
 }
 
-// k_resid_z and k_gamq_z for n <= 3 with one thread per (channel, d, point b, column s) forming the n2 rows
-// x = d*n2 + i' of its column: each thread reads its values of V (or of S_b) once, and for each i' the
-// wave writes a contiguous run of Z's row x (consecutive lanes hold consecutive columns b*n2 + s).  The
-// same sums in the same order as the one-output-per-thread forms above.
+// Per-matrix max |A| (|.| = |re|+|im|, abs_bits), one workgroup per matrix; `clear` (may be null) is zeroed.
+__global__ void __launch_bounds__(256) k_absmax(long tot, const z64* __restrict__ A,
+                                                unsigned long long* __restrict__ out,
+                                                unsigned long long* __restrict__ clear) {
+  __shared__ unsigned long long sr[4];
+  const int m = blockIdx.x, t = threadIdx.x;
+  unsigned long long v = 0;
+  for (long e = t; e < tot; e += 256) v = umax64(v, abs_bits(A[(long)m * tot + e]));
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v = umax64(v, __shfl_xor(v, o));
+  if ((t & 63) == 0) sr[t >> 6] = v;
+  __syncthreads();
+  if (t == 0) {
+    out[m] = umax64(umax64(sr[0], sr[1]), umax64(sr[2], sr[3]));
+    if (clear) clear[m] = 0;
+  }
+}
+
+// rel[m] = max|R| / max|B|, and rmax cleared for the next residual; a zero right-hand side counts as
+// converged when the residual is zero too, a NaN in the residual gives NaN.
+__global__ void k_resid_rel(int nmat, const unsigned long long* __restrict__ bmax,
+                            unsigned long long* __restrict__ rmax, double* __restrict__ rel) {
+  const int m = blockIdx.x * blockDim.x + threadIdx.x;
+  if (m >= nmat) return;
+  const double r = __longlong_as_double((long long)rmax[m]), b = __longlong_as_double((long long)bmax[m]);
+  rel[m] = b > 0.0 ? r / b : (r == 0.0 ? 0.0 : INFINITY);
+  rmax[m] = 0;
+}
+
+// Z = blockdiag(S)^T V with one thread per (channel, d, point b, column s) forming the n2 rows
+// x = d*n2 + i' of its column: each thread reads its values of V once, and for each i' the wave writes a
+// contiguous run of Z's row x (consecutive lanes hold consecutive columns b*n2 + s).  V by `mode`: Z_OPG
+// (1 + gamma^w)^T, Z_Y the solution, Z_ADD Y + R with the sum stored to Y (a step of the fixed-point
+// iteration: every element of Y belongs to one thread), Z_RHS B, stored to Y (its start).
+enum { Z_OPG = 0, Z_Y = 1, Z_ADD = 2, Z_RHS = 3 };
 template <int N2>
-__global__ void __launch_bounds__(256) k_resid_zt(Geom g, int npts, const z64* __restrict__ S,
-                                                  const z64* __restrict__ Y, const z64* __restrict__ opg_d,
-                                                  const z64* __restrict__ opg_m, z64* __restrict__ Z) {
+__global__ void __launch_bounds__(256) k_resid_zt(Geom g, int npts, int mode, const z64* __restrict__ S,
+                                                  z64* __restrict__ Y, const z64* __restrict__ R,
+                                                  const z64* __restrict__ opg_d, const z64* __restrict__ opg_m,
+                                                  z64* __restrict__ Z) {
   const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
   const long ncol = (long)npts * N2;
   if (idx >= 2L * g.nf * ncol) return;
@@ -357,14 +483,23 @@ __global__ void __launch_bounds__(256) k_resid_zt(Geom g, int npts, const z64* _
   const int b = col / N2, s = col - b * N2;
   const z64* Sd = S + ((long)b * g.nf + d) * (N2 * N2);
   z64 v[N2];
-  if (Y) {
-    const z64* Ym = Y + (long)(2 * b + ch) * g.N * N2;
-#pragma unroll
-    for (int cp = 0; cp < N2; ++cp) v[cp] = Ym[(long)(d * N2 + cp) * N2 + s];
-  } else {
+  if (mode == Z_OPG) {
     const z64* opg = ch == 0 ? opg_d : opg_m;
 #pragma unroll
     for (int cp = 0; cp < N2; ++cp) v[cp] = opg[s + (long)(d * N2 + cp) * N2];
+  } else {
+    const long o = (long)(2 * b + ch) * g.N * N2 + (long)d * N2 * N2 + s;
+    const z64* src = mode == Z_RHS ? R : Y;
+#pragma unroll
+    for (int cp = 0; cp < N2; ++cp) v[cp] = src[o + cp * N2];
+    if (mode == Z_ADD) {
+#pragma unroll
+      for (int cp = 0; cp < N2; ++cp) v[cp] = cadd(v[cp], R[o + cp * N2]);
+    }
+    if (mode != Z_Y) {
+#pragma unroll
+      for (int cp = 0; cp < N2; ++cp) Y[o + cp * N2] = v[cp];
+    }
   }
   z64* Zc = Z + ((long)ch * g.N + (long)d * N2) * ncol + col;
 #pragma unroll
@@ -376,6 +511,10 @@ __global__ void __launch_bounds__(256) k_resid_zt(Geom g, int npts, const z64* _
   }
 }
 
+// Zg[d*n2 + i'][b*n2 + s] = S_b[d][s][i'] (the channel-0 plane of the residual product's right
+// operand), so that C^T Zg (k_resid_gemm) is
+// gamma^q_d(s, r) = sum_d sum_i' S_b[d][s][i'] C_d(d*n2 + i', r) = sum_nu chi0^{nl,q} F^w_d
+// (main.F90:693-700, the accumulation of rectanglework over nu); threads as in k_resid_zt.
 template <int N2>
 __global__ void __launch_bounds__(256) k_gamq_zt(Geom g, int npts, const z64* __restrict__ S, z64* __restrict__ Z) {
   const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -389,33 +528,32 @@ __global__ void __launch_bounds__(256) k_gamq_zt(Geom g, int npts, const z64* __
   for (int ip = 0; ip < N2; ++ip) Zc[(long)ip * ncol] = Sd[ip];
 }
 
-// k_resid_z / k_resid_zt over both channels: Y (a solution) or, with Y null, (1 + gamma^w)^T
-static void resid_z(const Geom& g, int npts, const z64* S, const z64* Y, const z64* opgd, const z64* opgm, z64* Z,
-                    hipStream_t s) {
+static void resid_z(const Geom& g, int npts, int mode, const z64* S, z64* Y, const z64* R, const z64* opgd,
+                    const z64* opgm, z64* Z, hipStream_t s) {
   const long tz = 2L * g.nf * npts * g.n2;
 #define ADGA_RZ(NN)                                                                                                 \
-  if (g.n == NN) {                                                                                                 \
-    hipLaunchKernelGGL(k_resid_zt<NN * NN>, dim3((unsigned)((tz + 255) / 256)), dim3(256), 0, s, g, npts, S, Y,     \
-                       opgd, opgm, Z);                                                                             \
-    return;                                                                                                        \
+  case NN:                                                                                                         \
+    hipLaunchKernelGGL(k_resid_zt<NN * NN>, dim3((unsigned)((tz + 255) / 256)), dim3(256), 0, s, g, npts, mode, S, \
+                       Y, R, opgd, opgm, Z);                                                                       \
+    break;
+  switch (g.n) {
+    ADGA_RZ(1) ADGA_RZ(2) ADGA_RZ(3) ADGA_RZ(4) ADGA_RZ(5)
+    default: break;
   }
-  ADGA_RZ(1) ADGA_RZ(2) ADGA_RZ(3)
 #undef ADGA_RZ
-  const long tot = 2L * npts * g.N * g.n2;
-  hipLaunchKernelGGL(k_resid_z, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s, g, npts, S, Y, opgd, opgm, Z);
 }
 
 void launch_gamq_z(const Geom& g, int npts, const z64* S, z64* Z, hipStream_t s) {
   const long tz = (long)g.nf * npts * g.n2;
 #define ADGA_GZ(NN)                                                                                                 \
-  if (g.n == NN) {                                                                                                 \
+  case NN:                                                                                                         \
     hipLaunchKernelGGL(k_gamq_zt<NN * NN>, dim3((unsigned)((tz + 255) / 256)), dim3(256), 0, s, g, npts, S, Z);     \
-    return;                                                                                                        \
+    break;
+  switch (g.n) {
+    ADGA_GZ(1) ADGA_GZ(2) ADGA_GZ(3) ADGA_GZ(4) ADGA_GZ(5)
+    default: break;
   }
-  ADGA_GZ(1) ADGA_GZ(2) ADGA_GZ(3)
 #undef ADGA_GZ
-  long tot = (long)npts * g.N * g.n2;
-  hipLaunchKernelGGL(k_gamq_z, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s, g, npts, S, Z);
 }
 
 // gamma^q_d for every point of the batch, into G2 with the residual layout (point b at 2*b).
@@ -429,20 +567,45 @@ void launch_gamq(const Geom& g, int npts, const z64* S, const z64* cd, z64* Z, z
 // (1+gamma^w_d)^T (W^T (1+gamma^w_d)^T).
 void launch_rhs(const Geom& g, int npts, const z64* S, const z64* cd, const z64* cm, const z64* opgd,
                 const z64* opgm, z64* Z, z64* B, hipStream_t s, const VqTerm* vq) {
-  resid_z(g, npts, S, nullptr, opgd, opgm, Z, s);
+  resid_z(g, npts, Z_OPG, S, nullptr, nullptr, opgd, opgm, Z, s);
   resid_gemm(g, npts, 0, 2, cd, cm, Z, B, nullptr, nullptr, s);
   if (vq) launch_vq_add(g, npts, *vq, nullptr, B, s);
 }
 
+void launch_absmax_rhs(const Geom& g, int npts, const z64* B, const ResidNorm& nrm, hipStream_t s) {
+  hipLaunchKernelGGL(k_absmax, dim3(2 * npts), dim3(256), 0, s, (long)g.N * g.n2, B, nrm.bmax, nrm.rmax);
+}
+
+__global__ void k_add(long n, const z64* __restrict__ R, z64* __restrict__ Y) {
+  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) Y[i] = cadd(Y[i], R[i]);
+}
+
+void launch_add(long n, const z64* R, z64* Y, hipStream_t s) {
+  hipLaunchKernelGGL(k_add, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, n, R, Y);
+}
+
 // R = B - M Y with M Y = Y - C^T (blockdiag(S)^T Y), in FP64 from the unrounded factors S and C (with V(q):
-// minus (1 + gamma^w_d)^T (W^T Y) in the density channel).
-void launch_residual(const Geom& g, int npts, const z64* S, const z64* cd, const z64* cm, const z64* B,
-                     const z64* Y, z64* Z, z64* R, double* rel, hipStream_t s, const VqTerm* vq) {
+// minus (1 + gamma^w_d)^T (W^T Y) in the density channel).  Y: as given, or first Y += R (RESID_STEP) or
+// Y = B (RESID_START), folded into the kernel that reads it.  M = 1 - T with T Y = C^T (blockdiag(S)^T Y), so
+// the steps Y += R from Y = B sum the series (1 + T + T^2 + ...) B.
+void launch_residual(const Geom& g, int npts, const z64* S, const z64* cd, const z64* cm, const z64* B, z64* Y,
+                     z64* Z, z64* R, const ResidNorm& nrm, hipStream_t s, const VqTerm* vq, ResidMode mode,
+                     LuTimer* timer) {
   const int nmat = 2 * npts;
-  resid_z(g, npts, S, Y, nullptr, nullptr, Z, s);
-  resid_gemm(g, npts, 0, 2, cd, cm, Z, R, B, Y, s);
-  if (vq) launch_vq_add(g, npts, *vq, Y, R, s);
-  hipLaunchKernelGGL(k_resid_norm, dim3(nmat), dim3(256), 0, s, g, R, B, rel);
+  const int zm = mode == RESID_START ? Z_RHS : mode == RESID_STEP ? Z_ADD : Z_Y;
+  resid_z(g, npts, zm, S, Y, mode == RESID_START ? B : R, nullptr, nullptr, Z, s);
+  if (timer) {
+    timer->mark(s);
+    timer->flops += 8.0 * g.N * (double)g.N * g.n2 * nmat;
+  }
+  resid_gemm(g, npts, 0, 2, cd, cm, Z, R, B, Y, s, false, vq ? nullptr : nrm.rmax);
+  if (timer) timer->mark(s);
+  if (vq) {
+    launch_vq_add(g, npts, *vq, Y, R, s);
+    hipLaunchKernelGGL(k_absmax, dim3(nmat), dim3(256), 0, s, (long)g.N * g.n2, R, nrm.rmax, nullptr);
+  }
+  hipLaunchKernelGGL(k_resid_rel, dim3((nmat + 255) / 256), dim3(256), 0, s, nmat, nrm.bmax, nrm.rmax, nrm.rel);
 }
 
 }  // namespace adga

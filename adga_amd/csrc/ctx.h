@@ -35,7 +35,7 @@ struct FallbackBufs {
   int cap = 0;  // points
   z64 *S = nullptr, *B = nullptr, *Y = nullptr, *Z = nullptr, *R = nullptr, *M = nullptr, *inv = nullptr;
   z64 *W = nullptr, *Q = nullptr;  // V(q) rows and products of the gathered points
-  double* rel = nullptr;
+  adga::ResidNorm nrm{};
   int *piv = nullptr, *info = nullptr, *sel = nullptr;
 };
 
@@ -56,6 +56,7 @@ struct adga_ctx {
   std::string err;
   int refine_maxit = 12;
   double refine_tol = 1e-12;
+  bool series = true;    // option "series": contracting BSE systems are solved by fixed-point iteration, not by LU
   bool fallback = true;  // option "fallback": unconverged complex64 solves are solved again in complex128
   int batch = 256;
   int ldm = 0;
@@ -79,10 +80,13 @@ struct adga_ctx {
   int cap = 0;
   z64 *chi0q = nullptr, *S = nullptr, *gamq = nullptr, *Bp = nullptr, *Y = nullptr, *Z = nullptr, *R = nullptr,
       *mt = nullptr, *chi_out = nullptr, *bub_out = nullptr;
+  adga::ResidNorm nrm{};  // residual norms of the batch's matrices
+  int* qidx = nullptr;
+  // LU workspace, allocated by the first batch that factors (lu_cap points)
+  int lu_cap = 0;
   void* M = nullptr;
   void* inv = nullptr;  // per-matrix panel inverses of the LU
-  double* rel = nullptr;
-  int *piv = nullptr, *info = nullptr, *qidx = nullptr;
+  int *piv = nullptr, *info = nullptr;
   bool q_distinct = false;          // the current batch's q indices are pairwise different
   std::vector<unsigned char> qmark;  // host scratch of that test, zero between batches (nkp entries)
   int *act = nullptr, *keep = nullptr;  // per-matrix refinement flags, per-point "enters the self-energy" flags
@@ -232,8 +236,16 @@ inline int op_finish(adga_ctx* c, bool launched, const char* what) {
 
 // derivatives of one batch of points (positions p0 .. p0 + nb - 1 of npts) along every tangent direction,
 // after the forward work of the batch (api_tangent.cpp)
+// (factored: the batch's complex128 factors are in c->M; else its forward solve was the fixed-point iteration)
 void tangent_batch(adga_ctx* c, int nb, int p0, int npts, const std::vector<int>& keep, int nfailed,
-                   const TangentOut& out);
+                   const TangentOut& out, bool factored);
+// M Y = B for every matrix of a batch by fixed-point iteration in FP64; false where the LU is to be taken
+bool series_solve(adga_ctx* c, int nb, double tol, double accept, const z64* B, z64* Y, std::vector<double>& relh,
+                  std::vector<int>& left, int* steps = nullptr);
+// the FP64 mode's relative residual: the aim, and what a residual at its round-off may be
+constexpr double SERIES_TOL64 = 1e-15, SERIES_ACCEPT64 = 1e-14;
+// the batch's M in complex128, factored (api.cpp); false: BSE size outside the LU kernel's range
+bool factor_fp64(adga_ctx* c, int nb);
 void free_tangent(adga_ctx* c);
 // the twiddles and the k-grid transform of the G table (formed once); the pending omega's EOM flushed
 // (with its derivatives when tangent directions are set) (api.cpp)

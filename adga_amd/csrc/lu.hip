@@ -997,6 +997,8 @@ bool lu_op(int nmat, int N, int W, int ldm, const int* op, cplx<T>* M, int* piv,
 }
 }  // namespace
 
+bool lu_supported(int N) { return panel_cfg(N) >= 0 && N <= PERM_MAX_N; }
+
 // With a second stream the batch is split in two halves, the second one operation behind the
 // first on its own stream: while one half runs a latency-bound panel or a small update, the other
 // half's operation can use the rest of the machine.  The large Schur updates (those with 128x128
@@ -1006,7 +1008,7 @@ bool lu_op(int nmat, int N, int W, int ldm, const int* op, cplx<T>* M, int* piv,
 template <typename T>
 bool launch_lu(int nmat, int N, int W, int ldm, const int* ops, size_t nops, cplx<T>* M, int* piv, cplx<T>* inv,
                int* info, hipStream_t s, LuTimer* timer, const LuLanes* lanes) {
-  if (panel_cfg(N) < 0 || N > PERM_MAX_N || nmat < 1) return false;
+  if (!lu_supported(N) || nmat < 1) return false;
   const long mstride = (long)N * ldm, istride = (long)lu_inv_elems(N);
   // the batch in nl parts of about equal size (at least 8 matrices each), part j on lane j; after each join
   // lane j starts its next operation when lane j-1 has finished it, so the parts run staggered by one

@@ -37,8 +37,9 @@ enum {
 #define ADGA_INVERSE_MAX_N 4096
 
 enum {
-  ADGA_PREC_FP64 = 0,    /* complex128 LU and solve */
-  ADGA_PREC_REFINED = 1  /* complex64 LU, FP64 residuals and iterative refinement */
+  ADGA_PREC_FP64 = 0,    /* complex128 throughout: fixed-point iteration or LU (option "series") */
+  ADGA_PREC_REFINED = 1  /* to a relative residual of "refine_tol": FP64 fixed-point iteration, or complex64 LU
+                            with FP64 residuals and iterative refinement */
 };
 
 typedef struct adga_ctx adga_ctx;
@@ -73,7 +74,11 @@ int adga_ctx_create(const adga_dims *dims, const int *q_data, const int *k_data_
  * residual max|r|/max|b| every BSE solve must reach, default 1e-12), "refine_maxit" (default 12;
  * a matrix that has not converged by then, or whose residual a correction did not halve, or whose
  * complex64 LU met a zero pivot, is solved again in complex128 unless "fallback" is 0; its final
- * status then depends only on the complex128 solve), "do_eom" (1: the default; 0: no
+ * status then depends only on the complex128 solve), "series" (1, the default: the BSE systems of a batch, eta (1 - T) = B, are solved by the
+ * fixed-point iteration eta <- B + eta T in FP64 where T contracts, in the FP64 mode to the round-off of the
+ * residual, 1e-15 .. 1e-14, in the refined mode to "refine_tol"; batches that do not contract, or would need
+ * more steps than the LU costs, take the LU, and single points that do not converge the complex128 LU; 0: the
+ * LU always), "do_eom" (1: the default; 0: no
  * equation of motion, as the reference's do_eom = .false. for a q path),
  * "bubble" (0: direct k sum per point; 1: all q of the current omega at once by
  * k-grid DFT, cached per omega; 2: DFT when a batch has >= 64 points or the cache is valid, the
@@ -318,12 +323,13 @@ int adga_get_ndga(adga_ctx *ctx, const double *sigma_sum, double *n_dga_k, doubl
 
 /*
  * Statistics of the last adga_run_points call (nout <= 16 values): out[0] = max refinement
- * iterations, out[1] = max final relative residual of the points that succeeded, out[2..8] =
+ * iterations (complex64 corrections, or the fixed-point iteration's steps beyond its first), out[1] = max final relative residual of the points that succeeded, out[2..8] =
  * milliseconds spent in the reference's stage buckets Local, Chi0, Gammas, Inversion, Eta rest, EOM,
  * Chi (src/main.F90:484-783), out[9] = milliseconds of the batched LU factorisations, out[10] =
- * their number, out[11..13] = milliseconds, algorithmic flops and launches of the factorisation's
- * dominant GEMM kernel (the largest tile shape), out[14] = matrices solved again in complex128
- * after their complex64 refinement failed, out[15] = points with a non-zero status.
+ * their number (0 where no batch was factored), out[11..13] = milliseconds, algorithmic flops and launches
+ * of the BSE solve's dominant GEMM kernel (the factorisation's largest tile shape, or the iteration's residual
+ * product), out[14] = matrices solved again in complex128
+ * after their complex64 refinement or the refined mode's iteration failed, out[15] = points with a non-zero status.
  */
 int adga_get_stats(adga_ctx *ctx, double *out, int nout);
 
