@@ -155,6 +155,7 @@ void launch_dchi(const Geom& g, int npts, const z64* chi0q, const z64* dchi0q, c
                  const z64* gamd, const z64* gamm, const z64* dgamd, const z64* dgamm, const z64* Y, const z64* dY,
                  z64* dchi_out, z64* dbub_out, hipStream_t s);
 // k-grid convolutions (kconv.hip)
+bool dft_in_lds(const Geom& g);  // the fields' transforms run in LDS: the bubbles' P below may be null
 void dft3(const Geom& g, long nfield, int sign, const z64* tw, z64* a, z64* b, hipStream_t s);
 void launch_ghat(const Geom& g, const z64* tw, const z64* gt, z64* tmp, z64* ghat, hipStream_t s);
 void launch_bubble_all(const Geom& g, int iwb, const z64* tw, const z64* ghat, z64* P, z64* out, hipStream_t s);

@@ -750,8 +750,8 @@ int run_points_impl(adga_ctx* c, int npts, const int* iq, int precision, double*
         ensure_conv(c);
         if (!bub_hit) {
           size_t nb_all = (size_t)c->g.nf * g.n4 * g.nkp;  // sized for the largest box
-          if (!c->bub_p) {
-            dalloc(&c->bub_p, nb_all);
+          if (!c->bub_all) {
+            if (!adga::dft_in_lds(g) && !c->bub_p) dalloc(&c->bub_p, nb_all);
             dalloc(&c->bub_all, nb_all);
           }
           adga::launch_bubble_all(g, c->iwb, c->tw, c->ghat, c->bub_p, c->bub_all, s);

@@ -78,8 +78,8 @@ void tangent_batch(adga_ctx* c, int nb, int p0, int npts, const std::vector<int>
       if (!t_hit) {
         if (dir == 0) {
           if (!c->t_dbub_all) {
+            if (!adga::dft_in_lds(g) && !c->t_bub_p) dalloc(&c->t_bub_p, nall);
             dalloc(&c->t_dbub_all, nall * c->ndir);
-            dalloc(&c->t_bub_p, nall);
           }
           for (int d = 0; d < c->ndir; ++d)
             adga::launch_bubble_all_tangent(g, c->iwb, c->tw, c->ghat, c->t_dghat + d * tab, c->t_bub_p,

@@ -10,6 +10,8 @@
 // The transform is applied one axis at a time (a 3D DFT is three batched products with the
 // n_a x n_a twiddle matrix); each pass is bound by HBM streaming of the batch of fields.
 // A field is one contiguous grid (kz fastest, like k_index_3, kq_tools.f90:119-125).
+#include <algorithm>
+
 #include "adga_kernels.h"
 
 namespace adga {
@@ -117,8 +119,177 @@ static void dft_pass(long nfield, int nx, int ny, int nz, int axis, int sign, co
                      tw, in, out);
 }
 
-// Three axis passes: a -> b -> a -> b; the transform ends in b.
+// ---------------------------------------------------------------- whole transform in LDS
+// One workgroup transforms one field with every axis pass in LDS, so a field is read and written once instead
+// of once per axis, and fields that are products (the bubble's) are formed while they are loaded instead of
+// being stored first.  Rows along z are padded to an odd length: the passes, one line per thread, then read and
+// write without bank conflicts along every axis.
+//
+// A line of n points takes (n/2)^2 steps of four real FMAs: with p_k = x_k + x_(n-k) and m_k = x_k - x_(n-k),
+// X_R = x_0 + sum_k (p_k cos - i m_k sin) and X_(n-R) the same with + i, a quarter of the FMAs of the plain
+// n x n product, with compile-time cosines and sines.
+//
+// The bubble of all q at 20^3 k, three orbitals, 120 frequencies (9720 fields): the product 0.49 and three
+// passes of 0.65 ms -> 0.87 ms; 4860 fields of the EOM 3 x 0.33 -> 0.37; at 16^3 k, five orbitals, 80
+// frequencies (50000 fields) 1.23 + 3 x 1.34 -> 1.43 ms.  Bound by the load, line and store phases following
+// one another: a 20^3 field fills the CU's LDS, so that nothing runs beside them.
+constexpr int DFT_LDS = 10240;  // complex values of the largest padded field (the CU's 160 KB)
+constexpr int DFT_MAX = 24;     // longest axis
+
+// cos and sin of 2 pi j / n, folded to constants by the compiler (j and n are literals after unrolling)
+__device__ __forceinline__ double cos2pi(int j, int n) { return __builtin_cos(6.283185307179586476925 * j / n); }
+__device__ __forceinline__ double sin2pi(int j, int n) { return __builtin_sin(6.283185307179586476925 * j / n); }
+
+template <int NK>
+__device__ __forceinline__ void dft_line_inplace(z64* __restrict__ x, int stride, double sign) {
+  constexpr int H = (NK - 1) / 2;  // pairs (k, NK - k)
+  constexpr bool EVEN = NK % 2 == 0;
+  z64 v[NK];
+#pragma unroll
+  for (int k = 0; k < NK; ++k) v[k] = x[k * stride];
+#pragma unroll
+  for (int k = 1; k <= H; ++k) {
+    const z64 a = v[k], b = v[NK - k], m = csub(a, b);
+    v[k] = cadd(a, b);
+    v[NK - k] = mk(-sign * m.im, sign * m.re);  // sign i m
+  }
+#pragma unroll
+  for (int R = 0; R <= NK / 2; ++R) {
+    z64 c = v[0], s = mk(0.0, 0.0);
+    if (EVEN) c = (R % 2) ? csub(c, v[NK / 2]) : cadd(c, v[NK / 2]);
+#pragma unroll
+    for (int k = 1; k <= H; ++k) {
+      // the angle 2 pi j / NK folded to j <= NK / 2, so that few distinct constants stay in registers
+      const int j = R * k % NK, jj = 2 * j > NK ? NK - j : j;
+      const double co = cos2pi(jj, NK), si = 2 * j > NK ? -sin2pi(jj, NK) : sin2pi(jj, NK);
+      c.re = fma(co, v[k].re, c.re);
+      c.im = fma(co, v[k].im, c.im);
+      if (R > 0 && 2 * R != NK) {
+        s.re = fma(si, v[NK - k].re, s.re);
+        s.im = fma(si, v[NK - k].im, s.im);
+      }
+    }
+    x[R * stride] = cadd(c, s);
+    if (R > 0 && 2 * R != NK) x[(NK - R) * stride] = csub(c, s);
+  }
+}
+
+__device__ __forceinline__ void dft_line_n(int n, z64* x, int stride, double sign) {
+  switch (n) {
+#define ADGA_DLN(NK) \
+  case NK: dft_line_inplace<NK>(x, stride, sign); break;
+    ADGA_DLN(2) ADGA_DLN(3) ADGA_DLN(4) ADGA_DLN(5) ADGA_DLN(6) ADGA_DLN(7) ADGA_DLN(8) ADGA_DLN(9) ADGA_DLN(10)
+    ADGA_DLN(11) ADGA_DLN(12) ADGA_DLN(13) ADGA_DLN(14) ADGA_DLN(15) ADGA_DLN(16) ADGA_DLN(17) ADGA_DLN(18)
+    ADGA_DLN(19) ADGA_DLN(20) ADGA_DLN(21) ADGA_DLN(22) ADGA_DLN(23) ADGA_DLN(24)
+#undef ADGA_DLN
+    default: break;  // a single point
+  }
+}
+
+// What a field is made of: itself (`a`), the bubble's product of transforms
+// a = Ghat(nu_d)_il(-R) times b = Ghat(nu_d - omega)_k'j(R) for field (d, c = (i l)(k' j)), or that product's
+// derivative a(-R) db(R) + da(-R) b(R).
+enum { DFT_FIELD = 0, DFT_PRODUCT = 1, DFT_DERIVATIVE = 2 };
+struct DftSource {
+  const z64* a;
+  const z64* da;       // the derivative's table
+  int n2;
+  long a0, b0;         // first field of the nu and of the nu - omega table
+};
+
+template <int SRC>
+__global__ void __launch_bounds__(512) k_dft3_lds(int nx, int ny, int nz, double sign, DftSource src,
+                                                  z64* __restrict__ out) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char dft_lds[];
+  z64* x = reinterpret_cast<z64*>(dft_lds);
+  const int t = threadIdx.x, nt = blockDim.x;
+  const int per = nx * ny * nz, pz = nz | 1, pyz = ny * pz;
+  const long f = blockIdx.x;
+  // element e = t + i nt is (row r, z): its row and z advance by fixed amounts, no division per element
+  const int r0 = t / nz, z0 = t % nz, dr = nt / nz, dz = nt % nz;
+  auto next = [&](int& r, int& z) {
+    r += dr;
+    z += dz;
+    if (z >= nz) {
+      z -= nz;
+      ++r;
+    }
+  };
+  if constexpr (SRC != DFT_FIELD) {
+    const int n2 = src.n2, n4 = n2 * n2, c = (int)(f % n4);
+    const long d = f / n4;
+    const z64* a = src.a + (src.a0 + d * n2 + c / n2) * per;
+    const z64* b = src.a + (src.b0 + d * n2 + c % n2) * per;
+    const z64* da = src.da + (src.a0 + d * n2 + c / n2) * per;
+    const z64* db = src.da + (src.b0 + d * n2 + c % n2) * per;
+    int r = r0, z = z0, ry = r0 % ny, rx = r0 / ny;
+    const int dx = dr / ny, dy = dr % ny;
+#pragma unroll 4
+    for (int e = t; e < per; e += nt) {
+      const int m = (z ? nz - z : 0) + ((ry ? ny - ry : 0) + (rx ? nx - rx : 0) * ny) * nz;  // -R
+      z64 v;
+      if constexpr (SRC == DFT_PRODUCT) v = cmul(a[m], b[e]);
+      else v = cadd(cmul(a[m], db[e]), cmul(da[m], b[e]));
+      x[r * pz + z] = v;
+      const int rp = r;
+      next(r, z);
+      ry += dy + (r - rp - dr);
+      rx += dx;
+      if (ry >= ny) {
+        ry -= ny;
+        ++rx;
+      }
+    }
+  } else {
+    const z64* in = src.a + f * per;
+    int r = r0, z = z0;
+#pragma unroll 4
+    for (int e = t; e < per; e += nt) {
+      x[r * pz + z] = in[e];
+      next(r, z);
+    }
+  }
+  __syncthreads();
+  for (int axis = 0; axis < 3; ++axis) {
+    const int n = axis == 0 ? nx : axis == 1 ? ny : nz, lines = per / n;
+    const int stride = axis == 0 ? pyz : axis == 1 ? pz : 1;
+    for (int l = t; l < lines; l += nt) {
+      // lanes over z for the x and y passes, over y for the z pass, then the remaining axis
+      const int base = axis == 0 ? (l / nz) * pz + l % nz : axis == 1 ? (l / nz) * pyz + l % nz : l * pz;
+      dft_line_n(n, x + base, stride, sign);
+    }
+    __syncthreads();
+  }
+  z64* o = out + f * per;
+  int r = r0, z = z0;
+#pragma unroll 4
+  for (int e = t; e < per; e += nt) {
+    o[e] = x[r * pz + z];
+    next(r, z);
+  }
+}
+
+// Whether a field's transform runs in LDS: axes of at most 24 points (the lines' register form) and a padded
+// field within the LDS; else the three passes over HBM.
+bool dft_in_lds(const Geom& g) {
+  return g.nkx <= DFT_MAX && g.nky <= DFT_MAX && g.nkz <= DFT_MAX && g.nkx * g.nky * (g.nkz | 1) <= DFT_LDS;
+}
+
+template <int SRC>
+static void dft3_lds(const Geom& g, long nfield, int sign, const DftSource& src, z64* out, hipStream_t s) {
+  const int per = g.nkx * g.nky * g.nkz, lines = per / std::min({g.nkx, g.nky, g.nkz});
+  const int nt = std::min(512, std::max(64, (lines + 63) / 64 * 64));
+  hipLaunchKernelGGL(k_dft3_lds<SRC>, dim3((unsigned)nfield), dim3(nt), (size_t)g.nkx * g.nky * (g.nkz | 1) * sizeof(z64),
+                     s, g.nkx, g.nky, g.nkz, sign > 0 ? 1.0 : -1.0, src, out);
+}
+
+// The transform of the fields in a, in b (a is scratch).
 void dft3(const Geom& g, long nfield, int sign, const z64* tw, z64* a, z64* b, hipStream_t s) {
+  if (nfield <= 0) return;
+  if (dft_in_lds(g)) {
+    dft3_lds<DFT_FIELD>(g, nfield, sign, DftSource{a, nullptr, 0, 0, 0}, b, s);
+    return;
+  }
   dft_pass(nfield, g.nkx, g.nky, g.nkz, 2, sign, tw, a, b, s);
   dft_pass(nfield, g.nkx, g.nky, g.nkz, 1, sign, tw, b, a, s);
   dft_pass(nfield, g.nkx, g.nky, g.nkz, 0, sign, tw, a, b, s);
@@ -162,7 +333,16 @@ __global__ void k_bub_prod(Geom g, int iwb, const z64* __restrict__ ghat, z64* _
   P[idx] = cmul(a[mR], b[R]);
 }
 
+// the first fields of the tables G(nu) and G(nu - omega) of the box
+static DftSource bubble_source(const Geom& g, int iwb, const z64* ghat, const z64* dghat) {
+  return DftSource{ghat, dghat, g.n2, (long)(-g.iwf - g.glo) * g.n2, (long)(-g.iwf - iwb - g.glo) * g.n2};
+}
+
 void launch_bubble_all(const Geom& g, int iwb, const z64* tw, const z64* ghat, z64* P, z64* out, hipStream_t s) {
+  if (dft_in_lds(g)) {
+    dft3_lds<DFT_PRODUCT>(g, (long)g.nf * g.n4, -1, bubble_source(g, iwb, ghat, nullptr), out, s);
+    return;
+  }
   long tot = (long)g.nf * g.n4 * g.nkp;
   hipLaunchKernelGGL(k_bub_prod, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s, g, iwb, ghat, P);
   dft3(g, (long)g.nf * g.n4, -1, tw, P, out, s);
@@ -189,6 +369,10 @@ __global__ void k_bub_prod_tangent(Geom g, int iwb, const z64* __restrict__ ghat
 
 void launch_bubble_all_tangent(const Geom& g, int iwb, const z64* tw, const z64* ghat, const z64* dghat, z64* P,
                                z64* out, hipStream_t s) {
+  if (dft_in_lds(g)) {
+    dft3_lds<DFT_DERIVATIVE>(g, (long)g.nf * g.n4, -1, bubble_source(g, iwb, ghat, dghat), out, s);
+    return;
+  }
   long tot = (long)g.nf * g.n4 * g.nkp;
   hipLaunchKernelGGL(k_bub_prod_tangent, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s, g, iwb, ghat, dghat, P);
   dft3(g, (long)g.nf * g.n4, -1, tw, P, out, s);
