@@ -977,7 +977,7 @@ int adga_get_sigma(adga_ctx* c, double* sig_nl, double* sig_dmft, double* sig_hf
     eom_flush(c);
     adga::launch_fill_neg(g, g.nkp_eom, c->sig_nl, s);
     CK(hipGetLastError());
-    if (sig_nl) CK(hipMemcpyAsync(sig_nl, c->sig_nl, sizeof(z64) * g.n2 * g.nf * g.nkp_eom, hipMemcpyDeviceToHost, s));
+    if (sig_nl) download(c, sig_nl, c->sig_nl, (size_t)g.n2 * g.nf * g.nkp_eom);
     if (sig_dmft) CK(hipMemcpyAsync(sig_dmft, c->sig_dmft, sizeof(z64) * g.n2 * g.nf, hipMemcpyDeviceToHost, s));
     if (sig_hf) CK(hipMemcpyAsync(sig_hf, c->sig_hf, sizeof(z64) * g.n2 * g.nkp_eom, hipMemcpyDeviceToHost, s));
     CK(hipStreamSynchronize(s));

@@ -32,10 +32,6 @@ void ensure_tangent_batch(adga_ctx* c, int nb) {
   c->t_cap = nb;
 }
 
-void download(double* h, const z64* d, size_t count, hipStream_t s) {
-  CK(hipMemcpyAsync(h, d, count * sizeof(z64), hipMemcpyDeviceToHost, s));
-}
-
 }  // namespace
 
 namespace adga_host {
@@ -265,8 +261,7 @@ int adga_get_sigma_tangent(adga_ctx* c, double* dsigma_nl) {
     flush_eom(c);  // the pending omega's EOM and its derivatives
     for (int dir = 0; dir < c->ndir; ++dir) adga::launch_fill_neg(g, g.nkp_eom, c->t_sig + dir * nsig, s);
     CK(hipGetLastError());
-    download(dsigma_nl, c->t_sig, nsig * c->ndir, s);
-    CK(hipStreamSynchronize(s));
+    download(c, dsigma_nl, c->t_sig, nsig * c->ndir);
     return ADGA_OK;
   });
 }

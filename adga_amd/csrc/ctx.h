@@ -13,6 +13,7 @@
 
 #include "adga_amd.h"
 #include "adga_kernels.h"
+#include "hostcopy.h"
 
 using adga::c32;
 using adga::Geom;
@@ -135,6 +136,7 @@ struct adga_ctx {
   // device staging of caller arrays for the module-level entry points (api_modules.cpp)
   z64* stage[6] = {};
   size_t stage_n[6] = {};
+  adga_host::HostCopy hostcopy;  // pinned slots of large copies
   adga::LuTimer lut;       // events around the dominant GEMM kernel's launches
 };
 
@@ -188,6 +190,11 @@ void dfree(T*& p) {
 }
 inline void upload(z64* d, const double* h, size_t count, hipStream_t s) {
   CK(hipMemcpyAsync(d, h, count * sizeof(z64), hipMemcpyHostToDevice, s));
+}
+
+// the device's array into the caller's, complete on return
+inline void download(adga_ctx* c, double* h, const z64* d, size_t count) {
+  CK(c->hostcopy.to_host(h, d, count * sizeof(z64), c->stream));
 }
 
 inline int fail(adga_ctx* c, int code, const char* msg) {

@@ -117,3 +117,23 @@ def test_gpu_series_refuses_what_the_lu_refuses():
             ctx.run_points([1], "fp64")
     assert e.value.code == 1
     assert np.isfinite(inp.mu)
+
+
+@pytest.mark.parametrize("nk", [(16, 16, 16), (17, 19, 12)], ids=["16x16x16", "17x19x12"])
+def test_gpu_large_self_energy_download(nk):
+    """A self-energy above 16 MB comes back through pinned chunks, whole and partial ones (16.8 and 16.0 MB in
+    chunks of 2 MB): equal to the context's own sum over it, bit for bit on a second read."""
+    from adga_amd import api
+    wl = _workload(2, nk, 32, 1e-3)
+    inp = synth.build_inputs(wl)
+    pts = [(1, q) for q in (0, 5, 77)]
+    print(f"download {nk}", flush=True)
+    with api.Context(inp) as ctx:
+        a = api.run_loop(ctx, pts, lambda w, c: synth.chi_loc(inp, w, c), "fp64")["sigma_nl"]
+        b = ctx.get_sigma()[0]
+        loc = ctx.get_sigma_g_loc()[0]
+    assert a.nbytes > 15.5e6 and np.array_equal(a, b)
+    mean = a.mean(axis=3)
+    for i in range(2):
+        mean[i, i] += inp.siw[inp.iwmax - 32:inp.iwmax + 32, i]
+    assert rel_err(loc, mean) < 1e-13
