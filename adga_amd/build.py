@@ -14,7 +14,7 @@ ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libadga_amd.so")
-SOURCES = ["local.hip", "bse.hip", "lu.hip", "eom.hip", "kconv.hip", "onep.hip", "vq.hip", "modules.hip", "tangent.hip",
+SOURCES = ["local.hip", "bse.hip", "lu.hip", "gj.hip", "eom.hip", "kconv.hip", "onep.hip", "vq.hip", "modules.hip", "tangent.hip",
            "tail.hip", "lambda.hip", "inverse_noalloc.hip", "api.cpp", "api_modules.cpp", "api_tangent.cpp",
            "api_lambda.cpp", "hostcopy.cpp"]
 

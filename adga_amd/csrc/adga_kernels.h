@@ -39,8 +39,12 @@ bool lu_supported(int N);  // whether N is in the LU's range
 std::vector<int> lu_ops_factor(int N, int W);
 // factor + forward elimination of the right-hand-side columns [N, W) only (no backward substitution)
 std::vector<int> lu_ops_factor_fwd(int N, int W);
-// the same list as lu_ops_factor written into buf (at most cap ints); returns the number of ints the list needs
-size_t lu_ops_factor_into(int N, int W, int* buf, size_t cap);
+// The inverse of one n x n row-major complex128 matrix in A (gj.hip), n <= gj_max_n(): A, B and C are n x n,
+// G gj_scratch(n) complex, piv and pos n ints; returns the buffer, A or B, that holds it.  *info: the first column
+// without a pivot (1-based; the result is then undefined), or 0.
+int gj_max_n();
+size_t gj_scratch(int n);
+z64* launch_gj_inverse(int n, z64* A, z64* B, z64* C, z64* G, int* piv, int* pos, int* info, hipStream_t s);
 // Events around the launches of the BSE solve's dominant kernel (the factorisation's largest GEMM tile shape,
 // or the iteration's residual product):
 // mark() records one event; collect() (after the stream has completed) returns the summed

@@ -1141,6 +1141,20 @@ int adga_inverse_matrix_z(int n, double* m, int* ierr) {
   *ierr = 0;
   if (n > ADGA_INVERSE_MAX_N) return ADGA_E_ARG;  // the batched LU's largest size (pivot table in LDS)
   return guarded(nullptr, [&]() -> int {
+    if (n <= adga::gj_max_n()) {
+      // the Fortran matrix read row-major is its transpose, and so is the inverse
+      const size_t nn = (size_t)n * n;
+      DevBuf<> d(3 * nn + adga::gj_scratch(n) + n + 1);  // the buffers, G, and 2 n + 1 ints
+      z64 *a = d.p, *b = a + nn, *e = b + nn, *g = e + nn;
+      int *piv = reinterpret_cast<int*>(g + adga::gj_scratch(n)), *pos = piv + n, *info = pos + n;
+      CK(hipMemcpyAsync(a, m, sizeof(z64) * nn, hipMemcpyHostToDevice, nullptr));
+      const z64* x = adga::launch_gj_inverse(n, a, b, e, g, piv, pos, info, nullptr);
+      CK(hipGetLastError());
+      CK(hipMemcpy(ierr, info, sizeof(int), hipMemcpyDeviceToHost));
+      if (*ierr != 0) return ADGA_E_SINGULAR;
+      CK(hipMemcpy(m, x, sizeof(z64) * nn, hipMemcpyDeviceToHost));
+      return ADGA_OK;
+    }
     const int W = 2 * n, ldm = (W + 15) / 16 * 16;
     std::vector<z64> h((size_t)n * ldm);
     const z64* src = reinterpret_cast<const z64*>(m);

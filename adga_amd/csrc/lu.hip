@@ -25,6 +25,7 @@
 
 #include "adga_kernels.h"
 #include "mfma_gemm.h"
+#include "wave_ops.h"
 
 namespace adga {
 
@@ -76,67 +77,6 @@ __global__ void __launch_bounds__(WR * WC * 64) k_gemm3m(int nmat, int ntc, int 
   gemm3m_tile<T, TMT, TNT, WR, WC, KC>(
       M + (long)r0 * ldm + k0, ldm, M + (long)k0 * ldm + c0, ldm, [=](int r, int c) { return Cp[r * ldm + c]; },
       [=](int r, int c, cplx<T> v) { Cp[r * ldm + c] = v; }, m, n, K, false, true, rt, ct, lds);
-}
-
-// component-wise select of two complex values (a select of whole structs can turn into a select of
-// their addresses, which forces register arrays into scratch memory)
-template <typename T>
-__device__ __forceinline__ cplx<T> csel(bool c, cplx<T> a, cplx<T> b) {
-  return mk<T>(c ? a.re : b.re, c ? a.im : b.im);
-}
-
-// Lane moves inside 16-lane rows (DPP row_ror) and reductions over a row: every lane of the row
-// ends with the row's result.
-template <int CTRL>
-__device__ __forceinline__ int dpp_i(int v) {
-  return __builtin_amdgcn_update_dpp(v, v, CTRL, 0xf, 0xf, false);
-}
-template <int CTRL>
-__device__ __forceinline__ float dpp_v(float v) {
-  return __int_as_float(dpp_i<CTRL>(__float_as_int(v)));
-}
-template <int CTRL>
-__device__ __forceinline__ double dpp_v(double v) {
-  const long long b = __double_as_longlong(v);
-  const int lo = dpp_i<CTRL>((int)b), hi = dpp_i<CTRL>((int)(b >> 32));
-  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
-}
-template <typename T>
-__device__ __forceinline__ T row_max(T v) {  // no NaN among the values
-  T o = dpp_v<0x121>(v);
-  v = o > v ? o : v;
-  o = dpp_v<0x122>(v);
-  v = o > v ? o : v;
-  o = dpp_v<0x124>(v);
-  v = o > v ? o : v;
-  o = dpp_v<0x128>(v);
-  return o > v ? o : v;
-}
-__device__ __forceinline__ int row_min(int v) {
-  v = min(v, dpp_i<0x121>(v));
-  v = min(v, dpp_i<0x122>(v));
-  v = min(v, dpp_i<0x124>(v));
-  return min(v, dpp_i<0x128>(v));
-}
-template <typename T>
-__device__ __forceinline__ T lane_value(T v, int l);
-template <>
-__device__ __forceinline__ float lane_value(float v, int l) {
-  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
-}
-template <>
-__device__ __forceinline__ double lane_value(double v, int l) {
-  const long long b = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_readlane((int)b, l), hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
-  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
-}
-// the wave's maximum, the same value in every lane
-template <typename T>
-__device__ __forceinline__ T wave_max(T v) {
-  v = row_max(v);
-  const T a = lane_value(v, 0), b = lane_value(v, 16), c = lane_value(v, 32), d = lane_value(v, 48);
-  const T ab = a > b ? a : b, cd = c > d ? c : d;
-  return ab > cd ? ab : cd;
 }
 
 // Panel LDS (NW waves)
@@ -761,18 +701,12 @@ __global__ void __launch_bounds__(NTS) k_lu_solve(int N, int nrhs, int ns, int n
 // ---------------------------------------------------------------- host: operation lists
 namespace {
 
-// operation list: a growing vector, or (buf non-null) a caller's fixed array of cap ints, in which
-// case n still counts every int the list needs
+// operation list
 struct Ops {
   std::vector<int> v;
-  int* buf = nullptr;
-  size_t cap = 0, n = 0;
   void add(int ty, int a, int b, int c, int d, int e = 0, int f = 0) {
-    int o[8] = {ty, a, b, c, d, e, f, 0};
-    if (!buf) v.insert(v.end(), o, o + 8);
-    else if (n + 8 <= cap)
-      for (int i = 0; i < 8; ++i) buf[n + i] = o[i];
-    n += 8;
+    const int o[8] = {ty, a, b, c, d, e, f, 0};
+    v.insert(v.end(), o, o + 8);
   }
 };
 
@@ -862,15 +796,6 @@ std::vector<int> lu_ops_factor_fwd(int N, int W) {
   Ops ops;
   rec_lu(ops, N, W, 0, N, true);
   return ops.v;
-}
-
-size_t lu_ops_factor_into(int N, int W, int* buf, size_t cap) {
-  Ops ops;
-  ops.buf = buf;
-  ops.cap = cap;
-  rec_lu(ops, N, W, 0, N, true);
-  if (W > N) rec_trsm_u(ops, 0, N, N, W);
-  return ops.n;
 }
 
 namespace {
