@@ -69,7 +69,7 @@ void tangent_batch(adga_ctx* c, int nb, int p0, int npts, const std::vector<int>
     // of the omega at once by k-grid convolution (formed again, not stored from the forward pass, and kept
     // for the omega's next batches), or as direct sums per batch, as the forward bubble's mode chooses
     const bool t_hit = c->t_bub_valid && c->t_bub_iwb == c->iwb && c->t_bub_iwf == g.iwf;
-    if (c->t_dghat && (c->bubble_mode == 1 || (c->bubble_mode == 2 && (t_hit || nb >= 64)))) {
+    if (c->t_dghat && (c->bubble_mode == 1 || (c->bubble_mode == 2 && (t_hit || nb >= bubble_dft_points(c))))) {
       const size_t nall = (size_t)G.nf * G.n4 * G.nkp;  // sized for the largest box
       if (!t_hit) {
         if (dir == 0) {

@@ -19,7 +19,7 @@ namespace adga {
 // ---------------------------------------------------------------- A3: bubble
 // chi0q[b][d](i1 = i*n + j, i2 = l*n + k') = -beta/nkp sum_K G(K, nu_d)_il G(K - q_b, nu_d - omega)_k'j
 // (accumulate_chi0, one_particle_quant_module.f90:274-288; k-sum main.F90:647-657).
-// One block per (nu, point); thread = ((i,l), k-slice); n^2 accumulators per thread.
+// n <= 2: one block per (nu, point); thread = ((i,l), k-slice); n^2 accumulators per thread.
 // gt2 is the table of the second factor G(K - q, nu - omega) (gt itself, or a derivative table when the
 // tangent of the bubble is formed by the product rule); accumulate adds into chi0q.
 template <int NN>
@@ -66,19 +66,162 @@ __global__ void __launch_bounds__(256) k_bubble(Geom g, int iwb, const int* __re
   }
 }
 
+// The same on the FP64 matrix cores for n >= 3: at one nu and q a product of inner size nkp, the rows (i, l) and
+// columns (k', j) of the tables G(K, nu) and G(K - q, nu - omega) being the n^2 contiguous values of one K, in the
+// 16 lanes of an MFMA's operand as they lie in memory (n = 3, 4: one 16 x 16 tile, 5: 2 x 2).  A workgroup of
+// BUB_NW waves takes QB points at one nu, the points sharing the loads of the first factor and the indices of K;
+// wave w takes K = 4 w .. 4 w + 3 of every 4 BUB_NW and the waves' sums meet in LDS.  Workgroups of one nu follow
+// one another on one XCD, whose L2 then holds the two tables.
+// Bound by the matrix rate on padded tiles (n = 3: 9 of 16 rows and columns; 45 .. 53 TFLOP/s of padded products).
+// 5 orbitals, 16^3 k, 160 frequencies, 48 points: 10.2 ms with one thread per (i, l) and slice of k -> 4.97;
+// 4 orbitals, 12^3, 40 frequencies, 48 points: 0.61 -> 0.33; 3 orbitals, 20^3, 60 frequencies, 41 points: 1.03 ->
+// 0.93, one point 0.24 -> 0.17.
+constexpr int BUB_NW = 8;
+template <int NN, int QB>
+__global__ void __launch_bounds__(BUB_NW * 64) k_bubble_mm(Geom g, int iwb, int npts, int nqg,
+                                                           const int* __restrict__ qidx, const z64* __restrict__ gt,
+                                                           const z64* __restrict__ gt2, z64* __restrict__ chi0q,
+                                                           int accumulate) {
+  using M = Mfma<double>;
+  constexpr int N2 = NN * NN, T = (N2 + 15) / 16, STEP = 4 * BUB_NW;
+  __shared__ double red[BUB_NW][8][64];
+  const int per = (g.nf * nqg + 7) / 8;
+  const int work = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
+  if (work >= g.nf * nqg || (int)(blockIdx.x / 8) >= per) return;
+  const int d = work / nqg, b0 = (work % nqg) * QB;
+  const int lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int nx = g.nkx, ny = g.nky, nz = g.nkz;
+  const z64* g1 = gt + (long)(d - g.iwf - g.glo) * g.nkp * N2;
+  const z64* g2 = gt2 + (long)(d - g.iwf - iwb - g.glo) * g.nkp * N2;
+  int qx[QB], qy[QB], qz[QB];
+#pragma unroll
+  for (int u = 0; u < QB; ++u) {
+    const int q = qidx[min(b0 + u, npts - 1)];  // a partial group repeats its last point
+    qz[u] = q % nz;
+    qy[u] = q / nz % ny;
+    qx[u] = q / (nz * ny);
+  }
+  int el[T];  // a lane beyond the n^2 values repeats the last: its row or column of the tile is not used
+#pragma unroll
+  for (int i = 0; i < T; ++i) el[i] = min(i * 16 + li, N2 - 1);
+  f64x4 re[QB][T][T], im[QB][T][T];
+#pragma unroll
+  for (int u = 0; u < QB; ++u)
+#pragma unroll
+    for (int r = 0; r < T; ++r)
+#pragma unroll
+      for (int c = 0; c < T; ++c)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) re[u][r][c][v] = im[u][r][c][v] = 0.0;
+  // the lane's K and its coordinates, advanced by STEP without divisions
+  int K = 4 * wave + lg, kz = K % nz, ky = K / nz % ny, kx = K / (nz * ny) % nx;
+  const int sz = STEP % nz, sy = STEP / nz % ny, sx = STEP / (nz * ny) % nx;
+  struct Operands {
+    z64 a[T], x[QB][T];
+  };
+  auto fetch = [&](Operands& o) __attribute__((always_inline)) {
+    const int k = min(K, g.nkp - 1);
+#pragma unroll
+    for (int i = 0; i < T; ++i) o.a[i] = g1[k * N2 + el[i]];
+#pragma unroll
+    for (int u = 0; u < QB; ++u) {
+      const int z = kz - qz[u], y = ky - qy[u], w = kx - qx[u];
+      const int kq = (z < 0 ? z + nz : z) + ((y < 0 ? y + ny : y) + (w < 0 ? w + nx : w) * ny) * nz;
+#pragma unroll
+      for (int i = 0; i < T; ++i) o.x[u][i] = g2[kq * N2 + el[i]];
+    }
+    K += STEP;
+    kz += sz;
+    ky += sy;
+    kx += sx;
+    if (kz >= nz) kz -= nz, ++ky;
+    if (ky >= ny) ky -= ny, ++kx;
+    if (kx >= nx) kx -= nx;  // beyond nkp: only kept in range
+  };
+  const int full = g.nkp / STEP, steps = (g.nkp + STEP - 1) / STEP;
+  auto multiply = [&](Operands& o, int step) __attribute__((always_inline)) {
+    if (step >= full && step * STEP + 4 * wave + lg >= g.nkp) {  // no K of this lane's in the last step
+#pragma unroll
+      for (int i = 0; i < T; ++i) o.a[i] = mk(0.0, 0.0);
+    }
+#pragma unroll
+    for (int u = 0; u < QB; ++u)
+#pragma unroll
+      for (int r = 0; r < T; ++r)
+#pragma unroll
+        for (int c = 0; c < T; ++c) {
+          re[u][r][c] = M::op(o.a[r].re, o.x[u][c].re, re[u][r][c]);
+          im[u][r][c] = M::op(o.a[r].re, o.x[u][c].im, im[u][r][c]);
+          re[u][r][c] = M::op(-o.a[r].im, o.x[u][c].im, re[u][r][c]);
+          im[u][r][c] = M::op(o.a[r].im, o.x[u][c].re, im[u][r][c]);
+        }
+  };
+  Operands even, odd;  // the loads of a step are in flight during the products of the one before
+  fetch(even);
+  for (int k = 0; k < steps; k += 2) {
+    fetch(odd);
+    multiply(even, k);
+    if (k + 1 == steps) break;
+    fetch(even);
+    multiply(odd, k + 1);
+  }
+  const double f = -g.beta / g.nkp;
+#pragma unroll
+  for (int u = 0; u < QB; ++u)
+#pragma unroll
+    for (int r = 0; r < T; ++r)
+#pragma unroll
+      for (int c = 0; c < T; ++c) {
+        __syncthreads();
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          red[wave][v][lane] = re[u][r][c][v];
+          red[wave][4 + v][lane] = im[u][r][c][v];
+        }
+        __syncthreads();
+        // wave v < 4: register v of every lane, D[row(lg, v)][li]
+        if (wave < 4 && b0 + u < npts) {
+          z64 s = mk(0.0, 0.0);
+          for (int w = 0; w < BUB_NW; ++w) s = cadd(s, mk(red[w][wave][lane], red[w][4 + wave][lane]));
+          const int il = r * 16 + M::row(lg, wave), kj = c * 16 + li;
+          if (il < N2 && kj < N2) {
+            z64* o = chi0q + ((long)(b0 + u) * g.nf + d) * g.n4 + (il / NN * NN + kj % NN) +
+                     (il % NN * NN + kj / NN) * N2;
+            *o = accumulate ? cadd(*o, cscale(s, f)) : cscale(s, f);
+          }
+        }
+      }
+}
+
 void launch_bubble(const Geom& g, int iwb, int npts, const int* qidx, const z64* gt, z64* chi0q, hipStream_t s,
                    const z64* gt2, bool accumulate) {
-  dim3 grid(g.nf, npts);
   const z64* g2 = gt2 ? gt2 : gt;
   const int acc = accumulate ? 1 : 0;
-  switch (g.n) {
-    case 1: hipLaunchKernelGGL(k_bubble<1>, grid, dim3(256), 0, s, g, iwb, qidx, gt, g2, chi0q, acc); break;
-    case 2: hipLaunchKernelGGL(k_bubble<2>, grid, dim3(256), 0, s, g, iwb, qidx, gt, g2, chi0q, acc); break;
-    case 3: hipLaunchKernelGGL(k_bubble<3>, grid, dim3(256), 0, s, g, iwb, qidx, gt, g2, chi0q, acc); break;
-    case 4: hipLaunchKernelGGL(k_bubble<4>, grid, dim3(256), 0, s, g, iwb, qidx, gt, g2, chi0q, acc); break;
-    case 5: hipLaunchKernelGGL(k_bubble<5>, grid, dim3(256), 0, s, g, iwb, qidx, gt, g2, chi0q, acc); break;
-    default: break;
+  if (g.n >= 3) {
+    // two points per workgroup once that still leaves one for every CU (five orbitals: one point fills the
+    // registers; four points of fewer orbitals: 1.14 ms where two take 0.97)
+    const int QB = g.n == 5 ? 1 : 2;
+    const bool wide = QB > 1 && (long)g.nf * ((npts + QB - 1) / QB) >= 256;
+    const int nqg = wide ? (npts + QB - 1) / QB : npts;
+    const dim3 grid((unsigned)((g.nf * nqg + 7) / 8 * 8)), block(BUB_NW * 64);
+#define ADGA_BUB(NN, QB) \
+  hipLaunchKernelGGL((k_bubble_mm<NN, QB>), grid, block, 0, s, g, iwb, npts, nqg, qidx, gt, g2, chi0q, acc)
+    if (g.n == 3) {
+      if (wide) ADGA_BUB(3, 2);
+      else ADGA_BUB(3, 1);
+    } else if (g.n == 4) {
+      if (wide) ADGA_BUB(4, 2);
+      else ADGA_BUB(4, 1);
+    } else {
+      ADGA_BUB(5, 1);
+    }
+#undef ADGA_BUB
+    return;
   }
+  const dim3 grid(g.nf, npts);
+  if (g.n == 1) hipLaunchKernelGGL(k_bubble<1>, grid, dim3(256), 0, s, g, iwb, qidx, gt, g2, chi0q, acc);
+  else hipLaunchKernelGGL(k_bubble<2>, grid, dim3(256), 0, s, g, iwb, qidx, gt, g2, chi0q, acc);
 }
 
 // ---------------------------------------------------------------- S_nu

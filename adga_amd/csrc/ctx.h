@@ -257,6 +257,8 @@ void free_tangent(adga_ctx* c);
 // the twiddles and the k-grid transform of the G table (formed once); the pending omega's EOM flushed
 // (with its derivatives when tangent directions are set) (api.cpp)
 void conv_tables(adga_ctx* c);
+// points of a batch from which the bubble is formed for every q at once
+int bubble_dft_points(const adga_ctx* c);
 void flush_eom(adga_ctx* c);
 
 }  // namespace adga_host
