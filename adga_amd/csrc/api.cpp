@@ -1028,20 +1028,6 @@ int adga_get_nfock(adga_ctx* c, double* n_fock) {
   });
 }
 
-// The context's own sigma_sum in `ds` (n2 * 2 iwfmax_small * nkp_eom): the accumulated Sigma_nl (the pending
-// EOM convolved, the negative frequencies filled as adga_get_sigma does) plus siw on the orbital diagonal,
-// as add_siw_dmft forms it (src/eom_module.f90:237-251, src/main.F90:869) - a device copy instead of the
-// caller's array crossing PCIe.
-void own_sigma_sum(adga_ctx* c, z64* ds) {
-  const Geom& g = c->g;
-  eom_flush(c);
-  adga::launch_fill_neg(g, g.nkp_eom, c->sig_nl, c->stream);
-  CK(hipGetLastError());
-  CK(hipMemcpyAsync(ds, c->sig_nl, sizeof(z64) * g.n2 * g.nf * g.nkp_eom, hipMemcpyDeviceToDevice, c->stream));
-  adga::launch_add_siw(g, g.nkp_eom, c->siw, ds, c->stream);
-  CK(hipGetLastError());
-}
-
 int adga_get_sigma_g_loc(adga_ctx* c, const double* sigma_sum, double* sigma_loc, double* gloc) {
   if (!c) return ADGA_E_ARG;
   const Geom& g = c->g;
@@ -1051,13 +1037,18 @@ int adga_get_sigma_g_loc(adga_ctx* c, const double* sigma_sum, double* sigma_loc
   }
   return guarded(c, [&]() -> int {
     const size_t ns = (size_t)g.n2 * g.nf * g.nkp, nl = (size_t)g.n2 * g.nf, ng = (size_t)2 * g.iwmax * g.n2;
-    DevBuf<> ds(ns), dl(nl), dg(ng), dw(adga::op_sigma_loc_scratch(g));
-    if (sigma_sum)
-      upload(ds.p, sigma_sum, ns, c->stream);
+    // without the caller's array the context's own: the accumulated Sigma_nl (the pending EOM convolved) plus siw
+    // (src/main.F90:869), read where it lies
+    const bool own = !sigma_sum;
+    DevBuf<> ds(own ? 0 : ns), dl(nl), dg(ng), dw(adga::op_sigma_loc_scratch(g));
+    if (own)
+      eom_flush(c);
     else
-      own_sigma_sum(c, ds.p);
-    const int rc = op_finish(
-        c, adga::launch_op_sigma_g_loc(g, c->hk, c->siw, c->dc, ds.p, dl.p, dg.p, dw.p, c->stream), "get_sigma_g_loc");
+      upload(ds.p, sigma_sum, ns, c->stream);
+    const int rc = op_finish(c,
+                             adga::launch_op_sigma_g_loc(g, c->hk, c->siw, c->dc, own ? c->sig_nl : ds.p, own, dl.p,
+                                                         dg.p, dw.p, c->stream),
+                             "get_sigma_g_loc");
     if (rc != ADGA_OK) return rc;
     if (sigma_loc) CK(hipMemcpyAsync(sigma_loc, dl.p, sizeof(z64) * nl, hipMemcpyDeviceToHost, c->stream));
     if (gloc) CK(hipMemcpyAsync(gloc, dg.p, sizeof(z64) * ng, hipMemcpyDeviceToHost, c->stream));
@@ -1071,13 +1062,16 @@ int adga_get_ndga(adga_ctx* c, const double* sigma_sum, double* n_dga_k, double*
   return guarded(c, [&]() -> int {
     const Geom& g = c->g;
     const size_t ns = (size_t)g.n2 * g.nf * g.nkp_eom, nk = (size_t)g.nkp_eom * g.n2;
-    DevBuf<> ds(ns), dk(nk), dn((size_t)g.n);
-    if (sigma_sum)
-      upload(ds.p, sigma_sum, ns, c->stream);
+    const bool own = !sigma_sum;
+    DevBuf<> ds(own ? 0 : ns), dk(nk), dn((size_t)g.n);
+    if (own)
+      eom_flush(c);
     else
-      own_sigma_sum(c, ds.p);
-    const int rc = op_finish(
-        c, adga::launch_op_ndga(g, c->hk, c->siw, c->dc, c->keom, ds.p, dk.p, dn.p, c->stream), "get_ndga");
+      upload(ds.p, sigma_sum, ns, c->stream);
+    const int rc = op_finish(c,
+                             adga::launch_op_ndga(g, c->hk, c->siw, c->dc, c->keom, own ? c->sig_nl : ds.p, own, dk.p,
+                                                  dn.p, c->stream),
+                             "get_ndga");
     if (rc != ADGA_OK) return rc;
     if (n_dga_k) CK(hipMemcpyAsync(n_dga_k, dk.p, sizeof(z64) * nk, hipMemcpyDeviceToHost, c->stream));
     if (n_dga) CK(hipMemcpyAsync(n_dga, dn.p, sizeof(z64) * g.n, hipMemcpyDeviceToHost, c->stream));
