@@ -194,6 +194,15 @@ void launch_bubble_outer_add(const Geom& g, int npts, const int* qidx, const z64
 void launch_chi_phys(int n, long npts, const z64* chi, z64* out, hipStream_t s);
 void launch_lambda_sums(long npts, int nl, int nblk, double scale, const double* lams, const z64* chi, z64* part,
                         z64* out, hipStream_t s);
+// A solve of the sum rule (lambda.hip): lambda, its bracket [a, b] and the counts of the iteration
+enum LambdaStatus { LAMBDA_RUNNING = 0, LAMBDA_DONE, LAMBDA_MAXIT, LAMBDA_NO_BRACKET, LAMBDA_NONFINITE };
+struct LambdaState {
+  double lam, a, b, target, ftol;
+  int bracket, tries, k, maxit, iters, status;
+};
+void launch_lambda_init(const LambdaState& init, LambdaState* st, hipStream_t s);
+// one evaluation and the step it leads to; nothing once st->status is set
+void launch_lambda_newton(long npts, int nblk, double scale, LambdaState* st, const z64* chi, z64* part, hipStream_t s);
 void launch_lambda_apply(long npts, double lam, const z64* chi, z64* out, hipStream_t s);
 
 }  // namespace adga

@@ -1,7 +1,7 @@
 // The lambda correction of the final susceptibility (no counterpart in the reference): C-ABI entry points
 // adga_lambda_*.  The physical susceptibility of every (q, omega) point stays on the device; each evaluation
-// of the sum rule is one pair of FP64 reductions there (lambda.hip), and lambda is found on the host by a
-// safeguarded Newton iteration on f(lambda) = Re S(lambda) - target, S(lambda) = 1/(beta nqp) sum chi^lambda:
+// of the sum rule is one pair of FP64 reductions there (lambda.hip), and lambda is found there by a safeguarded
+// Newton iteration on f(lambda) = Re S(lambda) - target, S(lambda) = 1/(beta nqp) sum chi^lambda:
 // f decreases from +inf at the pole lambda_min = -1/max Re chi(q, omega = 0) and is convex there for
 // positive susceptibilities, so a Newton step that leaves the bracket [a, b] (f(a) > 0 > f(b)) is replaced
 // by bisection.
@@ -27,6 +27,7 @@ struct adga_lambda {
   z64* part = nullptr;     // partial sums
   z64* out = nullptr;      // final sums
   double* lams = nullptr;  // the lambdas of one call
+  adga::LambdaState* state = nullptr;  // a solve's iteration
   int cap = 0;             // lambdas the buffers hold
   int nblk = 256;
   hipStream_t s = nullptr;
@@ -79,6 +80,7 @@ void release(adga_lambda* h) {
   lfree(h->part);
   lfree(h->out);
   lfree(h->lams);
+  lfree(h->state);
   if (h->s) (void)hipStreamDestroy(h->s);
   h->s = nullptr;
 }
@@ -190,50 +192,32 @@ int adga_lambda_solve(adga_lambda* h, double target, double tol, int maxit, doub
   if (!h || !lambda || !(tol > 0) || maxit < 1 || !std::isfinite(target)) return ADGA_E_ARG;
   return lam_guarded(h, [&]() -> int {
     const double scale = 1.0 / (h->beta * h->nqp);
-    auto f = [&](double lam, double* df) {
-      z64 res[2];
-      sums(h, h->chi, h->npts, scale, 1, &lam, res);
-      if (!std::isfinite(res[0].re) || !std::isfinite(res[1].re)) throw NonFinite{};
-      *df = res[1].re;
-      return res[0].re - target;
-    };
+    ensure_cap(h, 1);
+    if (!h->state) lalloc(&h->state, 1);
     // bracket: a just above the pole (f -> +inf), b where f < 0
-    double a = h->lmin, b = 1.0, df = 0.0;
-    double fb = f(b, &df);
-    int it = 0;
-    while (fb > 0) {
-      if (++it > 200) {
-        h->err = "no lambda above the pole brings the sum below the target";
-        return ADGA_E_NOCONV;
-      }
-      a = b;
-      b = b > 0 ? 4.0 * b : 1.0;
-      fb = f(b, &df);
+    adga::LambdaState st{};
+    st.a = h->lmin;
+    st.lam = st.b = 1.0;
+    st.target = target;
+    st.ftol = tol * std::max(1.0, std::fabs(target));
+    st.bracket = 1;
+    st.maxit = maxit;
+    adga::launch_lambda_init(st, h->state, h->s);
+    // a solve takes some ten evaluations; those queued past its end cost 2 us each
+    for (int n = 12; st.status == adga::LAMBDA_RUNNING; n = 6) {
+      for (int i = 0; i < n; ++i) adga::launch_lambda_newton(h->npts, h->nblk, scale, h->state, h->chi, h->part, h->s);
+      LCK(hipGetLastError());
+      LCK(hipMemcpyAsync(&st, h->state, sizeof(st), hipMemcpyDeviceToHost, h->s));
+      LCK(hipStreamSynchronize(h->s));
     }
-    double x = b, fx = fb, dfx = df;
-    const double ftol = tol * std::max(1.0, std::fabs(target));
-    for (int k = 0; k < maxit; ++k) {
-      if (iters) *iters = k;
-      if (std::fabs(fx) <= ftol) {
-        *lambda = x;
-        return ADGA_OK;
-      }
-      double xn = (dfx < 0) ? x - fx / dfx : 0.5 * (a + b);
-      if (!(xn > a && xn < b)) xn = 0.5 * (a + b);  // Newton left the bracket: bisect
-      x = xn;
-      fx = f(x, &dfx);
-      if (fx > 0)
-        a = x;
-      else
-        b = x;
-      if (b - a <= 4e-16 * std::max(1.0, std::fabs(x))) {
-        if (iters) *iters = k + 1;
-        *lambda = x;
-        return ADGA_OK;
-      }
+    if (iters && !st.bracket) *iters = st.iters;
+    if (st.status == adga::LAMBDA_NONFINITE) throw NonFinite{};
+    if (st.status == adga::LAMBDA_NO_BRACKET) {
+      h->err = "no lambda above the pole brings the sum below the target";
+      return ADGA_E_NOCONV;
     }
-    if (iters) *iters = maxit;
-    *lambda = x;
+    *lambda = st.lam;
+    if (st.status == adga::LAMBDA_DONE) return ADGA_OK;
     h->err = "lambda: no convergence within maxit iterations";
     return ADGA_E_NOCONV;
   });

@@ -86,6 +86,93 @@ void launch_lambda_sums(long npts, int nl, int nblk, double scale, const double*
   hipLaunchKernelGGL(k_lambda_final, dim3(nl), dim3(LAM_THREADS), 0, s, nblk, scale, part, out);
 }
 
+// The safeguarded Newton iteration of a solve, one state machine per solve in device memory: an evaluation is a
+// k_lambda_eval (partial sums at st->lam) and a k_lambda_step (their sum, then the host rule's next lambda or the
+// end), so the host queues several and waits once instead of once per evaluation (11 evaluations of 36288 points:
+// 0.55 ms with a copy to and from the host for each, 0.22 so).  Evaluations queued beyond the end return at once.
+__global__ void k_lambda_init(LambdaState init, LambdaState* __restrict__ st) { *st = init; }
+
+__global__ void __launch_bounds__(LAM_THREADS) k_lambda_eval(long npts, const LambdaState* __restrict__ st,
+                                                             const z64* __restrict__ chi, z64* __restrict__ part) {
+  __shared__ z64 red[2 * LAM_THREADS];
+  if (st->status != LAMBDA_RUNNING) return;
+  const double lam = st->lam;
+  z64 s1 = mk(0.0, 0.0), s2 = mk(0.0, 0.0);
+  for (long p = (long)blockIdx.x * LAM_THREADS + threadIdx.x; p < npts; p += (long)gridDim.x * LAM_THREADS) {
+    const z64 c = chi[p];
+    const z64 cl = cdiv(c, mk(1.0 + lam * c.re, lam * c.im));
+    s1 = cadd(s1, cl);
+    s2 = cadd(s2, cmul(cl, cl));
+  }
+  block_reduce2(s1, s2, red);
+  if (threadIdx.x == 0) {
+    part[blockIdx.x * 2] = s1;
+    part[blockIdx.x * 2 + 1] = s2;
+  }
+}
+
+__global__ void __launch_bounds__(LAM_THREADS) k_lambda_step(int nblk, double scale, const z64* __restrict__ part,
+                                                             LambdaState* __restrict__ state) {
+  __shared__ z64 red[2 * LAM_THREADS];
+  LambdaState st = *state;
+  if (st.status != LAMBDA_RUNNING) return;
+  z64 s1 = mk(0.0, 0.0), s2 = mk(0.0, 0.0);
+  for (int b = threadIdx.x; b < nblk; b += LAM_THREADS) {
+    s1 = cadd(s1, part[b * 2]);
+    s2 = cadd(s2, part[b * 2 + 1]);
+  }
+  block_reduce2(s1, s2, red);
+  if (threadIdx.x != 0) return;
+  const double sum = scale * s1.re, fx = sum - st.target, dfx = -scale * s2.re;
+  auto next = [&] {  // the top of Newton's loop: the end, or the next x
+    st.iters = st.k < st.maxit ? st.k : st.maxit;
+    if (st.k >= st.maxit) {
+      st.status = LAMBDA_MAXIT;
+    } else if (fabs(fx) <= st.ftol) {
+      st.status = LAMBDA_DONE;
+    } else {
+      double xn = dfx < 0 ? st.lam - fx / dfx : 0.5 * (st.a + st.b);
+      if (!(xn > st.a && xn < st.b)) xn = 0.5 * (st.a + st.b);  // Newton left the bracket: bisect
+      st.lam = xn;
+    }
+  };
+  if (!isfinite(sum) || !isfinite(dfx)) {
+    st.status = LAMBDA_NONFINITE;
+  } else if (st.bracket) {  // lam = b of the bracket: f(b) < 0 is looked for
+    if (fx > 0) {
+      if (++st.tries > 200) {
+        st.status = LAMBDA_NO_BRACKET;
+      } else {
+        st.a = st.b;
+        st.b = st.b > 0 ? 4.0 * st.b : 1.0;
+        st.lam = st.b;
+      }
+    } else {
+      st.bracket = 0;
+      next();
+    }
+  } else {
+    (fx > 0 ? st.a : st.b) = st.lam;
+    if (st.b - st.a <= 4e-16 * fmax(1.0, fabs(st.lam))) {
+      st.iters = st.k + 1;
+      st.status = LAMBDA_DONE;
+    } else {
+      ++st.k;
+      next();
+    }
+  }
+  *state = st;
+}
+
+void launch_lambda_init(const LambdaState& init, LambdaState* st, hipStream_t s) {
+  hipLaunchKernelGGL(k_lambda_init, dim3(1), dim3(1), 0, s, init, st);
+}
+
+void launch_lambda_newton(long npts, int nblk, double scale, LambdaState* st, const z64* chi, z64* part, hipStream_t s) {
+  hipLaunchKernelGGL(k_lambda_eval, dim3(nblk), dim3(LAM_THREADS), 0, s, npts, st, chi, part);
+  hipLaunchKernelGGL(k_lambda_step, dim3(1), dim3(LAM_THREADS), 0, s, nblk, scale, part, st);
+}
+
 __global__ void k_lambda_apply(long npts, double lam, const z64* __restrict__ chi, z64* __restrict__ out) {
   const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= npts) return;
