@@ -24,14 +24,17 @@ void launch_bubble(const Geom& g, int iwb, int npts, const int* qidx, const z64*
                    const z64* gt2 = nullptr, bool accumulate = false);
 // Out = C_ch^T Z_ch for the channels ch0 .. ch0 + nch - 1 (C row-major as the left operand, Z and Out in the
 // residual layouts), plus B - Y when B is given, plus Out itself when accumulate; with rmax each matrix's
-// max |Out| as the bits of a double (atomic maximum: cleared by the caller)
+// max |Out| as the bits of a double (atomic maximum: cleared by the caller); rows r0 .. N - 1 of each matrix
 void resid_gemm(const Geom& g, int npts, int ch0, int nch, const z64* cd, const z64* cm, const z64* Z, z64* Out,
                 const z64* B, const z64* Y, hipStream_t s, bool accumulate = false,
-                unsigned long long* rmax = nullptr);
+                unsigned long long* rmax = nullptr, int r0 = 0);
+// the first row of a point's matrices that the EOM reads: nu >= 0 (eom_module.f90:211-227), the upper half
+inline int eom_row0(const Geom& g) { return g.n2 * g.iwf; }
 void launch_smat(const Geom& g, int npts, const z64* chi0q, const z64* winv, z64* S, hipStream_t s);
 template <typename T>
 void launch_build(const Geom& g, int npts, int ldm, const z64* S, const z64* cd, const z64* cm, cplx<T>* M,
                   hipStream_t s);
+// gamma^q_d, the rows eom_row0 .. N - 1
 void launch_gamq(const Geom& g, int npts, const z64* S, const z64* cd, z64* Z, z64* G2, hipStream_t s);
 // the right operand of gamma^q_d's product (S of each point in the residual product's layout)
 void launch_gamq_z(const Geom& g, int npts, const z64* S, z64* Z, hipStream_t s);
@@ -138,7 +141,7 @@ bool launch_gkiw(const Geom& g, int k, int iw, const z64* hk, const z64* siw, co
 void launch_chi_qw(const Geom& g, const z64* X, const z64* Y, z64* chi, hipStream_t s);
 void launch_ndmft(const Geom& g, const z64* giw, z64* nd, hipStream_t s);
 void launch_add_siw(const Geom& g, int nk, const z64* siw, z64* ss, hipStream_t s);
-// with vq non-null: V(q_b) = vq + qpos[b] n4 enters the density eta term and -V gamma^w_d / (beta nqp) is added
+// m_tot at the rows eom_row0 .. N - 1; with vq non-null: V(q_b) = vq + qpos[b] n4 enters the density eta term and -V gamma^w_d / (beta nqp) is added
 void launch_mtot(const Geom& g, int npts, const z64* u, const z64* ut, const z64* eta, const z64* gamq, z64* mt,
                  hipStream_t s, const int* qpos = nullptr, const z64* vq = nullptr, const z64* gamd = nullptr,
                  bool accumulate = false);

@@ -776,7 +776,7 @@ int run_points_impl(adga_ctx* c, int npts, const int* iq, int precision, double*
       }
       adga::launch_smat(g, nb, c->chi0q, c->winv, c->S, s);
       if (vtp) adga::launch_vq_w(g, nb, c->qpos, c->vq, c->chi0q, c->W, s);
-      adga::launch_gamq(g, nb, c->S, c->cd, c->Z, c->gamq, s);
+      if (c->do_eom) adga::launch_gamq(g, nb, c->S, c->cd, c->Z, c->gamq, s);
       adga::launch_rhs(g, nb, c->S, c->cd, c->cm, c->opgd, c->opgm, c->Z, c->Bp, s, vtp);
       CK(hipEventRecord(ev[2], s));
       int iters = 0;

@@ -110,10 +110,11 @@ void tangent_batch(adga_ctx* c, int nb, int p0, int npts, const std::vector<int>
     if (!c->do_eom) continue;
     // d m_tot = m_tot(U, U~; d eta, d gamma^q) + m_tot(dU, dU~; eta, gamma^q), with
     // d gamma^q_d = sum_nu (dS C_d + S dC_d)[nu rows]
+    const int eom0 = adga::eom_row0(g);
     adga::launch_gamq_z(g, nb, c->t_dS, c->t_Z1, s);
-    adga::resid_gemm(g, nb, 0, 1, c->cd, c->cd, c->t_Z1, c->t_dgamq, nullptr, nullptr, s);
+    adga::resid_gemm(g, nb, 0, 1, c->cd, c->cd, c->t_Z1, c->t_dgamq, nullptr, nullptr, s, false, nullptr, eom0);
     adga::launch_gamq_z(g, nb, c->S, c->t_Z1, s);
-    adga::resid_gemm(g, nb, 0, 1, dcd, dcd, c->t_Z1, c->t_dgamq, nullptr, nullptr, s, true);
+    adga::resid_gemm(g, nb, 0, 1, dcd, dcd, c->t_Z1, c->t_dgamq, nullptr, nullptr, s, true, nullptr, eom0);
     adga::launch_mtot(g, nb, c->u, c->ut, c->t_dY, c->t_dgamq, c->t_dmt, s);  // d eta = dY
     adga::launch_mtot(g, nb, c->du + (size_t)dir * G.n4, c->dut + (size_t)dir * G.n4, c->Y, c->gamq, c->t_dmt, s,
                       nullptr, nullptr, nullptr, true);

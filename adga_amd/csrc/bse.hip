@@ -390,7 +390,7 @@ __device__ __forceinline__ unsigned long long umax64(unsigned long long a, unsig
 }
 
 // Out[(2b + ch) N + r][s] = sum_x C_ch(x, r) Z_ch[x][b*n2 + s], plus (B - Y) at the same position
-// when B is given (the residual): complex FP64 products by the 3M method (X = Ar Br, Y = Ai Bi,
+// when B is given (the residual), for the rows r >= r0: complex FP64 products by the 3M method (X = Ar Br, Y = Ai Bi,
 // Z = (Ar + Ai)(Br + Bi), as gemm3m_tile), C read row-major as A(r, x) = C[r N + x], the output in the
 // point-major layout of Y.  With rmax, each matrix's max |Out| goes there from the output registers
 // (abs_bits, combined per column in LDS), instead of a second pass over Out.
@@ -409,20 +409,20 @@ template <int TM, int TN>
 __global__ void __launch_bounds__(256, TM == 64 ? 2 : 4)
 k_resid_gemm(Geom g, int npts, int ch0, int nch, const z64* __restrict__ cd, const z64* __restrict__ cm,
              const z64* __restrict__ Zall, z64* Out, const z64* __restrict__ B, const z64* __restrict__ Y,
-             int accumulate, unsigned long long* __restrict__ rmax) {
+             int accumulate, unsigned long long* __restrict__ rmax, int r0) {
   using V = f64x4;
   constexpr int KC = RG_KC, WR = 2, WC = 2, RB = TM / WR / 16, CB = TN / WC / 16;
   constexpr int LDA = KC + 1, LDB = TN + 8, BUF = TM * LDA + KC * LDB;  // strides without bank conflicts
   constexpr int PA = TM * KC / 256, PB = KC * TN / 256;
   __shared__ __attribute__((aligned(16))) z64 lds[2 * BUF];
   const int N = g.N, n2 = g.n2, ncol = npts * n2;
-  const int ntr = (N + TM - 1) / TM, ntc = (ncol + TN - 1) / TN, per = ntr * ntc, tot = nch * per;
+  const int ntr = (N - r0 + TM - 1) / TM, ntc = (ncol + TN - 1) / TN, per = ntr * ntc, tot = nch * per;
   const int share = (tot + 7) / 8, slot = (int)blockIdx.x >> 3, id = ((int)blockIdx.x & 7) * share + slot;
   if (slot >= share || id >= tot) return;
   const int ch = ch0 + id / per, e0 = id % per, full = ntc / RG_GC * RG_GC;
   const int gw = e0 < full * ntr ? RG_GC : ntc - full;  // columns of this tile's group
   const int gc = e0 < full * ntr ? e0 / (RG_GC * ntr) * RG_GC : full, ge = e0 - gc * ntr;
-  const int rt = ge / gw * TM, ct = (gc + ge % gw) * TN;
+  const int rt = r0 + ge / gw * TM, ct = (gc + ge % gw) * TN;
   const z64* A = ch == 0 ? cd : cm;
   const z64* Z = Zall + (long)ch * N * ncol;
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
@@ -560,22 +560,22 @@ k_resid_gemm(Geom g, int npts, int ch0, int nch, const z64* __restrict__ cd, con
   }
 }
 
-// Out = C_ch^T Z_ch (+ B - Y when B is given, + Out itself when accumulate).  64 x 64 tiles from four rounds
+// Out = C_ch^T Z_ch (+ B - Y when B is given, + Out itself when accumulate), rows r0 .. N - 1.  64 x 64 tiles from four rounds
 // of the chip's 512 such workgroups on; below, 32 x 32 tiles lose less to the last round and to few
 // workgroups (64 x 64 against 32 x 32: N = 1080, 27000 columns 3.21 / 3.50 ms; N = 4000, 2400 columns
 // 4.26 / 4.40; N = 2000, 3200 columns 1.44 / 1.39; N = 540, 738 columns 89 / 50 us; N = 40, 1024 columns 15 / 8).
 void resid_gemm(const Geom& g, int npts, int ch0, int nch, const z64* cd, const z64* cm, const z64* Z, z64* Out,
-                const z64* B, const z64* Y, hipStream_t s, bool accumulate, unsigned long long* rmax) {
+                const z64* B, const z64* Y, hipStream_t s, bool accumulate, unsigned long long* rmax, int r0) {
   auto tiles = [&](int tile) {
-    return nch * ((long)(g.N + tile - 1) / tile) * (((long)npts * g.n2 + tile - 1) / tile);
+    return nch * ((long)(g.N - r0 + tile - 1) / tile) * (((long)npts * g.n2 + tile - 1) / tile);
   };
   auto grid = [](long n) { return dim3((unsigned)((n + 7) / 8 * 8)); };
   if (tiles(64) >= 2048)
     hipLaunchKernelGGL((k_resid_gemm<64, 64>), grid(tiles(64)), dim3(256), 0, s, g, npts, ch0, nch, cd, cm, Z, Out, B,
-                       Y, accumulate ? 1 : 0, rmax);
+                       Y, accumulate ? 1 : 0, rmax, r0);
   else
     hipLaunchKernelGGL((k_resid_gemm<32, 32>), grid(tiles(32)), dim3(256), 0, s, g, npts, ch0, nch, cd, cm, Z, Out, B,
-                       Y, accumulate ? 1 : 0, rmax);
+                       Y, accumulate ? 1 : 0, rmax, r0);
 }
 
 // Per-matrix max |A| (|.| = |re|+|im|, abs_bits), one workgroup per matrix; `clear` (may be null) is zeroed.
@@ -699,10 +699,11 @@ void launch_gamq_z(const Geom& g, int npts, const z64* S, z64* Z, hipStream_t s)
 #undef ADGA_GZ
 }
 
-// gamma^q_d for every point of the batch, into G2 with the residual layout (point b at 2*b).
+// gamma^q_d for every point of the batch, into G2 with the residual layout (point b at 2*b).  The EOM, which
+// alone reads it, sums over nu >= 0 (eom_row0): half the rows, half the product.
 void launch_gamq(const Geom& g, int npts, const z64* S, const z64* cd, z64* Z, z64* G2, hipStream_t s) {
   launch_gamq_z(g, npts, S, Z, s);
-  resid_gemm(g, npts, 0, 1, cd, cd, Z, G2, nullptr, nullptr, s);
+  resid_gemm(g, npts, 0, 1, cd, cd, Z, G2, nullptr, nullptr, s, false, nullptr, eom_row0(g));
 }
 
 // Right-hand side of the eta system: eta A = (1+gamma^w)(1 - A) = (1+gamma^w) blockdiag(S) C, i.e.

@@ -96,16 +96,16 @@ __global__ void __launch_bounds__(256) k_chi_wg(Geom g, const z64* __restrict__ 
 
 // m_tot = -(U + V - U~/2) eta_d /(beta nqp) + 1.5 U~ eta_m /(beta nqp) + U gamma^q_d /(beta nqp)
 //        - V gamma^w_d /(beta nqp)   (eom_module.f90:183-207; the V terms only with V(q): vq non-null).
-// Output (n2, N) Fortran per point.
+// Output (n2, N) Fortran per point, the half nu >= 0 that the EOM sums over.
 __global__ void k_mtot(Geom g, int npts, const z64* __restrict__ u, const z64* __restrict__ ut,
                        const z64* __restrict__ eta, const z64* __restrict__ gamq, z64* __restrict__ mt,
                        const int* __restrict__ qpos, const z64* __restrict__ vq, const z64* __restrict__ gamd,
                        int accumulate) {
   long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  long per = (long)g.n2 * g.N;
-  if (idx >= per * npts) return;
-  int b = (int)(idx / per);
-  long e = idx % per;
+  const long per = (long)g.n2 * g.N, half = per / 2;
+  if (idx >= half * npts) return;
+  int b = (int)(idx / half);
+  long e = half + idx % half;
   int s = (int)(e % g.n2);
   long x = e / g.n2;
   const z64* ed = eta + (long)(2 * b) * per;
@@ -130,7 +130,8 @@ __global__ void k_mtot(Geom g, int npts, const z64* __restrict__ u, const z64* _
   m = cadd(cscale(t2, a2), m);
   m = cadd(cscale(t3, a3), m);
   if (v) m = cadd(cscale(t4, a1), m);
-  mt[idx] = accumulate ? cadd(mt[idx], m) : m;
+  z64* out = mt + b * per + e;
+  *out = accumulate ? cadd(*out, m) : m;
 }
 
 // Sigma_nl(i, l, nu, k) += sum_b sum_{j,k'} m_b(i*n + j, n2*(iwf + nu) + l*n + k') G(k - q_b, nu - omega)_{jk'}
@@ -241,8 +242,9 @@ __global__ void __launch_bounds__(256) k_mtot_t(Geom g, int npts, const z64* __r
                                                 const int* __restrict__ qpos, const z64* __restrict__ vq,
                                                 const z64* __restrict__ gamd, int accumulate) {
   const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (long)npts * g.N) return;
-  const int b = (int)(idx / g.N), x = (int)(idx - (long)b * g.N);
+  const int half = g.N / 2;
+  if (idx >= (long)npts * half) return;
+  const int b = (int)(idx / half), x = half + (int)(idx - (long)b * half);
   const long per = (long)N2 * g.N;
   const z64* ed = eta + (long)(2 * b) * per + (long)x * N2;
   const z64* em = eta + (long)(2 * b + 1) * per + (long)x * N2;
@@ -284,7 +286,7 @@ __global__ void __launch_bounds__(256) k_mtot_t(Geom g, int npts, const z64* __r
 
 void launch_mtot(const Geom& g, int npts, const z64* u, const z64* ut, const z64* eta, const z64* gamq, z64* mt,
                  hipStream_t s, const int* qpos, const z64* vq, const z64* gamd, bool accumulate) {
-  const long tx = (long)npts * g.N;
+  const long tx = (long)npts * (g.N / 2);
 #define ADGA_MT(NN)                                                                                                 \
   if (g.n == NN) {                                                                                                 \
     if (vq)                                                                                                        \
@@ -297,7 +299,7 @@ void launch_mtot(const Geom& g, int npts, const z64* u, const z64* ut, const z64
   }
   ADGA_MT(1) ADGA_MT(2) ADGA_MT(3)
 #undef ADGA_MT
-  long tot = (long)npts * g.n2 * g.N;
+  long tot = (long)npts * g.n2 * (g.N / 2);
   hipLaunchKernelGGL(k_mtot, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s, g, npts, u, ut, eta, gamq, mt,
                      qpos, vq, gamd, accumulate ? 1 : 0);
 }
