@@ -11,6 +11,8 @@
 // happens inside the factorisation.  B and every residual are formed in FP64
 // from the unrounded S and C, so the residual is on the scale of eta itself.
 // M is stored row-major per matrix (row r, column c at r*ldm + c).
+#include <type_traits>
+
 #include "adga_kernels.h"
 #include "mfma_gemm.h"
 
@@ -397,9 +399,12 @@ __device__ __forceinline__ unsigned long long umax64(unsigned long long a, unsig
 //
 // Bound by the FP64 matrix cores: four waves per workgroup, K staged through two LDS buffers in chunks of
 // RG_KC, one barrier per chunk, the next k's fragments loaded ahead of each k's MFMAs, and two (64 x 64 tile,
-// 32 x 32 per wave) to four (32 x 32 tile, 16 x 16 per wave) workgroups per CU, so that one's barriers and
-// staging run under another's MFMAs.  An eight-wave 128 x 64 tile, alone on its CU, took 3.83 ms against 3.21
-// (49 against 59 TFLOP/s issued; an MFMA loop alone reaches 77) at N = 1080, 27000 columns.
+// 32 x 32 per wave) to four (32 x 32 tile, 16 x 16 per wave) workgroups per CU, so that one's barriers run under
+// another's MFMAs.  Two workgroups of a CU tend to run in step, though, and what a wave does between its last MFMA
+// of a chunk and the barrier then stands still: the staging and the next loads are issued between MFMAs instead,
+// from offsets computed once.  N = 1080, 13500 columns: 3.85 -> 3.43 ms, the matrix cores busy for 73 -> 80% of it
+// (6% are the last round of workgroups); N = 4000, 1200 columns 4.36 -> 3.87; N = 2000, 1600 columns (32 x 32)
+// 1.30 -> 1.16.  An eight-wave 128 x 64 tile, alone on its CU, is a fifth slower than four waves.
 // Workgroup b runs on XCD b % 8; each XCD takes a contiguous eighth of the tiles in an order of RG_GC columns
 // by all rows, so that the 64 or 128 resident workgroups of an XCD share their C and Z panels through its L2
 // and no XCD holds more than one tile more than another (whole columns per XCD: N = 4000, 1200 columns 5.25
@@ -427,41 +432,58 @@ k_resid_gemm(Geom g, int npts, int ch0, int nch, const z64* __restrict__ cd, con
   const z64* Z = Zall + (long)ch * N * ncol;
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int wr = (wave / WC) * (TM / WR), wc = (wave % WC) * (TN / WC), li = lane & 15, lg = lane >> 4;
-  const bool inside = rt + TM <= N && ct + TN <= ncol;
   V x[RB][CB], y[RB][CB], z[RB][CB];
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
     for (int cb = 0; cb < CB; ++cb) x[rb][cb] = y[rb][cb] = z[rb][cb] = V{0, 0, 0, 0};
+  // This thread's elements of a chunk: A(row + 16 i, k = kb + t % KC), Z(k = kb + SB i + t / TN, col), as
+  // offsets from a base that all threads share.  Rows and columns beyond the edge are read at the last one:
+  // they only enter outputs that are not stored.
+  static_assert(PA == PB && PA % 2 == 0 && KC == 16, "two halves of a chunk in two of its four k steps");
+  constexpr int SA = 256 / KC, SB = 256 / TN;
+  const z64* At = A + (long)rt * N;
+  const z64* Zt = Z + ct;
+  unsigned oa[PA];  // bytes
+#pragma unroll
+  for (int i = 0; i < PA; ++i)
+    oa[i] = (unsigned)sizeof(z64) * ((unsigned)min(i * SA + t / KC, N - 1 - rt) * (unsigned)N + (unsigned)(t % KC));
+  const unsigned ob =
+      (unsigned)sizeof(z64) * ((unsigned)(t / TN) * (unsigned)ncol + (unsigned)min(t % TN, ncol - 1 - ct));
+  auto ld = [](const z64* base, unsigned off) {
+    return *reinterpret_cast<const z64*>(reinterpret_cast<const char*>(base) + off);
+  };
   z64 pa[PA], pb[PB];
+  auto fetch1 = [&](int kb, int i) {  // elements i of a whole chunk
+    pa[i] = ld(At + kb, oa[i]);
+    pb[i] = ld(Zt + (long)(kb + i * SB) * ncol, ob);
+  };
   auto fetch = [&](int kb) {
-    const bool whole = inside && kb + KC <= N;
+    if (kb + KC <= N) {
+#pragma unroll
+      for (int i = 0; i < PA; ++i) fetch1(kb, i);
+      return;
+    }
 #pragma unroll
     for (int i = 0; i < PA; ++i) {
-      const int e = t + i * 256, row = rt + e / KC, k = kb + e % KC;
-      pa[i] = whole || (row < N && k < N) ? A[(long)row * N + k] : mk(0.0, 0.0);
-    }
-#pragma unroll
-    for (int i = 0; i < PB; ++i) {
-      const int e = t + i * 256, k = kb + e / TN, col = ct + e % TN;
-      pb[i] = whole || (k < N && col < ncol) ? Z[(long)k * ncol + col] : mk(0.0, 0.0);
+      pa[i] = kb + t % KC < N ? ld(At + kb, oa[i]) : mk(0.0, 0.0);
+      pb[i] = kb + i * SB + t / TN < N ? ld(Zt + (long)(kb + i * SB) * ncol, ob) : mk(0.0, 0.0);
     }
   };
-  auto stage = [&](int b) {
+  auto stage1 = [&](int b, int i) {
     z64* As = lds + b * BUF;
     z64* Bs = As + TM * LDA;
-#pragma unroll
-    for (int i = 0; i < PA; ++i) {
-      const int e = t + i * 256;
-      As[(e / KC) * LDA + e % KC] = pa[i];
-    }
-#pragma unroll
-    for (int i = 0; i < PB; ++i) {
-      const int e = t + i * 256;
-      Bs[(e / TN) * LDB + e % TN] = pb[i];
-    }
+    As[(t / KC + i * SA) * LDA + t % KC] = pa[i];
+    Bs[(t / TN + i * SB) * LDB + t % TN] = pb[i];
   };
-  auto compute = [&](int b, int kend) {  // k in [kend, KC) of a last, partial chunk are staged zeros
+  auto stage = [&](int b) {
+#pragma unroll
+    for (int i = 0; i < PA; ++i) stage1(b, i);
+  };
+  // the chunk in buffer b; k in [kend, KC) of a last, partial chunk are staged zeros.  With `next` >= 0 the
+  // second and third of its four k steps each also write half of the staged chunk to the other buffer and
+  // start the loads of the chunk at `next`, between MFMAs.
+  auto compute = [&](int b, int kend, auto feed, int next) {
     const z64* Ap = lds + b * BUF + (wr + li) * LDA + lg;
     const z64* Bp = lds + b * BUF + TM * LDA + lg * LDB + wc + li;
     z64 a[2][RB], v[2][CB];
@@ -491,17 +513,36 @@ k_resid_gemm(Geom g, int npts, int ch0, int nch, const z64* __restrict__ cd, con
           x[rb][cb] = Mfma<double>::op(a[p][rb].re, v[p][cb].re, x[rb][cb]);
           y[rb][cb] = Mfma<double>::op(a[p][rb].im, v[p][cb].im, y[rb][cb]);
           z[rb][cb] = Mfma<double>::op(as[rb], vs[cb], z[rb][cb]);
+          if constexpr (decltype(feed)::value) {
+            constexpr int HALF = PA / 2, PER = RB * CB;
+            const int j = rb * CB + cb;
+            if (kk == 4 || kk == 8)
+#pragma unroll
+              for (int i = 0; i < HALF; ++i)
+                if (i * PER / HALF == j) {
+                  stage1(b ^ 1, (kk / 4 - 1) * HALF + i);
+                  fetch1(next, (kk / 4 - 1) * HALF + i);
+                }
+          }
         }
+      if constexpr (decltype(feed)::value) __builtin_amdgcn_sched_barrier(0);
     }
   };
+  using Feed = std::integral_constant<bool, true>;
+  using Plain = std::integral_constant<bool, false>;
   fetch(0);
   stage(0);
   if (KC < N) fetch(KC);
   __syncthreads();
   int b = 0, kb = 0;
+  for (; kb + 3 * KC <= N; kb += KC) {  // a buffer is written after the barrier that ended its reading
+    compute(b, KC, Feed{}, kb + 2 * KC);
+    __syncthreads();
+    b ^= 1;
+  }
   for (; kb + KC < N; kb += KC) {
-    compute(b, KC);
-    stage(b ^ 1);  // last read in the previous chunk, before the barrier that ended it
+    compute(b, KC, Plain{}, 0);
+    stage(b ^ 1);
     if (kb + 2 * KC < N) fetch(kb + 2 * KC);
     __syncthreads();
     b ^= 1;
@@ -529,7 +570,7 @@ k_resid_gemm(Geom g, int npts, int ch0, int nch, const z64* __restrict__ cd, con
           cin[rb][cb][v] = c;
         }
   }
-  compute(b, N - kb);
+  compute(b, N - kb, Plain{}, 0);
   unsigned long long mx[CB] = {};
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb)
