@@ -24,10 +24,11 @@ void launch_bubble(const Geom& g, int iwb, int npts, const int* qidx, const z64*
                    const z64* gt2 = nullptr, bool accumulate = false);
 // Out = C_ch^T Z_ch for the channels ch0 .. ch0 + nch - 1 (C row-major as the left operand, Z and Out in the
 // residual layouts), plus B - Y when B is given, plus Out itself when accumulate; with rmax each matrix's
-// max |Out| as the bits of a double (atomic maximum: cleared by the caller); rows r0 .. N - 1 of each matrix
+// max |result| as the bits of a double (atomic maximum: cleared by the caller); rows r0 .. N - 1 of each matrix;
+// with update Y plus the result is stored (Out may be Y)
 void resid_gemm(const Geom& g, int npts, int ch0, int nch, const z64* cd, const z64* cm, const z64* Z, z64* Out,
                 const z64* B, const z64* Y, hipStream_t s, bool accumulate = false,
-                unsigned long long* rmax = nullptr, int r0 = 0);
+                unsigned long long* rmax = nullptr, int r0 = 0, bool update = false);
 // the first row of a point's matrices that the EOM reads: nu >= 0 (eom_module.f90:211-227), the upper half
 inline int eom_row0(const Geom& g) { return g.n2 * g.iwf; }
 void launch_smat(const Geom& g, int npts, const z64* chi0q, const z64* winv, z64* S, hipStream_t s);
@@ -110,6 +111,8 @@ struct ResidNorm {
 void launch_absmax_rhs(const Geom& g, int npts, const z64* B, const ResidNorm& nrm, hipStream_t s);
 void launch_add(long n, const z64* R, z64* Y, hipStream_t s);  // Y += R
 enum ResidMode { RESID_OF = 0, RESID_STEP = 1, RESID_START = 2 };
+// whether after a step R is still to be added to Y
+bool resid_step_pending(const VqTerm* vq);
 void launch_residual(const Geom& g, int npts, const z64* S, const z64* cd, const z64* cm, const z64* B, z64* Y,
                      z64* Z, z64* R, const ResidNorm& nrm, hipStream_t s, const VqTerm* vq = nullptr,
                      ResidMode mode = RESID_OF, LuTimer* timer = nullptr);

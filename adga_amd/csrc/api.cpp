@@ -450,7 +450,7 @@ bool series_solve(adga_ctx* c, int nb, double tol, double accept, const z64* B, 
     if (!(relh[2 * b] <= accept && relh[2 * b + 1] <= accept)) left.push_back(b);
   if (8 * left.size() > (size_t)nb) return false;
   // the last residual is at hand: one more step, whose residual is below the one tested by the contraction
-  adga::launch_add(2L * nb * g.N * g.n2, c->R, Y, s);
+  if (adga::resid_step_pending(vtp)) adga::launch_add(2L * nb * g.N * g.n2, c->R, Y, s);
   return true;
 }
 

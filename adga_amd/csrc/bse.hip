@@ -394,8 +394,9 @@ __device__ __forceinline__ unsigned long long umax64(unsigned long long a, unsig
 // Out[(2b + ch) N + r][s] = sum_x C_ch(x, r) Z_ch[x][b*n2 + s], plus (B - Y) at the same position
 // when B is given (the residual), for the rows r >= r0: complex FP64 products by the 3M method (X = Ar Br, Y = Ai Bi,
 // Z = (Ar + Ai)(Br + Bi), as gemm3m_tile), C read row-major as A(r, x) = C[r N + x], the output in the
-// point-major layout of Y.  With rmax, each matrix's max |Out| goes there from the output registers
-// (abs_bits, combined per column in LDS), instead of a second pass over Out.
+// point-major layout of Y.  With `update` what is stored is Y plus that result (Out may be Y).  With rmax, each
+// matrix's max |result| goes there from the output registers (abs_bits, combined per column in LDS), instead of
+// a second pass over it.
 //
 // Bound by the FP64 matrix cores: four waves per workgroup, K staged through two LDS buffers in chunks of
 // RG_KC, one barrier per chunk, the next k's fragments loaded ahead of each k's MFMAs, and two (64 x 64 tile,
@@ -413,8 +414,8 @@ constexpr int RG_KC = 16, RG_GC = 8;
 template <int TM, int TN>
 __global__ void __launch_bounds__(256, TM == 64 ? 2 : 4)
 k_resid_gemm(Geom g, int npts, int ch0, int nch, const z64* __restrict__ cd, const z64* __restrict__ cm,
-             const z64* __restrict__ Zall, z64* Out, const z64* __restrict__ B, const z64* __restrict__ Y,
-             int accumulate, unsigned long long* __restrict__ rmax, int r0) {
+             const z64* __restrict__ Zall, z64* Out, const z64* __restrict__ B, const z64* Y, int accumulate,
+             int update, unsigned long long* __restrict__ rmax, int r0) {
   using V = f64x4;
   constexpr int KC = RG_KC, WR = 2, WC = 2, RB = TM / WR / 16, CB = TN / WC / 16;
   constexpr int LDA = KC + 1, LDB = TN + 8, BUF = TM * LDA + KC * LDB;  // strides without bank conflicts
@@ -573,7 +574,17 @@ k_resid_gemm(Geom g, int npts, int ch0, int nch, const z64* __restrict__ cd, con
   compute(b, N - kb, Plain{}, 0);
   unsigned long long mx[CB] = {};
 #pragma unroll
-  for (int rb = 0; rb < RB; ++rb)
+  for (int rb = 0; rb < RB; ++rb) {
+    z64 yv[CB][4];  // Y again, all of a block row's loads before its stores (Out may be Y itself)
+    if (update) {
+#pragma unroll
+      for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int row = rt + wr + rb * 16 + Mfma<double>::row(lg, v), col = ct + wc + cb * 16 + li;
+          yv[cb][v] = row < N && col < ncol ? Y[at(row, col)] : mk(0.0, 0.0);
+        }
+    }
 #pragma unroll
     for (int cb = 0; cb < CB; ++cb)
 #pragma unroll
@@ -582,10 +593,11 @@ k_resid_gemm(Geom g, int npts, int ch0, int nch, const z64* __restrict__ cd, con
         if (row < N && col < ncol) {
           z64 o = mk(x[rb][cb][v] - y[rb][cb][v], (z[rb][cb][v] - x[rb][cb][v]) - y[rb][cb][v]);
           if (add) o = cadd(cin[rb][cb][v], o);
-          Out[at(row, col)] = o;
           mx[cb] = umax64(mx[cb], abs_bits(o));
+          Out[at(row, col)] = update ? cadd(yv[cb][v], o) : o;
         }
       }
+  }
   if (rmax) {
     __syncthreads();  // the tile's LDS reads are done
     unsigned long long* sm = reinterpret_cast<unsigned long long*>(lds);
@@ -606,17 +618,18 @@ k_resid_gemm(Geom g, int npts, int ch0, int nch, const z64* __restrict__ cd, con
 // workgroups (64 x 64 against 32 x 32: N = 1080, 27000 columns 3.21 / 3.50 ms; N = 4000, 2400 columns
 // 4.26 / 4.40; N = 2000, 3200 columns 1.44 / 1.39; N = 540, 738 columns 89 / 50 us; N = 40, 1024 columns 15 / 8).
 void resid_gemm(const Geom& g, int npts, int ch0, int nch, const z64* cd, const z64* cm, const z64* Z, z64* Out,
-                const z64* B, const z64* Y, hipStream_t s, bool accumulate, unsigned long long* rmax, int r0) {
+                const z64* B, const z64* Y, hipStream_t s, bool accumulate, unsigned long long* rmax, int r0,
+                bool update) {
   auto tiles = [&](int tile) {
     return nch * ((long)(g.N - r0 + tile - 1) / tile) * (((long)npts * g.n2 + tile - 1) / tile);
   };
   auto grid = [](long n) { return dim3((unsigned)((n + 7) / 8 * 8)); };
   if (tiles(64) >= 2048)
     hipLaunchKernelGGL((k_resid_gemm<64, 64>), grid(tiles(64)), dim3(256), 0, s, g, npts, ch0, nch, cd, cm, Z, Out, B,
-                       Y, accumulate ? 1 : 0, rmax, r0);
+                       Y, accumulate ? 1 : 0, update ? 1 : 0, rmax, r0);
   else
     hipLaunchKernelGGL((k_resid_gemm<32, 32>), grid(tiles(32)), dim3(256), 0, s, g, npts, ch0, nch, cd, cm, Z, Out, B,
-                       Y, accumulate ? 1 : 0, rmax, r0);
+                       Y, accumulate ? 1 : 0, update ? 1 : 0, rmax, r0);
 }
 
 // Per-matrix max |A| (|.| = |re|+|im|, abs_bits), one workgroup per matrix; `clear` (may be null) is zeroed.
@@ -652,7 +665,7 @@ __global__ void k_resid_rel(int nmat, const unsigned long long* __restrict__ bma
 // x = d*n2 + i' of its column: each thread reads its values of V once, and for each i' the wave writes a
 // contiguous run of Z's row x (consecutive lanes hold consecutive columns b*n2 + s).  V by `mode`: Z_OPG
 // (1 + gamma^w)^T, Z_Y the solution, Z_ADD Y + R with the sum stored to Y (a step of the fixed-point
-// iteration: every element of Y belongs to one thread), Z_RHS B, stored to Y (its start).
+// iteration: every element of Y belongs to one thread), Z_RHS B (its start; stored to Y unless that is null).
 enum { Z_OPG = 0, Z_Y = 1, Z_ADD = 2, Z_RHS = 3 };
 template <int N2>
 __global__ void __launch_bounds__(256) k_resid_zt(Geom g, int npts, int mode, const z64* __restrict__ S,
@@ -680,7 +693,7 @@ __global__ void __launch_bounds__(256) k_resid_zt(Geom g, int npts, int mode, co
 #pragma unroll
       for (int cp = 0; cp < N2; ++cp) v[cp] = cadd(v[cp], R[o + cp * N2]);
     }
-    if (mode != Z_Y) {
+    if (mode == Z_ADD || (mode == Z_RHS && Y)) {
 #pragma unroll
       for (int cp = 0; cp < N2; ++cp) Y[o + cp * N2] = v[cp];
     }
@@ -771,20 +784,31 @@ void launch_add(long n, const z64* R, z64* Y, hipStream_t s) {
 }
 
 // R = B - M Y with M Y = Y - C^T (blockdiag(S)^T Y), in FP64 from the unrounded factors S and C (with V(q):
-// minus (1 + gamma^w_d)^T (W^T Y) in the density channel).  Y: as given, or first Y += R (RESID_STEP) or
-// Y = B (RESID_START), folded into the kernel that reads it.  M = 1 - T with T Y = C^T (blockdiag(S)^T Y), so
-// the steps Y += R from Y = B sum the series (1 + T + T^2 + ...) B.
+// minus (1 + gamma^w_d)^T (W^T Y) in the density channel), and its norms.  M = 1 - T with
+// T Y = C^T (blockdiag(S)^T Y), so steps Y += R from Y = B sum the series (1 + T + T^2 + ...) B.
+//   RESID_OF     of Y as given, stored to R
+//   RESID_START  of Y = B, RESID_STEP of the last call's Y + R, for the fixed-point iteration: without V(q) the
+//                product stores Y + R over Y at once and R nowhere, five passes over a solution's array a step
+//                (B, Y, Y + R, and Y, Z of the next operand) where R stored, added as the next operand is
+//                formed and by a kernel of its own at the end took eight and three more; with V(q), whose term
+//                is added to R by kernels after the product, the next call adds R (resid_step_pending).
+bool resid_step_pending(const VqTerm* vq) { return vq != nullptr; }
+
 void launch_residual(const Geom& g, int npts, const z64* S, const z64* cd, const z64* cm, const z64* B, z64* Y,
                      z64* Z, z64* R, const ResidNorm& nrm, hipStream_t s, const VqTerm* vq, ResidMode mode,
                      LuTimer* timer) {
   const int nmat = 2 * npts;
-  const int zm = mode == RESID_START ? Z_RHS : mode == RESID_STEP ? Z_ADD : Z_Y;
-  resid_z(g, npts, zm, S, Y, mode == RESID_START ? B : R, nullptr, nullptr, Z, s);
+  const bool start = mode == RESID_START, update = mode != RESID_OF && !resid_step_pending(vq);
+  if (start)
+    resid_z(g, npts, Z_RHS, S, update ? nullptr : Y, B, nullptr, nullptr, Z, s);
+  else
+    resid_z(g, npts, mode == RESID_STEP && !update ? Z_ADD : Z_Y, S, Y, R, nullptr, nullptr, Z, s);
   if (timer) {
     timer->mark(s);
     timer->flops += 8.0 * g.N * (double)g.N * g.n2 * nmat;
   }
-  resid_gemm(g, npts, 0, 2, cd, cm, Z, R, B, Y, s, false, vq ? nullptr : nrm.rmax);
+  resid_gemm(g, npts, 0, 2, cd, cm, Z, update ? Y : R, B, update && start ? B : Y, s, false, vq ? nullptr : nrm.rmax,
+             0, update);
   if (timer) timer->mark(s);
   if (vq) {
     launch_vq_add(g, npts, *vq, Y, R, s);
