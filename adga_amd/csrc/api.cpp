@@ -872,7 +872,8 @@ int run_points_impl(adga_ctx* c, int npts, const int* iq, int precision, double*
         }
       }
       CK(hipEventRecord(ev[4], s));
-      adga::launch_chi(g, nb, c->Y, c->chi0q, c->chi0w, c->gamd, c->gamm, c->bubloc, c->chi_out, c->bub_out, s);
+      adga::launch_chi(g, nb, c->Y, c->chi0q, c->chi0w, c->gamd, c->gamm, c->bubloc, c->R, c->chi_out,
+                       c->bub_out, s);
       if (c->bubble_range >= 1) {
         // the large range's frequencies outside the box enter bubble_nl (main.F90:644-663, debug option
         // "Bubble"): all q of the omega as one convolution, kept for the omega's next batches

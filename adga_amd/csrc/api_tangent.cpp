@@ -106,7 +106,7 @@ void tangent_batch(adga_ctx* c, int nb, int p0, int npts, const std::vector<int>
                                        c->t_dY, false, s))
       throw HipError{hipErrorInvalidValue, "tangent solve: BSE size outside the solve kernel's range"};
     adga::launch_dchi(g, nb, c->chi0q, c->t_dchi0q, c->chi0w, dw, c->gamd, c->gamm, dgamd, dgamm, c->Y, c->t_dY,
-                      c->t_dchi + (size_t)dir * 2 * nb * g.n4, c->t_dbub + (size_t)dir * nb * g.n4, s);
+                      c->t_Z1, c->t_dchi + (size_t)dir * 2 * nb * g.n4, c->t_dbub + (size_t)dir * nb * g.n4, s);
     if (!c->do_eom) continue;
     // d m_tot = m_tot(U, U~; d eta, d gamma^q) + m_tot(dU, dU~; eta, gamma^q), with
     // d gamma^q_d = sum_nu (dS C_d + S dC_d)[nu rows]

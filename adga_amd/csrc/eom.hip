@@ -1,5 +1,8 @@
 // A8 (eta), A9 (chi contraction), A10 (dynamic EOM), A11 (local/static EOM) on gfx950.
+#include <algorithm>
+
 #include "adga_kernels.h"
+#include "mfma_gemm.h"
 
 namespace adga {
 
@@ -10,40 +13,159 @@ namespace adga {
 // chi_ch(q) (non-local part) = beta^-2 gamma^w_ch . (chi0^q - chi0^w) + beta^-2 eta_ch . chi0^q, where
 // (X . Y)(s, s2) = sum_{d, i3} X(s, d*n2 + i3) Y(i3, s2, d)  (susc_module.f90:34-56, main.F90:666-769);
 // bubble_nl(q) = sum_d chi0^q / beta^2 - sum_d chi0^w / beta^2  (main.F90:654-663).
-__global__ void k_chi(Geom g, int npts, const z64* __restrict__ chi0q, const z64* __restrict__ chi0w,
-                      const z64* __restrict__ gam_d, const z64* __restrict__ gam_m, const z64* __restrict__ eta,
-                      const z64* __restrict__ bubloc, z64* __restrict__ chi_out, z64* __restrict__ bub_out) {
-  long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (long)npts * 2 * g.n4) return;
-  int e = (int)(idx % g.n4);
-  int ch = (int)((idx / g.n4) % 2);
-  int b = (int)(idx / (2 * g.n4));
-  int s = e % g.n2, s2 = e / g.n2;
-  const z64* gam = ch == 0 ? gam_d : gam_m;
-  const z64* et = eta + (long)(2 * b + ch) * g.n2 * g.N;
-  const z64* cq = chi0q + (long)b * g.nf * g.n4;
-  z64 a1 = mk(0.0, 0.0), a2 = mk(0.0, 0.0), bs = mk(0.0, 0.0);
-  for (int d = 0; d < g.nf; ++d) {
-    for (int i3 = 0; i3 < g.n2; ++i3) {
-      long x = (long)d * g.n2 + i3;
-      z64 c = cq[(long)d * g.n4 + i3 + s2 * g.n2];
-      z64 cnl = c;
-      if (i3 == s2) cnl = csub(c, chi0w[s2 + d * g.n2]);
-      a1 = cfma(gam[s + x * g.n2], cnl, a1);
-      a2 = cfma(et[s + x * g.n2], c, a2);
+//
+// A form g . (c - w) + e . c is that with c = chi0^q of each point, w = chi0^w, g per channel and e per channel
+// and point; the derivative of chi is the sum of two (product rule): (dg, de, c, w) and (g, e, dc, dw).
+//
+// One workgroup per point and slice of frequencies, for n >= 3: both factors of each product are loaded as they
+// lie, every element into one lane of a matrix fragment, where threads that each form outputs load them n2 times
+// over and are bound by the L1 cache (a thread per row and slice: three orbitals, 120 frequencies, 1500 points
+// 0.69 ms, 0.33 here; a thread per output: five orbitals, 160 frequencies, 48 points 2.15 ms, 0.15 here; the
+// derivative with three, 80 frequencies, 500 points 0.70 ms, 0.16 here).  Now bound by the loads of c and e
+// (0.70 GB in the first, 2.1 TB/s).  Four waves take every fourth step of four x = d n2 + i3, are added in
+// LDS in a fixed order, and the slices' sums by k_chi_sum.
+struct ChiForm {
+  const z64 *c, *w, *gd, *gm, *e;
+};
+template <int NT>
+struct ChiForms {
+  ChiForm f[NT];
+};
+template <int N2, int NT>
+__global__ void __launch_bounds__(256) k_chi_mm(Geom g, int slices, ChiForms<NT> fs, z64* __restrict__ part) {
+  constexpr int N4 = N2 * N2, T = (N2 + 15) / 16;
+  __shared__ z64 sum[4][2 * N4];
+  const int b = blockIdx.x, sl = blockIdx.y, t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int li = lane & 15, lg = lane >> 4;
+  const int d0 = (int)((long)g.nf * sl / slices), d1 = (int)((long)g.nf * (sl + 1) / slices);
+  const int x0 = d0 * N2, x1 = d1 * N2;
+  f64x4 re[2][T][T], im[2][T][T];
+#pragma unroll
+  for (int ch = 0; ch < 2; ++ch)
+#pragma unroll
+    for (int r = 0; r < T; ++r)
+#pragma unroll
+      for (int q = 0; q < T; ++q) re[ch][r][q] = im[ch][r][q] = f64x4{0, 0, 0, 0};
+#pragma unroll
+  for (int k = 0; k < NT; ++k) {
+    const ChiForm f = fs.f[k];
+    const z64* cq = f.c + (long)b * g.nf * N4;
+    const z64* eb = f.e + (long)(2 * b) * g.N * N2;
+    for (int xs = x0 + 4 * wave; xs < x1; xs += 16) {
+      const int x = xs + lg, d = x / N2, i3 = x - d * N2;
+      const bool in = x < x1;
+      z64 c[T], n[T], a[2][2][T];  // c, c - w; g and e of the two channels
+#pragma unroll
+      for (int q = 0; q < T; ++q) {
+        const int s2 = q * 16 + li;
+        const bool ok = in && s2 < N2;
+        c[q] = ok ? cq[(long)d * N4 + i3 + s2 * N2] : mk(0.0, 0.0);
+        n[q] = ok && s2 == i3 ? csub(c[q], f.w[x]) : c[q];
+      }
+#pragma unroll
+      for (int r = 0; r < T; ++r) {
+        const int s = r * 16 + li;
+        const bool ok = in && s < N2;
+        const long o = (long)x * N2 + s;
+        a[0][0][r] = ok ? f.gd[o] : mk(0.0, 0.0);
+        a[0][1][r] = ok ? eb[o] : mk(0.0, 0.0);
+        a[1][0][r] = ok ? f.gm[o] : mk(0.0, 0.0);
+        a[1][1][r] = ok ? eb[(long)g.N * N2 + o] : mk(0.0, 0.0);
+      }
+#pragma unroll
+      for (int ch = 0; ch < 2; ++ch)
+#pragma unroll
+        for (int p = 0; p < 2; ++p)
+#pragma unroll
+          for (int r = 0; r < T; ++r)
+#pragma unroll
+            for (int q = 0; q < T; ++q) {
+              const z64 u = a[ch][p][r], v = p == 0 ? n[q] : c[q];
+              re[ch][r][q] = Mfma<double>::op(u.re, v.re, re[ch][r][q]);
+              im[ch][r][q] = Mfma<double>::op(u.re, v.im, im[ch][r][q]);
+              re[ch][r][q] = Mfma<double>::op(-u.im, v.im, re[ch][r][q]);
+              im[ch][r][q] = Mfma<double>::op(u.im, v.re, im[ch][r][q]);
+            }
     }
-    if (ch == 0) bs = cadd(bs, cq[(long)d * g.n4 + s + s2 * g.n2]);
   }
-  double ib2 = 1.0 / (g.beta * g.beta);
-  z64 v = cadd(cscale(a1, ib2), cscale(a2, ib2));
-  chi_out[((long)b * 2 + ch) * g.n4 + e] = v;
-  if (ch == 0) bub_out[(long)b * g.n4 + e] = csub(cscale(bs, ib2), bubloc[e]);
+#pragma unroll
+  for (int ch = 0; ch < 2; ++ch)
+#pragma unroll
+    for (int r = 0; r < T; ++r)
+#pragma unroll
+      for (int q = 0; q < T; ++q)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int s = r * 16 + Mfma<double>::row(lg, v), s2 = q * 16 + li;
+          if (s < N2 && s2 < N2) sum[wave][ch * N4 + s + s2 * N2] = mk(re[ch][r][q][v], im[ch][r][q][v]);
+        }
+  __syncthreads();
+  z64* out = part + ((long)b * slices + sl) * (3 * N4);
+  for (int e = t; e < 2 * N4; e += 256)
+    out[e] = cadd(cadd(sum[0][e], sum[1][e]), cadd(sum[2][e], sum[3][e]));
+  const ChiForm f = fs.f[NT - 1];  // its c summed over the frequencies; of a derivative, minus its w
+  const z64* cq = f.c + (long)b * g.nf * N4;
+  for (int e = t; e < N4; e += 256) {
+    z64 bs = mk(0.0, 0.0);
+#pragma unroll 4
+    for (int d = d0; d < d1; ++d) {
+      z64 v = cq[(long)d * N4 + e];
+      if (NT == 2 && e / N2 == e % N2) v = csub(v, f.w[d * N2 + e % N2]);
+      bs = cadd(bs, v);
+    }
+    out[2 * N4 + e] = bs;
+  }
 }
 
-// The same for n <= 3 with one workgroup per point: thread (k slice, channel, row s) accumulates row s of
+// The slices' sums in order, over beta^2: chi_out (channel, n4) per point, and bub_out, less bubloc if given.
+__global__ void __launch_bounds__(256) k_chi_sum(Geom g, int npts, int slices, const z64* __restrict__ part,
+                                                 const z64* __restrict__ bubloc, z64* __restrict__ chi_out,
+                                                 z64* __restrict__ bub_out) {
+  const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  const int per = 3 * g.n4;
+  if (idx >= (long)npts * per) return;
+  const int b = (int)(idx / per), e = (int)(idx - (long)b * per);
+  const z64* p = part + (long)b * slices * per + e;
+  z64 v = p[0];
+  for (int k = 1; k < slices; ++k) v = cadd(v, p[(long)k * per]);
+  v = cscale(v, 1.0 / (g.beta * g.beta));
+  if (e < 2 * g.n4) {
+    chi_out[(long)b * 2 * g.n4 + e] = v;
+  } else {
+    const int f = e - 2 * g.n4;
+    bub_out[(long)b * g.n4 + f] = bubloc ? csub(v, bubloc[f]) : v;
+  }
+}
+
+// Slices until 2048 workgroups are in flight, of eight frequencies or more; `part` (3 n4 values per point and
+// slice) fits a solution's array of 2 n4 per point and frequency.
+template <int NT>
+static bool chi_mm(const Geom& g, int npts, const ChiForms<NT>& fs, z64* part, const z64* bubloc, z64* chi_out,
+                   z64* bub_out, hipStream_t s) {
+  const int slices = std::max(1, std::min((2047 + npts) / npts, g.nf / 8));
+  const dim3 grid((unsigned)npts, (unsigned)slices);
+  switch (g.n) {
+    case 3: hipLaunchKernelGGL((k_chi_mm<9, NT>), grid, dim3(256), 0, s, g, slices, fs, part); break;
+    case 4: hipLaunchKernelGGL((k_chi_mm<16, NT>), grid, dim3(256), 0, s, g, slices, fs, part); break;
+    case 5: hipLaunchKernelGGL((k_chi_mm<25, NT>), grid, dim3(256), 0, s, g, slices, fs, part); break;
+    default: return false;
+  }
+  const long tot = (long)npts * 3 * g.n4;
+  hipLaunchKernelGGL(k_chi_sum, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s, g, npts, slices, part, bubloc,
+                     chi_out, bub_out);
+  return true;
+}
+
+bool launch_dchi_mm(const Geom& g, int npts, const z64* chi0q, const z64* dchi0q, const z64* chi0w, const z64* dchi0w,
+                    const z64* gamd, const z64* gamm, const z64* dgamd, const z64* dgamm, const z64* Y, const z64* dY,
+                    z64* part, z64* dchi_out, z64* dbub_out, hipStream_t s) {
+  return chi_mm<2>(g, npts, {{{chi0q, chi0w, dgamd, dgamm, dY}, {dchi0q, dchi0w, gamd, gamm, Y}}}, part, nullptr,
+                   dchi_out, dbub_out, s);
+}
+
+// The same for n <= 2, whose n2 values fill little of a matrix fragment, with one workgroup per point: thread (k slice, channel, row s) accumulates row s of
 // chi_ch over its slice of x = d*n2 + i3 (the n2 values of chi0^q at one x are read by every thread of the
-// slice), the slices are summed through LDS, and threads 0 .. n4-1 form bubble_nl (summed over d in the
-// same order as k_chi).  The chi sums run in another order than k_chi's: roundoff-level differences.
+// slice), the slices are summed through LDS, and threads 0 .. n4-1 form bubble_nl (summed over d in order).
 template <int N2>
 __global__ void __launch_bounds__(256) k_chi_wg(Geom g, const z64* __restrict__ chi0q, const z64* __restrict__ chi0w,
                                                 const z64* __restrict__ gam_d, const z64* __restrict__ gam_m,
@@ -216,20 +338,16 @@ __global__ void k_eom_static(Geom g, const z64* __restrict__ u, const z64* __res
 }
 
 void launch_chi(const Geom& g, int npts, const z64* eta, const z64* chi0q, const z64* chi0w, const z64* gamd,
-                const z64* gamm, const z64* bubloc, z64* chi_out, z64* bub_out, hipStream_t s) {
-  if (g.n <= 3) {
+                const z64* gamm, const z64* bubloc, z64* part, z64* chi_out, z64* bub_out, hipStream_t s) {
 #define ADGA_CHI_WG(NN)                                                                                          \
   if (g.n == NN) {                                                                                              \
     hipLaunchKernelGGL(k_chi_wg<NN * NN>, dim3((unsigned)npts), dim3(256), 0, s, g, chi0q, chi0w, gamd, gamm, eta, \
                        bubloc, chi_out, bub_out);                                                               \
     return;                                                                                                     \
   }
-    ADGA_CHI_WG(1) ADGA_CHI_WG(2) ADGA_CHI_WG(3)
+  ADGA_CHI_WG(1) ADGA_CHI_WG(2)
 #undef ADGA_CHI_WG
-  }
-  long t2 = (long)npts * 2 * g.n4;
-  hipLaunchKernelGGL(k_chi, dim3((unsigned)((t2 + 127) / 128)), dim3(128), 0, s, g, npts, chi0q, chi0w, gamd, gamm,
-                     eta, bubloc, chi_out, bub_out);
+  chi_mm<1>(g, npts, {{{chi0q, chi0w, gamd, gamm, eta}}}, part, bubloc, chi_out, bub_out, s);
 }
 
 // k_mtot for n <= 3 with one thread per (point b, x) forming the n2 values s of its row: eta_d, eta_m and

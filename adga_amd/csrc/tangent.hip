@@ -223,6 +223,7 @@ void launch_tangent_rhs(const Geom& g, int npts, const z64* S, const z64* dS, co
 // Derivative of chi_ch(q) (non-local part) and of the non-local bubble:
 //   beta^-2 [dgamma . (chi0q - chi0w) + gamma . (dchi0q - dchi0w) + deta . chi0q + eta . dchi0q],
 //   beta^-2 (sum_nu dchi0q - sum_nu dchi0w)   (eta from Y^T, deta from dY^T).
+// One thread per output, for n <= 2.
 __global__ void k_dchi(Geom g, int npts, const z64* __restrict__ chi0q, const z64* __restrict__ dchi0q,
                        const z64* __restrict__ chi0w, const z64* __restrict__ dchi0w, const z64* __restrict__ gam_d,
                        const z64* __restrict__ gam_m, const z64* __restrict__ dgam_d, const z64* __restrict__ dgam_m,
@@ -269,7 +270,10 @@ __global__ void k_dchi(Geom g, int npts, const z64* __restrict__ chi0q, const z6
 
 void launch_dchi(const Geom& g, int npts, const z64* chi0q, const z64* dchi0q, const z64* chi0w, const z64* dchi0w,
                  const z64* gamd, const z64* gamm, const z64* dgamd, const z64* dgamm, const z64* Y, const z64* dY,
-                 z64* dchi_out, z64* dbub_out, hipStream_t s) {
+                 z64* part, z64* dchi_out, z64* dbub_out, hipStream_t s) {
+  if (launch_dchi_mm(g, npts, chi0q, dchi0q, chi0w, dchi0w, gamd, gamm, dgamd, dgamm, Y, dY, part, dchi_out, dbub_out,
+                     s))
+    return;
   const long tot = (long)npts * 2 * g.n4;
   hipLaunchKernelGGL(k_dchi, dim3((unsigned)((tot + 127) / 128)), dim3(128), 0, s, g, npts, chi0q, dchi0q, chi0w,
                      dchi0w, gamd, gamm, dgamd, dgamm, Y, dY, dchi_out, dbub_out);
