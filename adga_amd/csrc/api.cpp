@@ -102,13 +102,16 @@ void ensure_conv(adga_ctx* c) {
   dalloc(&c->tw, tw.size());
   CK(hipMemcpy(c->tw, tw.data(), sizeof(z64) * tw.size(), hipMemcpyHostToDevice));
   size_t ng = (size_t)g.nw * g.n2 * g.nkp;
-  z64* tmp = nullptr;
-  dalloc(&tmp, ng);
   dalloc(&c->ghat, ng);
-  adga::launch_ghat(g, c->tw, c->gt, tmp, c->ghat, c->stream);
+  if (adga::dft_in_lds(g)) {
+    adga::launch_ghat(g, c->tw, c->gt, nullptr, c->ghat, c->stream);
+    CK(hipGetLastError());
+    return;
+  }
+  DevBuf<> tmp(ng);
+  adga::launch_ghat(g, c->tw, c->gt, tmp.p, c->ghat, c->stream);
   CK(hipGetLastError());
   CK(hipStreamSynchronize(c->stream));
-  dfree(tmp);
 }
 
 void eom_flush(adga_ctx* c);

@@ -194,7 +194,7 @@ int adga_set_tangents(adga_ctx* c, int ndir, const double* dhk, const double* ds
       conv_tables(c);
       const size_t ngt = (size_t)g.nw * g.n2 * g.nkp;
       dalloc(&c->t_dghat, ngt * ndir);
-      DevBuf<> tmp(ngt);
+      DevBuf<> tmp(adga::dft_in_lds(g) ? 0 : ngt);
       for (int d = 0; d < ndir; ++d) adga::launch_ghat(g, c->tw, c->dgt + d * ngt, tmp.p, c->t_dghat + d * ngt, s);
     }
     if (eom_dft) {

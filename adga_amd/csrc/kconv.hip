@@ -188,13 +188,14 @@ __device__ __forceinline__ void dft_line_n(int n, z64* x, int stride, double sig
 
 // What a field is made of: itself (`a`), the bubble's product of transforms
 // a = Ghat(nu_d)_il(-R) times b = Ghat(nu_d - omega)_k'j(R) for field (d, c = (i l)(k' j)), or that product's
-// derivative a(-R) db(R) + da(-R) b(R).
-enum { DFT_FIELD = 0, DFT_PRODUCT = 1, DFT_DERIVATIVE = 2 };
+// derivative a(-R) db(R) + da(-R) b(R), or component ab of the G table [w][k][ab] at frequency w, read in place
+// (field (w, ab); the n2 workgroups of a frequency run on one XCD, whose L2 holds the lines they share).
+enum { DFT_FIELD = 0, DFT_PRODUCT = 1, DFT_DERIVATIVE = 2, DFT_TABLE = 3 };
 struct DftSource {
   const z64* a;
   const z64* da;       // the derivative's table
   int n2;
-  long a0, b0;         // first field of the nu and of the nu - omega table
+  long a0, b0;         // first field of the nu and of the nu - omega table; a0 of DFT_TABLE: its frequencies
 };
 
 template <int SRC>
@@ -204,7 +205,12 @@ __global__ void __launch_bounds__(512) k_dft3_lds(int nx, int ny, int nz, double
   z64* x = reinterpret_cast<z64*>(dft_lds);
   const int t = threadIdx.x, nt = blockDim.x;
   const int per = nx * ny * nz, pz = nz | 1, pyz = ny * pz;
-  const long f = blockIdx.x;
+  long f = blockIdx.x;
+  if constexpr (SRC == DFT_TABLE) {
+    const long slot = f >> 3, w = slot / src.n2 * 8 + (f & 7);
+    if (w >= src.a0) return;
+    f = w * src.n2 + slot % src.n2;
+  }
   // element e = t + i nt is (row r, z): its row and z advance by fixed amounts, no division per element
   const int r0 = t / nz, z0 = t % nz, dr = nt / nz, dz = nt % nz;
   auto next = [&](int& r, int& z) {
@@ -215,7 +221,7 @@ __global__ void __launch_bounds__(512) k_dft3_lds(int nx, int ny, int nz, double
       ++r;
     }
   };
-  if constexpr (SRC != DFT_FIELD) {
+  if constexpr (SRC == DFT_PRODUCT || SRC == DFT_DERIVATIVE) {
     const int n2 = src.n2, n4 = n2 * n2, c = (int)(f % n4);
     const long d = f / n4;
     const z64* a = src.a + (src.a0 + d * n2 + c / n2) * per;
@@ -241,11 +247,12 @@ __global__ void __launch_bounds__(512) k_dft3_lds(int nx, int ny, int nz, double
       }
     }
   } else {
-    const z64* in = src.a + f * per;
+    const int n2 = SRC == DFT_TABLE ? src.n2 : 1;
+    const z64* in = SRC == DFT_TABLE ? src.a + f / n2 * per * n2 + f % n2 : src.a + f * per;
     int r = r0, z = z0;
 #pragma unroll 4
     for (int e = t; e < per; e += nt) {
-      x[r * pz + z] = in[e];
+      x[r * pz + z] = in[(long)e * n2];
       next(r, z);
     }
   }
@@ -307,8 +314,15 @@ __global__ void k_gt_fields(Geom g, const z64* __restrict__ gt, z64* __restrict_
   out[idx] = gt[(w * g.nkp + k) * g.n2 + ab];
 }
 
-// Ghat[w][ab][R] = sum_k G(k, nu_w)_ab e^{-ikR}, for every frequency of the G table.
+// Ghat[w][ab][R] = sum_k G(k, nu_w)_ab e^{-ikR}, for every frequency of the G table (tmp: as large as it, only
+// where the transform takes the passes over HBM).  In LDS the strided reads of the table cost less than a pass
+// that transposes it: three orbitals, 20^3, 60 frequencies 0.40 -> 0.20 ms, and a first pass along 41 q points
+// 8.2 -> 7.5 ms with the scratch's allocation and release gone.
 void launch_ghat(const Geom& g, const z64* tw, const z64* gt, z64* tmp, z64* ghat, hipStream_t s) {
+  if (dft_in_lds(g)) {
+    dft3_lds<DFT_TABLE>(g, (g.nw + 7L) / 8 * 8 * g.n2, -1, DftSource{gt, nullptr, g.n2, g.nw, 0}, ghat, s);
+    return;
+  }
   long tot = (long)g.nw * g.n2 * g.nkp;
   hipLaunchKernelGGL(k_gt_fields, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s, g, gt, tmp);
   dft3(g, (long)g.nw * g.n2, -1, tw, tmp, ghat, s);
