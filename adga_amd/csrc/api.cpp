@@ -136,6 +136,17 @@ void widen_gtable(adga_ctx* c) {
   CK(hipStreamSynchronize(c->stream));
 }
 
+// The accumulated m_tot (and its derivatives) zero again.  Only a pending omega leaves anything there, in the
+// first part of each array, its box's (3.3 GB and 1.05 ms for the largest box of five orbitals on 16^3).
+void eom_clear(adga_ctx* c) {
+  if (!c->eom_pending) return;
+  const size_t per = (size_t)c->g.n4 * c->g.nkp, used = sizeof(z64) * c->eom_g.iwf * per;
+  CK(hipMemsetAsync(c->macc, 0, used, c->stream));
+  for (int d = 0; d < c->ndir && c->t_macc; ++d)
+    CK(hipMemsetAsync(c->t_macc + d * c->g.iwf * per, 0, used, c->stream));
+  c->eom_pending = false;
+}
+
 void eom_flush(adga_ctx* c) {
   if (!c->eom_pending) return;
   const size_t nm = (size_t)c->g.iwf * c->g.n4 * c->g.nkp;
@@ -153,9 +164,7 @@ void eom_flush(adga_ctx* c) {
   adga::launch_eom_flush(c->eom_g, c->eom_iwb, c->keom, c->tw, c->ghat, c->macc, c->mwork, c->sig_nl, c->stream,
                          tan.ndir ? &tan : nullptr);
   CK(hipGetLastError());
-  CK(hipMemsetAsync(c->macc, 0, sizeof(z64) * nm, c->stream));
-  if (tan.ndir) CK(hipMemsetAsync(c->t_macc, 0, sizeof(z64) * nm * tan.ndir, c->stream));
-  c->eom_pending = false;
+  eom_clear(c);
 }
 
 // LU operation list of the current omega's BSE size; prec 0: complex128 LU, prec 1: complex64 LU
@@ -1092,10 +1101,7 @@ int adga_reset_sigma(adga_ctx* c) {
     CK(hipMemsetAsync(c->sig_dmft, 0, sizeof(z64) * g.n2 * g.nf, c->stream));
     CK(hipMemsetAsync(c->sig_hf, 0, sizeof(z64) * g.n2 * g.nkp_eom, c->stream));
     if (c->t_sig) CK(hipMemsetAsync(c->t_sig, 0, sizeof(z64) * g.n2 * g.nf * g.nkp_eom * c->ndir, c->stream));
-    if (c->macc) CK(hipMemsetAsync(c->macc, 0, sizeof(z64) * (size_t)g.iwf * g.n4 * g.nkp, c->stream));
-    if (c->t_macc)
-      CK(hipMemsetAsync(c->t_macc, 0, sizeof(z64) * (size_t)g.iwf * g.n4 * g.nkp * c->ndir, c->stream));
-    c->eom_pending = false;
+    eom_clear(c);
     c->bub_valid = false;  // the next batch forms the bubble of its omega again
     c->t_bub_valid = false;
     CK(hipStreamSynchronize(c->stream));
