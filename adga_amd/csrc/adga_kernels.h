@@ -115,7 +115,7 @@ enum ResidMode { RESID_OF = 0, RESID_STEP = 1, RESID_START = 2 };
 bool resid_step_pending(const VqTerm* vq);
 void launch_residual(const Geom& g, int npts, const z64* S, const z64* cd, const z64* cm, const z64* B, z64* Y,
                      z64* Z, z64* R, const ResidNorm& nrm, hipStream_t s, const VqTerm* vq = nullptr,
-                     ResidMode mode = RESID_OF, LuTimer* timer = nullptr);
+                     ResidMode mode = RESID_OF, LuTimer* timer = nullptr, bool norm = true);
 // V(q) (vq.hip): W of a batch (qpos: 0-based q list positions, vq: (n2, n2, nqp)); the density matrices'
 // term; Out_{2b} += (1 + gamma^w_d)^T (W^T X) with X = (1 + gamma^w_d)^T (Y null) or the density solution Y
 void launch_vq_w(const Geom& g, int npts, const int* qpos, const z64* vq, const z64* chi0q, z64* W, hipStream_t s);

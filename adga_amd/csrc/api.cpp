@@ -418,7 +418,8 @@ bool series_solve(adga_ctx* c, int nb, double tol, double accept, const z64* B, 
     prev.assign(relh.begin(), relh.begin() + 2 * k);
     for (int j = 0; j < count; ++j)
       adga::launch_residual(g, k, c->S, c->cd, c->cm, B, Y, c->Z, c->R, c->nrm, s, vtp,
-                            j == 0 ? mode : adga::RESID_STEP, k == nb && !(start && j == 0) ? &c->lut : nullptr);
+                            j == 0 ? mode : adga::RESID_STEP, k == nb && !(start && j == 0) ? &c->lut : nullptr,
+                            j + 1 == count);  // only the last one's norms are read
     CK(hipMemcpyAsync(relh.data(), c->nrm.rel, sizeof(double) * 2 * k, hipMemcpyDeviceToHost, s));
     CK(hipStreamSynchronize(s));
     done += count;

@@ -615,8 +615,9 @@ k_resid_gemm(Geom g, int npts, int ch0, int nch, const z64* __restrict__ cd, con
 
 // Out = C_ch^T Z_ch (+ B - Y when B is given, + Out itself when accumulate), rows r0 .. N - 1.  64 x 64 tiles from four rounds
 // of the chip's 512 such workgroups on; below, 32 x 32 tiles lose less to the last round and to few
-// workgroups (64 x 64 against 32 x 32: N = 1080, 27000 columns 3.21 / 3.50 ms; N = 4000, 2400 columns
-// 4.26 / 4.40; N = 2000, 3200 columns 1.44 / 1.39; N = 540, 738 columns 89 / 50 us; N = 40, 1024 columns 15 / 8).
+// workgroups (64 x 64 against 32 x 32, columns of both channels: N = 1080, 27000 columns 3.37 / 3.64 ms;
+// N = 4000, 2400 columns 3.89 / 4.25; below the line, timed before the staging moved between the MFMAs:
+// N = 2000, 3200 columns 1.44 / 1.39; N = 540, 738 columns 89 / 50 us; N = 40, 1024 columns 15 / 8).
 void resid_gemm(const Geom& g, int npts, int ch0, int nch, const z64* cd, const z64* cm, const z64* Z, z64* Out,
                 const z64* B, const z64* Y, hipStream_t s, bool accumulate, unsigned long long* rmax, int r0,
                 bool update) {
@@ -784,7 +785,7 @@ void launch_add(long n, const z64* R, z64* Y, hipStream_t s) {
 }
 
 // R = B - M Y with M Y = Y - C^T (blockdiag(S)^T Y), in FP64 from the unrounded factors S and C (with V(q):
-// minus (1 + gamma^w_d)^T (W^T Y) in the density channel), and its norms.  M = 1 - T with
+// minus (1 + gamma^w_d)^T (W^T Y) in the density channel), and with `norm` its norms.  M = 1 - T with
 // T Y = C^T (blockdiag(S)^T Y), so steps Y += R from Y = B sum the series (1 + T + T^2 + ...) B.
 //   RESID_OF     of Y as given, stored to R
 //   RESID_START  of Y = B, RESID_STEP of the last call's Y + R, for the fixed-point iteration: without V(q) the
@@ -796,7 +797,7 @@ bool resid_step_pending(const VqTerm* vq) { return vq != nullptr; }
 
 void launch_residual(const Geom& g, int npts, const z64* S, const z64* cd, const z64* cm, const z64* B, z64* Y,
                      z64* Z, z64* R, const ResidNorm& nrm, hipStream_t s, const VqTerm* vq, ResidMode mode,
-                     LuTimer* timer) {
+                     LuTimer* timer, bool norm) {
   const int nmat = 2 * npts;
   const bool start = mode == RESID_START, update = mode != RESID_OF && !resid_step_pending(vq);
   if (start)
@@ -807,14 +808,15 @@ void launch_residual(const Geom& g, int npts, const z64* S, const z64* cd, const
     timer->mark(s);
     timer->flops += 8.0 * g.N * (double)g.N * g.n2 * nmat;
   }
-  resid_gemm(g, npts, 0, 2, cd, cm, Z, update ? Y : R, B, update && start ? B : Y, s, false, vq ? nullptr : nrm.rmax,
-             0, update);
+  resid_gemm(g, npts, 0, 2, cd, cm, Z, update ? Y : R, B, update && start ? B : Y, s, false,
+             norm && !vq ? nrm.rmax : nullptr, 0, update);
   if (timer) timer->mark(s);
   if (vq) {
     launch_vq_add(g, npts, *vq, Y, R, s);
-    hipLaunchKernelGGL(k_absmax, dim3(nmat), dim3(256), 0, s, (long)g.N * g.n2, R, nrm.rmax, nullptr);
+    if (norm) hipLaunchKernelGGL(k_absmax, dim3(nmat), dim3(256), 0, s, (long)g.N * g.n2, R, nrm.rmax, nullptr);
   }
-  hipLaunchKernelGGL(k_resid_rel, dim3((nmat + 255) / 256), dim3(256), 0, s, nmat, nrm.bmax, nrm.rmax, nrm.rel);
+  if (norm)
+    hipLaunchKernelGGL(k_resid_rel, dim3((nmat + 255) / 256), dim3(256), 0, s, nmat, nrm.bmax, nrm.rmax, nrm.rel);
 }
 
 }  // namespace adga

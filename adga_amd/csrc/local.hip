@@ -76,9 +76,13 @@ __global__ void k_local_bubble(Geom g, int iwb, const z64* __restrict__ giw, z64
 
 // ---------------------------------------------------------------- A5: chi0^w F
 // C(i1, i2) = 0.5 (X(i1,i2) + X(i2,i1)) * winv(i2) - delta(i1,i2), Fortran column-major
-// (main.F90:529-553).  32x32 tiles through LDS so both X reads are coalesced.
-__global__ void __launch_bounds__(256) k_chi0wF(int N, const z64* __restrict__ x, const z64* __restrict__ winv,
-                                                z64* __restrict__ c) {
+// (main.F90:529-553).  32x32 tiles through LDS so both X reads are coalesced; blockIdx.z: the channel (a launch
+// each cost small boxes 5 us more).
+__global__ void __launch_bounds__(256) k_chi0wF(int N, const z64* __restrict__ xd, const z64* __restrict__ xm,
+                                                const z64* __restrict__ winv, z64* __restrict__ cd,
+                                                z64* __restrict__ cm) {
+  const z64* x = blockIdx.z == 0 ? xd : xm;
+  z64* c = blockIdx.z == 0 ? cd : cm;
   __shared__ z64 tile[32][33];
   int bx = blockIdx.x * 32, by = blockIdx.y * 32;  // bx: i1 block, by: i2 block
   int tx = threadIdx.x % 32, ty = threadIdx.x / 32;  // 8 rows of threads
@@ -102,13 +106,19 @@ __global__ void __launch_bounds__(256) k_chi0wF(int N, const z64* __restrict__ x
 }
 
 // gamma^w(s, j) = sum_d C(d*n2 + s, j); (1+gamma^w)(s, j) = gamma^w(s, j) + [j % n2 == s]
-// (main.F90:557-571, 616-625).  Output (n2, N) Fortran.
-__global__ void k_gammaw(Geom g, const z64* __restrict__ c, z64* __restrict__ gam, z64* __restrict__ opg) {
+// (main.F90:557-571, 616-625).  Output (n2, N) Fortran; blockIdx.y: the channel.  The sums run in order, eight
+// loads ahead: a small box has too few threads to hide a load each.
+__global__ void k_gammaw(Geom g, const z64* __restrict__ cd, const z64* __restrict__ cm, z64* __restrict__ gam_d,
+                         z64* __restrict__ gam_m, z64* __restrict__ opg_d, z64* __restrict__ opg_m) {
+  const z64* c = blockIdx.y == 0 ? cd : cm;
+  z64* gam = blockIdx.y == 0 ? gam_d : gam_m;
+  z64* opg = blockIdx.y == 0 ? opg_d : opg_m;
   long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (idx >= (long)g.n2 * g.N) return;
   int s = (int)(idx % g.n2);
   long j = idx / g.n2;
   z64 acc = mk(0.0, 0.0);
+#pragma unroll 8
   for (int d = 0; d < g.nf; ++d) acc = cadd(acc, c[(long)(d * g.n2 + s) + j * g.N]);
   gam[idx] = acc;
   if ((int)(j % g.n2) == s) acc.re += 1.0;
@@ -125,6 +135,7 @@ __global__ void k_local_chi(Geom g, const z64* __restrict__ gam_d, const z64* __
   int s1 = idx % g.n2, s2 = idx / g.n2;
   z64 ad = mk(0.0, 0.0), am = mk(0.0, 0.0), bl = mk(0.0, 0.0);
   double ib2 = 1.0 / (g.beta * g.beta);
+#pragma unroll 8
   for (int d = 0; d < g.nf; ++d) {
     z64 w = chi0w[s2 + d * g.n2];  // diagonal element chi0w(s2, s2, d)
     long col = (long)(d * g.n2 + s2) * g.n2;
@@ -142,13 +153,11 @@ void launch_local(const Geom& g, int iwb, const z64* giw, const z64* xd, const z
                   z64* chiloc_m, z64* bubloc, hipStream_t s) {
   int nb = (g.n2 * g.nf + 255) / 256;
   hipLaunchKernelGGL(k_local_bubble, dim3(nb), dim3(256), 0, s, g, iwb, giw, winv, chi0w);
-  dim3 tg((g.N + 31) / 32, (g.N + 31) / 32);
-  hipLaunchKernelGGL(k_chi0wF, tg, dim3(256), 0, s, g.N, xd, winv, cd);
-  hipLaunchKernelGGL(k_chi0wF, tg, dim3(256), 0, s, g.N, xm, winv, cm);
+  dim3 tg((g.N + 31) / 32, (g.N + 31) / 32, 2);
+  hipLaunchKernelGGL(k_chi0wF, tg, dim3(256), 0, s, g.N, xd, xm, winv, cd, cm);
   long tot = (long)g.n2 * g.N;
-  dim3 gg((unsigned)((tot + 255) / 256));
-  hipLaunchKernelGGL(k_gammaw, gg, dim3(256), 0, s, g, cd, gam_d, opg_d);
-  hipLaunchKernelGGL(k_gammaw, gg, dim3(256), 0, s, g, cm, gam_m, opg_m);
+  dim3 gg((unsigned)((tot + 255) / 256), 2);
+  hipLaunchKernelGGL(k_gammaw, gg, dim3(256), 0, s, g, cd, cm, gam_d, gam_m, opg_d, opg_m);
   hipLaunchKernelGGL(k_local_chi, dim3((g.n4 + 255) / 256), dim3(256), 0, s, g, gam_d, gam_m, chi0w, chiloc_d,
                      chiloc_m, bubloc);
 }
