@@ -1,6 +1,6 @@
 // adga_inverse_matrix_z_noalloc: the inverse of adga_inverse_matrix_z (the same kernels, gj.hip) with every
 // device buffer it needs carved from one file-scope device array, so that a call makes no device allocation.
-// Each GPU the library runs on holds its own copy of the array (about 50.9 MB at the largest n) until the
+// Each GPU the library runs on holds its own copy of the array (about 51.1 MB at the largest n) until the
 // process ends; every call on a GPU shares it, so calls that overlap on one GPU race.
 #include <hip/hip_runtime.h>
 
@@ -15,7 +15,7 @@ using adga::z64;
 
 constexpr int NA_MAX_N = ADGA_INVERSE_NOALLOC_MAX_N;
 constexpr long NA_MAT = (long)NA_MAX_N * NA_MAX_N;  // complex elements of a matrix buffer, three of them
-constexpr long NA_G = 2L * NA_MAX_N * 16;           // the panels (gj_scratch at NA_MAX_N)
+constexpr long NA_G = 3L * NA_MAX_N * 16 + 1;       // the panels (gj_scratch at NA_MAX_N)
 constexpr long NA_INTS = 2 * NA_MAX_N + 1;          // pivots, row states, status
 constexpr long NA_ELEMS = 3 * NA_MAT + NA_G + (NA_INTS * (long)sizeof(int) + sizeof(z64) - 1) / sizeof(z64);
 constexpr int NA_MAX_DEV = 64;
