@@ -3,6 +3,7 @@
 #include <cmath>
 #include <cstring>
 #include <mutex>
+#include <numeric>
 
 #include "ctx.h"
 
@@ -62,25 +63,11 @@ void ensure_batch(adga_ctx* c, int nb) {
   c->cap = nb;
 }
 
-// LU workspace of a batch of nb points (sized for complex128 and the largest box), apart from the rest: a
-// context whose batches all converge by fixed-point iteration never holds it
-void ensure_lu(adga_ctx* c, int nb) {
-  if (nb <= c->lu_cap) return;
-  free_lu(c);
-  nb = std::max(nb, c->cap);
-  const Geom& g = c->g;
-  dalloc((char**)&c->M, 2 * nb * (size_t)g.N * c->ldm * sizeof(z64));
-  dalloc((char**)&c->inv, 2 * nb * adga::lu_inv_elems(g.N) * sizeof(z64));
-  dalloc(&c->piv, 2 * nb * (size_t)g.N);
-  dalloc(&c->info, 2 * nb);
-  dalloc(&c->act, 2 * nb);
-  c->lu_cap = nb;
-}
-
 // V(q) workspace of a batch of nb points
 void ensure_vq_batch(adga_ctx* c, int nb) {
   if (nb <= c->vq_cap) return;
   dfree(c->W); dfree(c->vqQ); dfree(c->qpos);
+  c->vq_cap = 0;
   const Geom& g = c->g;
   dalloc(&c->W, (size_t)nb * g.N * g.n2);
   dalloc(&c->vqQ, (size_t)nb * g.n4);
@@ -90,7 +77,8 @@ void ensure_vq_batch(adga_ctx* c, int nb) {
 
 void ensure_conv(adga_ctx* c) {
   const Geom& g = c->g;
-  if (c->tw) return;
+  if (c->ghat) return;  // allocated last: then the rest is there too
+  dfree(c->tw);
   // forward twiddles e^{-2 pi i R k / n} of the three axes
   std::vector<z64> tw;
   for (int n : {g.nkx, g.nky, g.nkz})
@@ -102,13 +90,14 @@ void ensure_conv(adga_ctx* c) {
   dalloc(&c->tw, tw.size());
   CK(hipMemcpy(c->tw, tw.data(), sizeof(z64) * tw.size(), hipMemcpyHostToDevice));
   size_t ng = (size_t)g.nw * g.n2 * g.nkp;
-  dalloc(&c->ghat, ng);
   if (adga::dft_in_lds(g)) {
+    dalloc(&c->ghat, ng);
     adga::launch_ghat(g, c->tw, c->gt, nullptr, c->ghat, c->stream);
     CK(hipGetLastError());
     return;
   }
   DevBuf<> tmp(ng);
+  dalloc(&c->ghat, ng);
   adga::launch_ghat(g, c->tw, c->gt, tmp.p, c->ghat, c->stream);
   CK(hipGetLastError());
   CK(hipStreamSynchronize(c->stream));
@@ -259,38 +248,78 @@ namespace {
 // Steps of the fixed-point iteration (series_solve) that cost about what the LU of the same batch does.
 int series_steps(const Geom& g) { return std::min(8 + g.N / (4 * g.n2), 2 + g.N / 8); }
 
-// FP64 LU solve of the points `pts` (batch positions) whose complex64 refinement or iteration did not converge:
-// their S and right-hand sides are gathered, the density and magnetic matrices rebuilt in complex128,
-// factored, solved and checked, and the solutions scattered back into the batch's Y.  Updates the
-// points' entries of relh / infoh and returns the number of matrices re-solved.
-int fallback_fp64(adga_ctx* c, const std::vector<int>& pts, std::vector<double>& relh, std::vector<int>& infoh) {
+// Workspace of solve_fp64, sized for the largest box (c->g): one point, or with `full` at most 4 GB of complex128
+// matrices (two per point) and 32 points; where memory does not reach, half as many, and so on.
+void ensure_fallback(adga_ctx* c, bool full) {
+  FallbackBufs& f = c->fb;
+  const Geom& G = c->g;
+  const size_t per_mat = (size_t)G.N * c->ldm, pmat = (size_t)G.N * G.n2;
+  const size_t fit = ((size_t)4 << 30) / (2 * per_mat * sizeof(z64));
+  int cap = full ? (int)std::max<size_t>(1, std::min<size_t>(32, fit)) : 1;
+  for (; cap > f.cap; cap /= 2) {
+    free_fallback(c);
+    try {
+      dalloc(&f.S, (size_t)cap * G.nf * G.n4);
+      dalloc(&f.B, 2 * cap * pmat);
+      dalloc(&f.Y, 2 * cap * pmat);
+      dalloc(&f.Z, 2 * cap * pmat);
+      dalloc(&f.R, 2 * cap * pmat);
+      dalloc(&f.M, 2 * cap * per_mat);
+      dalloc(&f.inv, 2 * cap * adga::lu_inv_elems(G.N));
+      alloc_norm(f.nrm, 2 * cap);
+      dalloc(&f.piv, 2 * cap * (size_t)G.N);
+      dalloc(&f.info, 2 * cap);
+      dalloc(&f.sel, cap);
+      f.cap = cap;
+    } catch (const HipError& e) {
+      free_fallback(c);
+      if (e.e != hipErrorOutOfMemory || cap == 1) throw;
+      (void)hipGetLastError();
+    }
+  }
+}
+
+}  // namespace
+
+namespace adga_host {
+// LU workspace of a batch of nb points (sized for complex128 and the largest box), apart from the rest: a context
+// whose batches all converge by fixed-point iteration never holds it.  False where memory does not reach for it
+// (150 GB for 4000 points of N = 1080): the batch's points are then solved a few at a time (solve_fp64).
+bool ensure_lu(adga_ctx* c, int nb) {
+  if (nb <= c->lu_cap) return true;
+  free_lu(c);
+  const Geom& g = c->g;
+  try {
+    dalloc((char**)&c->M, 2 * nb * (size_t)g.N * c->ldm * sizeof(z64));
+    dalloc((char**)&c->inv, 2 * nb * adga::lu_inv_elems(g.N) * sizeof(z64));
+    dalloc(&c->piv, 2 * nb * (size_t)g.N);
+    dalloc(&c->info, 2 * nb);
+    dalloc(&c->act, 2 * nb);
+  } catch (const HipError& e) {
+    free_lu(c);
+    if (e.e != hipErrorOutOfMemory) throw;
+    (void)hipGetLastError();
+    return false;
+  }
+  c->lu_cap = nb;
+  return true;
+}
+
+// FP64 LU solve of the points `pts` (batch positions) of M Y = B, a few at a time: their S and right-hand sides are
+// gathered, the density and magnetic matrices built in complex128, factored, solved and checked, and the solutions
+// scattered into Y.  For points whose complex64 refinement or iteration did not converge, and for all of a batch
+// whose factors do not fit the memory.  Updates the points' entries of relh / infoh and returns the number of
+// matrices solved.
+int solve_fp64(adga_ctx* c, const std::vector<int>& pts, const z64* B, z64* Y, std::vector<double>& relh,
+               std::vector<int>& infoh) {
   const Geom& g = c->gw;
   hipStream_t s = c->stream;
   if (pts.empty()) return 0;
   const std::vector<int>& ops64 = ensure_ops(c, 0);
   FallbackBufs& f = c->fb;
-  if (f.cap == 0) {
-    // sized for the largest box (c->g); at most 4 GB of complex128 matrices (two per point), at most
-    // 32 points per round
-    const Geom& G = c->g;
-    const size_t per_mat = (size_t)G.N * c->ldm;
-    const size_t fit = ((size_t)4 << 30) / (2 * per_mat * sizeof(z64));
-    const int cap = (int)std::max<size_t>(1, std::min<size_t>(32, fit));
-    const size_t pmat = (size_t)G.N * G.n2;
-    dalloc(&f.S, (size_t)cap * G.nf * G.n4);
-    dalloc(&f.B, 2 * cap * pmat);
-    dalloc(&f.Y, 2 * cap * pmat);
-    dalloc(&f.Z, 2 * cap * pmat);
-    dalloc(&f.R, 2 * cap * pmat);
-    dalloc(&f.M, 2 * cap * per_mat);
-    dalloc(&f.inv, 2 * cap * adga::lu_inv_elems(G.N));
-    alloc_norm(f.nrm, 2 * cap);
-    dalloc(&f.piv, 2 * cap * (size_t)G.N);
-    dalloc(&f.info, 2 * cap);
-    dalloc(&f.sel, cap);
-    f.cap = cap;
-  }
-  if (c->vq && !f.W) {
+  ensure_fallback(c, true);
+  if (c->vq && !f.Q) {
+    dfree(f.W);
     dalloc(&f.W, (size_t)f.cap * c->g.N * c->g.n2);
     dalloc(&f.Q, (size_t)f.cap * c->g.n4);
   }
@@ -302,7 +331,7 @@ int fallback_fp64(adga_ctx* c, const std::vector<int>& pts, std::vector<double>&
     const int k = (int)std::min<size_t>(f.cap, pts.size() - i0);
     CK(hipMemcpyAsync(f.sel, &pts[i0], sizeof(int) * k, hipMemcpyHostToDevice, s));
     adga::launch_gather(k, slen, f.sel, c->S, f.S, false, s);
-    adga::launch_gather(k, blen, f.sel, c->Bp, f.B, false, s);
+    adga::launch_gather(k, blen, f.sel, B, f.B, false, s);
     adga::launch_build<double>(g, k, c->ldm, f.S, c->cd, c->cm, f.M, s);
     const adga::VqTerm fv{f.W, c->opgd, f.Q};
     if (c->vq) {
@@ -314,7 +343,7 @@ int fallback_fp64(adga_ctx* c, const std::vector<int>& pts, std::vector<double>&
       throw HipError{hipErrorInvalidValue, "FP64 re-solve: BSE size outside the LU kernel's range"};
     adga::launch_absmax_rhs(g, k, f.B, f.nrm, s);
     adga::launch_residual(g, k, f.S, c->cd, c->cm, f.B, f.Y, f.Z, f.R, f.nrm, s, c->vq ? &fv : nullptr);
-    adga::launch_gather(k, blen, f.sel, f.Y, c->Y, true, s);
+    adga::launch_gather(k, blen, f.sel, f.Y, Y, true, s);
     r.resize(2 * k);
     inf.resize(2 * k);
     CK(hipMemcpyAsync(r.data(), f.nrm.rel, sizeof(double) * 2 * k, hipMemcpyDeviceToHost, s));
@@ -329,7 +358,9 @@ int fallback_fp64(adga_ctx* c, const std::vector<int>& pts, std::vector<double>&
   }
   return done;
 }
+}  // namespace adga_host
 
+namespace {
 // FP64 iterative refinement of the complex64 solves of a batch of nb points (2 nb matrices), per
 // matrix: a matrix stops when its relative residual max|r|/max|b| reaches refine_tol; it is handed to
 // the FP64 re-solve when its complex64 LU met an exactly zero pivot, a residual is not finite, a
@@ -380,7 +411,7 @@ int refine(adga_ctx* c, int nb, std::vector<double>& relh, std::vector<int>& inf
       pts.push_back(b);
       resolved[2 * b] = resolved[2 * b + 1] = 1;
     }
-  c->stats[14] += fallback_fp64(c, pts, relh, infoh);
+  c->stats[14] += solve_fp64(c, pts, c->Bp, c->Y, relh, infoh);
   return iters;
 }
 
@@ -469,7 +500,6 @@ bool series_solve(adga_ctx* c, int nb, double tol, double accept, const z64* B, 
 
 bool factor_fp64(adga_ctx* c, int nb) {
   const Geom& g = c->gw;
-  ensure_lu(c, nb);
   const adga::VqTerm vt{c->W, c->opgd, c->vqQ};
   adga::launch_build<double>(g, nb, c->ldm, c->S, c->cd, c->cm, (z64*)c->M, c->stream);
   if (c->vq) adga::launch_vq_build<double>(g, nb, c->ldm, vt, (z64*)c->M, c->stream);
@@ -756,18 +786,6 @@ int run_points_impl(adga_ctx* c, int npts, const int* iq, int precision, double*
       const adga::VqTerm* vtp = c->vq ? &vt : nullptr;
       const int nmat = 2 * nb;
       CK(hipEventRecord(ev[0], s));
-      // local EOM for points at the Gamma point (main.F90:635-639)
-      for (int b = 0; b < nb && c->do_eom; ++b)
-        if (iq[p0 + b] == 1) {
-          adga::launch_eom_local(g, c->iwb, c->iwb == 0, c->u, c->gamd, c->giw, c->ndmft, c->sig_dmft, s);
-          if (c->vq && c->iwb == 0) adga::launch_eom_hartree_v(g, c->vq, c->ndmft, c->sig_hf, s);
-        }
-      if (c->vq && c->do_eom && c->iwb == 0) {
-        // non-local Fock term of every point at omega = 0 (calc_eom_static, main.F90:635-637)
-        ensure_nfock(c);
-        adga::launch_eom_fock(g, nb, c->qpos, c->qidx, c->keom, c->vq, c->nfock, c->sig_hf, s);
-      }
-      CK(hipEventRecord(ev[1], s));
       const bool bub_hit = c->bub_valid && c->bub_iwb == c->iwb && c->bub_iwf == g.iwf;
       const bool use_dft = c->bubble_mode == 1 || (c->bubble_mode == 2 && (bub_hit || nb >= bubble_dft_points(c)));
       if (use_dft) {
@@ -791,7 +809,7 @@ int run_points_impl(adga_ctx* c, int npts, const int* iq, int precision, double*
       if (vtp) adga::launch_vq_w(g, nb, c->qpos, c->vq, c->chi0q, c->W, s);
       if (c->do_eom) adga::launch_gamq(g, nb, c->S, c->cd, c->Z, c->gamq, s);
       adga::launch_rhs(g, nb, c->S, c->cd, c->cm, c->opgd, c->opgm, c->Z, c->Bp, s, vtp);
-      CK(hipEventRecord(ev[2], s));
+      CK(hipEventRecord(ev[1], s));
       int iters = 0;
       double maxrel = 0.0;
       bool lu_ok = adga::lu_supported(g.N), factored = false;
@@ -807,16 +825,24 @@ int run_points_impl(adga_ctx* c, int npts, const int* iq, int precision, double*
                                              &steps);
       if (series && !left.empty() && (tan || !c->fallback)) series = false;  // these need every point's factors
       if (series) {
-        CK(hipEventRecord(ev[3], s));
+        CK(hipEventRecord(ev[2], s));
         for (int b : left) resolved[2 * b] = resolved[2 * b + 1] = 1;
-        const int again = fallback_fp64(c, left, relh, infoh);
+        const int again = solve_fp64(c, left, c->Bp, c->Y, relh, infoh);
         if (prec == 1) {
           c->stats[14] += again;
           iters = std::max(0, steps - 1);  // the steps that correct Y = (1 + T) B
         }
+      } else if (lu_ok && !ensure_lu(c, nb)) {
+        CK(hipEventRecord(ev[2], s));
+        left.resize(nb);
+        std::iota(left.begin(), left.end(), 0);
+        resolved.assign(nmat, 1);
+        c->lut.used = 0;
+        c->lut.flops = 0.0;
+        const int again = solve_fp64(c, left, c->Bp, c->Y, relh, infoh);
+        if (prec == 1) c->stats[14] += again;
       } else if (lu_ok) {
         factored = true;
-        ensure_lu(c, nb);
         c->lut.used = 0;  // the timer brackets the factorisation's kernel, not an iteration given up
         c->lut.flops = 0.0;
         const bool rhs = carry_rhs(c, prec);
@@ -829,7 +855,7 @@ int run_points_impl(adga_ctx* c, int npts, const int* iq, int precision, double*
           adga::launch_build<double>(g, nb, c->ldm, c->S, c->cd, c->cm, (z64*)c->M, s);
           if (vtp) adga::launch_vq_build<double>(g, nb, c->ldm, vt, (z64*)c->M, s);
           if (rhs) adga::launch_rhs_into_m<double>(nmat, g.N, n2, c->ldm, c->Bp, (z64*)c->M, s);
-          CK(hipEventRecord(ev[3], s));
+          CK(hipEventRecord(ev[2], s));
           CK(hipEventRecord(c->ev_lu[0], s));
           lu_ok = adga::launch_lu<double>(nmat, g.N, W, c->ldm, ops, (z64*)c->M, c->piv, (z64*)c->inv, c->info, s,
                                           &c->lut, &lanes);
@@ -849,7 +875,7 @@ int run_points_impl(adga_ctx* c, int npts, const int* iq, int precision, double*
           adga::launch_build<float>(g, nb, c->ldm, c->S, c->cd, c->cm, (c32*)c->M, s);
           if (vtp) adga::launch_vq_build<float>(g, nb, c->ldm, vt, (c32*)c->M, s);
           if (rhs) adga::launch_rhs_into_m<float>(nmat, g.N, n2, c->ldm, c->Bp, (c32*)c->M, s);
-          CK(hipEventRecord(ev[3], s));
+          CK(hipEventRecord(ev[2], s));
           CK(hipEventRecord(c->ev_lu[0], s));
           lu_ok = adga::launch_lu<float>(nmat, g.N, W, c->ldm, ops, (c32*)c->M, c->piv, (c32*)c->inv, c->info, s,
                                          &c->lut, &lanes);
@@ -884,7 +910,7 @@ int run_points_impl(adga_ctx* c, int npts, const int* iq, int precision, double*
           ++nfailed;
         }
       }
-      CK(hipEventRecord(ev[4], s));
+      CK(hipEventRecord(ev[3], s));
       adga::launch_chi(g, nb, c->Y, c->chi0q, c->chi0w, c->gamd, c->gamm, c->bubloc, c->R, c->chi_out,
                        c->bub_out, s);
       if (c->bubble_range >= 1) {
@@ -904,7 +930,30 @@ int run_points_impl(adga_ctx* c, int npts, const int* iq, int precision, double*
         }
         adga::launch_bubble_outer_add(g, nb, c->qidx, c->outer_all, c->bub_out, s);
       }
-      CK(hipEventRecord(ev[5], s));
+      CK(hipEventRecord(ev[4], s));
+      // what the batch adds to the self-energy comes last, after everything that can fail for want of memory: a call
+      // that was refused can be repeated
+      if (tan && !factored) ensure_fallback(c, false);  // the derivatives' solves
+      if (c->do_eom && c->eom_mode == 1) {
+        ensure_conv(c);
+        if (!c->macc) {
+          const size_t nm = (size_t)c->g.iwf * g.n4 * g.nkp;  // sized for the largest box
+          DevBuf<> m(nm);
+          dalloc(&c->mwork, nm);
+          std::swap(c->macc, m.p);
+          CK(hipMemsetAsync(c->macc, 0, sizeof(z64) * nm, s));
+        }
+      }
+      if (c->vq && c->do_eom && c->iwb == 0) ensure_nfock(c);
+      // local EOM for points at the Gamma point (main.F90:635-639)
+      for (int b = 0; b < nb && c->do_eom; ++b)
+        if (iq[p0 + b] == 1) {
+          adga::launch_eom_local(g, c->iwb, c->iwb == 0, c->u, c->gamd, c->giw, c->ndmft, c->sig_dmft, s);
+          if (c->vq && c->iwb == 0) adga::launch_eom_hartree_v(g, c->vq, c->ndmft, c->sig_hf, s);
+        }
+      // non-local Fock term of every point at omega = 0 (calc_eom_static, main.F90:635-637)
+      if (c->vq && c->do_eom && c->iwb == 0)
+        adga::launch_eom_fock(g, nb, c->qpos, c->qidx, c->keom, c->vq, c->nfock, c->sig_hf, s);
       if (c->do_eom) {
         adga::launch_mtot(g, nb, c->u, c->ut, c->Y, c->gamq, c->mt, s, c->qpos, c->vq, c->gamd);  // eta = Y
         if (nfailed > 0) {
@@ -912,13 +961,6 @@ int run_points_impl(adga_ctx* c, int npts, const int* iq, int precision, double*
           adga::launch_zero_points(nb, (long)n2 * g.N, c->keep, c->mt, s);
         }
         if (c->eom_mode == 1) {
-          ensure_conv(c);
-          if (!c->macc) {
-            size_t nm = (size_t)c->g.iwf * g.n4 * g.nkp;  // sized for the largest box
-            dalloc(&c->macc, nm);
-            dalloc(&c->mwork, nm);
-            CK(hipMemsetAsync(c->macc, 0, sizeof(z64) * nm, s));
-          }
           if (c->eom_pending && (c->eom_iwb != c->iwb || c->eom_g.iwf != g.iwf)) eom_flush(c);
           adga::launch_eom_scatter(g, nb, c->qidx, c->mt, c->macc, s, c->q_distinct);
           c->eom_pending = true;
@@ -928,7 +970,7 @@ int run_points_impl(adga_ctx* c, int npts, const int* iq, int precision, double*
           adga::launch_eom_direct(g, c->iwb, nb, c->qidx, c->keom, c->mt, c->gt, c->sig_nl, s);
         }
       }
-      CK(hipEventRecord(ev[6], s));
+      CK(hipEventRecord(ev[5], s));
       CK(hipGetLastError());
       if (tan) tangent_batch(c, nb, p0, npts, keep, nfailed, *tan, factored);
       chih.resize((size_t)2 * nb * g.n4);
@@ -936,14 +978,13 @@ int run_points_impl(adga_ctx* c, int npts, const int* iq, int precision, double*
       CK(hipMemcpyAsync(chih.data(), c->chi_out, sizeof(z64) * chih.size(), hipMemcpyDeviceToHost, s));
       CK(hipMemcpyAsync(bubh.data(), c->bub_out, sizeof(z64) * bubh.size(), hipMemcpyDeviceToHost, s));
       CK(hipStreamSynchronize(s));
-      float ms[6];
-      for (int k = 0; k < 6; ++k) CK(hipEventElapsedTime(&ms[k], ev[k], ev[k + 1]));
-      c->stats[2 + 5] += ms[0];            // EOM (local part)
-      c->stats[2 + 1] += ms[1];            // Chi0
-      c->stats[2 + 2] += ms[2];            // Gammas (BSE build)
-      c->stats[2 + 3] += ms[3];            // Inversion (LU, solve, refinement, FP64 re-solves)
-      c->stats[2 + 6] += ms[4];            // Chi (eta + contraction)
-      c->stats[2 + 5] += ms[5];            // EOM
+      float ms[5];
+      for (int k = 0; k < 5; ++k) CK(hipEventElapsedTime(&ms[k], ev[k], ev[k + 1]));
+      c->stats[2 + 1] += ms[0];            // Chi0
+      c->stats[2 + 2] += ms[1];            // Gammas (BSE build)
+      c->stats[2 + 3] += ms[2];            // Inversion (iteration, LU, solve, refinement, FP64 re-solves)
+      c->stats[2 + 6] += ms[3];            // Chi (eta + contraction)
+      c->stats[2 + 5] += ms[4];            // EOM
       if (factored) {
         float lums = 0.f;
         CK(hipEventElapsedTime(&lums, c->ev_lu[0], c->ev_lu[1]));

@@ -5,6 +5,7 @@
 // factors): each direction costs two bubble passes (product rule: the bubble is formed again, not
 // stored), a right-hand side and a solve with the existing factors, chi's contraction and two EOM passes.
 #include <cstring>
+#include <numeric>
 
 #include "ctx.h"
 
@@ -17,6 +18,7 @@ void ensure_tangent_batch(adga_ctx* c, int nb) {
   for (z64** p : {&c->t_dchi0q, &c->t_dS, &c->t_Z1, &c->t_Z2, &c->t_B, &c->t_dY, &c->t_dgamq, &c->t_dmt,
                   &c->t_dchi, &c->t_dbub})
     dfree(*p);
+  c->t_cap = 0;
   const Geom& g = c->g;  // the largest box
   const size_t per_pt = (size_t)g.nf * g.n4, pmat = (size_t)g.N * g.n2;
   dalloc(&c->t_dchi0q, nb * per_pt);
@@ -57,7 +59,7 @@ void tangent_batch(adga_ctx* c, int nb, int p0, int npts, const std::vector<int>
   ensure_tangent_batch(c, nb);
   const int nmat = 2 * nb;
   std::vector<double> relh;
-  std::vector<int> left;
+  std::vector<int> left, infoh;
   const size_t tab = (size_t)G.nw * G.nkp * G.n2, loc = (size_t)G.n2 * G.nf, cc = (size_t)G.N * G.N,
                pm = (size_t)G.n2 * G.N, nsig = (size_t)G.n2 * G.nf * G.nkp_eom;
   for (int dir = 0; dir < c->ndir; ++dir) {
@@ -91,14 +93,23 @@ void tangent_batch(adga_ctx* c, int nb, int p0, int npts, const std::vector<int>
       adga::launch_bubble(g, c->iwb, nb, c->qidx, c->gt, c->t_dchi0q, s, dgt, true);
     }
     adga::launch_dsmat(g, nb, c->chi0q, c->t_dchi0q, c->winv, dwinv, c->t_dS, s);
-    // d eta: M d eta^T = C^T Z1 + dC^T Z2, by the forward solve's iteration or with its complex128 factors
+    // d eta: M d eta^T = C^T Z1 + dC^T Z2, by the forward solve's iteration or with its complex128 factors; formed
+    // here if the forward solve needed none, and kept for the next directions, or without memory for them a few
+    // points at a time
     adga::launch_tangent_rhs(g, nb, c->S, c->t_dS, c->cd, c->cm, dcd, dcm, c->opgd, c->opgm, dgamd, dgamm, c->Y,
                              c->t_Z1, c->t_Z2, c->t_B, s);
     if (!factored) {
       relh.assign(nmat, 0.0);
-      if (!series_solve(c, nb, SERIES_TOL64, SERIES_ACCEPT64, c->t_B, c->t_dY, relh, left) || !left.empty()) {
+      infoh.assign(nmat, 0);
+      const bool iterated = c->series && series_solve(c, nb, SERIES_TOL64, SERIES_ACCEPT64, c->t_B, c->t_dY, relh, left) &&
+                            left.empty();
+      if (!iterated && ensure_lu(c, nb)) {
         if (!factor_fp64(c, nb)) throw HipError{hipErrorInvalidValue, "tangent solve: BSE size outside the LU's range"};
         factored = true;
+      } else if (!iterated) {
+        left.resize(nb);
+        std::iota(left.begin(), left.end(), 0);
+        solve_fp64(c, left, c->t_B, c->t_dY, relh, infoh);
       }
     }
     if (factored &&

@@ -53,7 +53,7 @@ struct adga_ctx {
   int device = 0;      // the device current at creation: the context's streams belong to it
   long lane_key = -1;  // shape of this context's factorisation whose trial time is pending (-1: none)
   int lane_trial = 0;  // its lane count
-  hipEvent_t ev[7] = {}, ev_lu[2] = {};    // stage and LU timing of adga_run_points
+  hipEvent_t ev[6] = {}, ev_lu[2] = {};    // stage and LU timing of adga_run_points
   std::string err;
   int refine_maxit = 12;
   double refine_tol = 1e-12;
@@ -251,8 +251,13 @@ bool series_solve(adga_ctx* c, int nb, double tol, double accept, const z64* B, 
                   std::vector<int>& left, int* steps = nullptr);
 // the FP64 mode's relative residual: the aim, and what a residual at its round-off may be
 constexpr double SERIES_TOL64 = 1e-15, SERIES_ACCEPT64 = 1e-14;
-// the batch's M in complex128, factored (api.cpp); false: BSE size outside the LU kernel's range
+// the LU workspace of a batch (M, inv, piv, info, act of the context); false: not enough memory (api.cpp)
+bool ensure_lu(adga_ctx* c, int nb);
+// the batch's M in complex128, factored, in the workspace; false: BSE size outside the LU kernel's range
 bool factor_fp64(adga_ctx* c, int nb);
+// M Y = B of the points `pts` by complex128 LU a few at a time; returns the matrices solved
+int solve_fp64(adga_ctx* c, const std::vector<int>& pts, const z64* B, z64* Y, std::vector<double>& relh,
+               std::vector<int>& infoh);
 void free_tangent(adga_ctx* c);
 // the twiddles and the k-grid transform of the G table (formed once); the pending omega's EOM flushed
 // (with its derivatives when tangent directions are set) (api.cpp)

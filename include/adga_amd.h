@@ -329,7 +329,8 @@ int adga_get_ndga(adga_ctx *ctx, const double *sigma_sum, double *n_dga_k, doubl
  * their number (0 where no batch was factored), out[11..13] = milliseconds, algorithmic flops and launches
  * of the BSE solve's dominant GEMM kernel (the factorisation's largest tile shape, or the iteration's residual
  * product), out[14] = matrices solved again in complex128
- * after their complex64 refinement or the refined mode's iteration failed, out[15] = points with a non-zero status.
+ * after their complex64 refinement or the refined mode's iteration failed, or at once where the factors of a
+ * batch did not fit the memory, out[15] = points with a non-zero status.
  */
 int adga_get_stats(adga_ctx *ctx, double *out, int nout);
 
