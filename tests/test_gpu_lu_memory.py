@@ -11,6 +11,7 @@ from adga_amd import synth
 
 pytestmark = pytest.mark.gpu
 NPTS = 8420
+GPU_BYTES = 288 << 30
 
 
 def _setup(noise=1e-3):
@@ -21,12 +22,11 @@ def _setup(noise=1e-3):
 
 
 def test_gpu_lu_beyond_memory():
-    import torch
     from adga_amd import _lib, api
     inp, x = _setup()
     iq = np.arange(1, NPTS + 1, dtype=np.int32)
     need = 2 * NPTS * 1080 * 1088 * 16
-    assert need > torch.cuda.get_device_properties(0).total_memory
+    assert need > 1.02 * GPU_BYTES
     out = []
     for batch in (NPTS, 2000):
         print(f"LU of {NPTS} points in batches of {batch}", flush=True)
