@@ -241,7 +241,14 @@ namespace adga_host {
 // per (nu, orbital component, k), so the line is a number of points.  Three orbitals, 20^3, 60 frequencies: 0.51 ms
 // at any number against 0.43 / 0.61 ms for 16 / 24 points summed directly; five, 16^3, 40: 1.05 against 0.98 for 24
 // and 1.23 for 32.  Four orbitals fill the matrix tiles of the direct sum (12^3, 40: 0.42 against 0.41 for 64).
-int bubble_dft_points(const adga_ctx* c) { return c->g.n == 3 || c->g.n == 5 ? 24 : 64; }
+// Grids whose transform does not run in LDS take three passes over HBM, some three times as long, and a second
+// table: 64 for every number of orbitals.
+int bubble_dft_points(const adga_ctx* c) {
+  return adga::dft_in_lds(c->g) && (c->g.n == 3 || c->g.n == 5) ? 24 : 64;
+}
+bool bubble_by_dft(const adga_ctx* c, int nb, bool hit) {
+  return c->bubble_mode == 1 || (c->bubble_mode == 2 && (hit || nb >= bubble_dft_points(c)));
+}
 }  // namespace adga_host
 
 namespace {
@@ -258,7 +265,7 @@ void ensure_fallback(adga_ctx* c, bool full) {
   int cap = full ? (int)std::max<size_t>(1, std::min<size_t>(32, fit)) : 1;
   for (; cap > f.cap; cap /= 2) {
     free_fallback(c);
-    try {
+    auto alloc = [&] {
       dalloc(&f.S, (size_t)cap * G.nf * G.n4);
       dalloc(&f.B, 2 * cap * pmat);
       dalloc(&f.Y, 2 * cap * pmat);
@@ -271,11 +278,9 @@ void ensure_fallback(adga_ctx* c, bool full) {
       dalloc(&f.info, 2 * cap);
       dalloc(&f.sel, cap);
       f.cap = cap;
-    } catch (const HipError& e) {
-      free_fallback(c);
-      if (e.e != hipErrorOutOfMemory || cap == 1) throw;
-      (void)hipGetLastError();
-    }
+    };
+    if (cap == 1) alloc();
+    else if (!fits_memory(alloc)) free_fallback(c);
   }
 }
 
@@ -289,20 +294,16 @@ bool ensure_lu(adga_ctx* c, int nb) {
   if (nb <= c->lu_cap) return true;
   free_lu(c);
   const Geom& g = c->g;
-  try {
+  const bool ok = fits_memory([&] {
     dalloc((char**)&c->M, 2 * nb * (size_t)g.N * c->ldm * sizeof(z64));
     dalloc((char**)&c->inv, 2 * nb * adga::lu_inv_elems(g.N) * sizeof(z64));
     dalloc(&c->piv, 2 * nb * (size_t)g.N);
     dalloc(&c->info, 2 * nb);
     dalloc(&c->act, 2 * nb);
-  } catch (const HipError& e) {
-    free_lu(c);
-    if (e.e != hipErrorOutOfMemory) throw;
-    (void)hipGetLastError();
-    return false;
-  }
-  c->lu_cap = nb;
-  return true;
+  });
+  if (ok) c->lu_cap = nb;
+  else free_lu(c);
+  return ok;
 }
 
 // FP64 LU solve of the points `pts` (batch positions) of M Y = B, a few at a time: their S and right-hand sides are
@@ -787,15 +788,21 @@ int run_points_impl(adga_ctx* c, int npts, const int* iq, int precision, double*
       const int nmat = 2 * nb;
       CK(hipEventRecord(ev[0], s));
       const bool bub_hit = c->bub_valid && c->bub_iwb == c->iwb && c->bub_iwf == g.iwf;
-      const bool use_dft = c->bubble_mode == 1 || (c->bubble_mode == 2 && (bub_hit || nb >= bubble_dft_points(c)));
+      bool use_dft = bubble_by_dft(c, nb, bub_hit);
+      if (use_dft && !bub_hit) {
+        const size_t nb_all = (size_t)c->g.nf * g.n4 * g.nkp;  // sized for the largest box
+        const auto tables = [&] {
+          ensure_conv(c);
+          if (!adga::dft_in_lds(g) && !c->bub_p) dalloc(&c->bub_p, nb_all);
+          if (!c->bub_all) dalloc(&c->bub_all, nb_all);
+        };
+        // the default mode sums directly where the tables do not fit the memory
+        use_dft = fits_memory(tables);
+        if (!use_dft && !c->bub_all) dfree(c->bub_p);
+        if (!use_dft && c->bubble_mode == 1) throw HipError{hipErrorOutOfMemory, "the bubble of every q"};
+      }
       if (use_dft) {
-        ensure_conv(c);
         if (!bub_hit) {
-          size_t nb_all = (size_t)c->g.nf * g.n4 * g.nkp;  // sized for the largest box
-          if (!c->bub_all) {
-            if (!adga::dft_in_lds(g) && !c->bub_p) dalloc(&c->bub_p, nb_all);
-            dalloc(&c->bub_all, nb_all);
-          }
           adga::launch_bubble_all(g, c->iwb, c->tw, c->ghat, c->bub_p, c->bub_all, s);
           c->bub_valid = true;
           c->bub_iwb = c->iwb;

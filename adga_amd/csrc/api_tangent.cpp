@@ -62,31 +62,36 @@ void tangent_batch(adga_ctx* c, int nb, int p0, int npts, const std::vector<int>
   std::vector<int> left, infoh;
   const size_t tab = (size_t)G.nw * G.nkp * G.n2, loc = (size_t)G.n2 * G.nf, cc = (size_t)G.N * G.N,
                pm = (size_t)G.n2 * G.N, nsig = (size_t)G.n2 * G.nf * G.nkp_eom;
+  // the derivatives' bubbles: for every q of the omega at once by k-grid convolution (formed again, not stored from
+  // the forward pass, and kept for the omega's next batches), or as direct sums per batch, as the forward bubble's
+  // mode chooses
+  const size_t nall = (size_t)G.nf * G.n4 * G.nkp;  // sized for the largest box
+  const bool t_hit = c->t_bub_valid && c->t_bub_iwb == c->iwb && c->t_bub_iwf == g.iwf;
+  bool dft = c->t_dghat && bubble_by_dft(c, nb, t_hit);
+  if (dft && !t_hit) {
+    const auto tables = [&] {
+      if (!adga::dft_in_lds(g) && !c->t_bub_p) dalloc(&c->t_bub_p, nall);
+      if (!c->t_dbub_all) dalloc(&c->t_dbub_all, nall * c->ndir);
+    };
+    dft = fits_memory(tables);
+    if (!dft && !c->t_dbub_all) dfree(c->t_bub_p);
+    if (!dft && c->bubble_mode == 1) throw HipError{hipErrorOutOfMemory, "the bubbles' derivatives of every q"};
+  }
+  if (dft && !t_hit) {
+    for (int d = 0; d < c->ndir; ++d)
+      adga::launch_bubble_all_tangent(g, c->iwb, c->tw, c->ghat, c->t_dghat + d * tab, c->t_bub_p,
+                                      c->t_dbub_all + d * nall, s);
+    c->t_bub_valid = true;
+    c->t_bub_iwb = c->iwb;
+    c->t_bub_iwf = g.iwf;
+  }
   for (int dir = 0; dir < c->ndir; ++dir) {
     const z64* dgt = c->dgt + dir * tab;
     const z64 *dw = c->t_dw + dir * loc, *dwinv = c->t_dwinv + dir * loc;
     const z64 *dcd = c->t_dcd + dir * cc, *dcm = c->t_dcm + dir * cc;
     const z64 *dgamd = c->t_dgamd + dir * pm, *dgamm = c->t_dgamm + dir * pm;
-    // dchi0q = bubble(dG(k, nu), G(k - q, nu - omega)) + bubble(G(k, nu), dG(k - q, nu - omega)): for every q
-    // of the omega at once by k-grid convolution (formed again, not stored from the forward pass, and kept
-    // for the omega's next batches), or as direct sums per batch, as the forward bubble's mode chooses
-    const bool t_hit = c->t_bub_valid && c->t_bub_iwb == c->iwb && c->t_bub_iwf == g.iwf;
-    if (c->t_dghat && (c->bubble_mode == 1 || (c->bubble_mode == 2 && (t_hit || nb >= bubble_dft_points(c))))) {
-      const size_t nall = (size_t)G.nf * G.n4 * G.nkp;  // sized for the largest box
-      if (!t_hit) {
-        if (dir == 0) {
-          if (!c->t_dbub_all) {
-            if (!adga::dft_in_lds(g) && !c->t_bub_p) dalloc(&c->t_bub_p, nall);
-            dalloc(&c->t_dbub_all, nall * c->ndir);
-          }
-          for (int d = 0; d < c->ndir; ++d)
-            adga::launch_bubble_all_tangent(g, c->iwb, c->tw, c->ghat, c->t_dghat + d * tab, c->t_bub_p,
-                                            c->t_dbub_all + d * nall, s);
-          c->t_bub_valid = true;
-          c->t_bub_iwb = c->iwb;
-          c->t_bub_iwf = g.iwf;
-        }
-      }
+    // dchi0q = bubble(dG(k, nu), G(k - q, nu - omega)) + bubble(G(k, nu), dG(k - q, nu - omega))
+    if (dft) {
       adga::launch_bubble_gather(g, nb, c->qidx, c->t_dbub_all + dir * nall, c->t_dchi0q, s);
     } else {
       adga::launch_bubble(g, c->iwb, nb, c->qidx, dgt, c->t_dchi0q, s, c->gt, false);

@@ -188,6 +188,18 @@ void dfree(T*& p) {
   if (p) (void)hipFree((void*)p);
   p = nullptr;
 }
+// runs allocations; false where memory does not reach for them (what some of them obtained stays)
+template <typename F>
+bool fits_memory(F&& alloc) {
+  try {
+    alloc();
+    return true;
+  } catch (const HipError& e) {
+    if (e.e != hipErrorOutOfMemory) throw;
+    (void)hipGetLastError();
+    return false;
+  }
+}
 inline void upload(z64* d, const double* h, size_t count, hipStream_t s) {
   CK(hipMemcpyAsync(d, h, count * sizeof(z64), hipMemcpyHostToDevice, s));
 }
@@ -262,8 +274,8 @@ void free_tangent(adga_ctx* c);
 // the twiddles and the k-grid transform of the G table (formed once); the pending omega's EOM flushed
 // (with its derivatives when tangent directions are set) (api.cpp)
 void conv_tables(adga_ctx* c);
-// points of a batch from which the bubble is formed for every q at once
-int bubble_dft_points(const adga_ctx* c);
+// whether a batch of nb points takes the bubble of every q at once (`hit`: it is there already), by the context's mode
+bool bubble_by_dft(const adga_ctx* c, int nb, bool hit);
 void flush_eom(adga_ctx* c);
 
 }  // namespace adga_host

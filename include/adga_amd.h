@@ -81,8 +81,9 @@ int adga_ctx_create(const adga_dims *dims, const int *q_data, const int *k_data_
  * LU always), "do_eom" (1: the default; 0: no
  * equation of motion, as the reference's do_eom = .false. for a q path),
  * "bubble" (0: direct k sum per point; 1: all q of the current omega at once by
- * k-grid DFT, cached per omega; 2: DFT when a batch has enough points (24 with three or five orbitals,
- * 64 otherwise) or the cache is valid, the default), "eom" (0: direct sum per batch; 1: m_tot accumulated on the q grid and convolved with
+ * k-grid DFT, cached per omega; 2: DFT when a batch has enough points (24 with three or five orbitals on
+ * a grid whose axes have at most 24 points and whose padded field fits the LDS, nkpx nkpy (nkpz | 1) <= 10240;
+ * 64 otherwise) or the cache is valid, and the tables of every q fit the memory, the default), "eom" (0: direct sum per batch; 1: m_tot accumulated on the q grid and convolved with
  * G by k-grid DFT when omega changes or the self-energy is read, the default), "lu_streams" (1: each
  * batch's LU on one stream; 2 .. 4: the batch split into that many parts on as many streams, each one
  * operation behind the previous, the large Schur updates on the whole batch; 0, the default: chosen per
