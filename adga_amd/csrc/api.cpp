@@ -460,7 +460,7 @@ bool series_solve(adga_ctx* c, int nb, double tol, double accept, const z64* B, 
       if (start) rho[m] = fell;
       need[m] = 0;
       if (r <= tol) continue;
-      if (!start && r <= 8 * accept && !(fell < 0.5)) continue;  // at round-off
+      if (!start && r <= 8 * SERIES_ACCEPT64 && !(fell < 0.5)) continue;  // at round-off
       rho[m] = std::max(rho[m], fell);
       const double n = rho[m] < 1.0 && std::isfinite(r) ? std::ceil(std::log(tol / r) / std::log(rho[m])) : INFINITY;
       need[m] = (int)std::min(n, (double)kmax + 1);

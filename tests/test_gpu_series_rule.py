@@ -1,0 +1,33 @@
+"""The fixed-point iteration's decisions (option series = 1): which points go on, which are solved by an LU, and what
+accuracy the refined mode leaves."""
+import numpy as np
+import pytest
+
+from adga_amd import synth
+from test_gpu_series import _workload
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(wl, npts, precision, change=None, **opt):
+    """(results, statistics) of the first npts q points at omega = 1 in one batch"""
+    from adga_amd import api
+    inp = synth.build_inputs(wl)
+    if change:
+        change(inp)
+    print(f"n={wl.n} N={wl.maxdim} points={npts} noise={wl.noise} {precision} {opt}", flush=True)
+    with api.Context(inp, batch=npts, **opt) as ctx:
+        ctx.set_local_omega(1, *[synth.chi_loc(inp, 1, c) for c in ("dens", "magn")])
+        r = ctx.run_points(np.arange(1, npts + 1, dtype=np.int32), precision)
+        st = ctx.stats()
+    assert (r["status"] == 0).all()
+    return r, st
+
+
+@pytest.mark.parametrize("noise,tol", [(0.5, 1e-6), (0.6, 1e-6), (0.65, 1e-6), (0.5, 1e-9), (0.55, 1e-9)])
+def test_gpu_series_goes_on_above_round_off(noise, tol):
+    """N = 400, contractions of 0.5 to 0.7 a step: a residual that falls by less than half a step, a few times above
+    the caller's tolerance, is not at round-off; the iteration goes on to the tolerance."""
+    st = _run(_workload(1, (4, 4, 4), 200, noise), 64, "refined", refine_tol=tol)[1]
+    assert st["n_lu_launches"] == 0 and st["n_fp64_resolved"] == 0
+    assert st["refine_resid"] <= tol
