@@ -252,8 +252,29 @@ bool bubble_by_dft(const adga_ctx* c, int nb, bool hit) {
 }  // namespace adga_host
 
 namespace {
-// Steps of the fixed-point iteration (series_solve) that cost about what the LU of the same batch does.
-int series_steps(const Geom& g) { return std::min(8 + g.N / (4 * g.n2), 2 + g.N / 8); }
+// Steps of the fixed-point iteration (series_solve) that cost no more than the LU of the same batch, in complex128
+// (prec 0) or in complex64 with its refinement (1).  Measured, in steps, the LU costs (N = 40, 512 points) 10 / 3,
+// (136, 301) 40 / 22, (200, 512) 75 / 37, (540, 41) 100 / 75, (540, 500) 50 / 30, (960, 200) 48 / 40, (1080, 500)
+// 75 / 42, (2000, 64) 50 / 33, (4000, 16) 110 / 60.  None for the smallest in the refined mode: 512 points of N = 40
+// take 0.41 to 0.44 ms by the iteration, 0.43 by the LU and 0.48 by the LU after a look at the contraction.
+int series_steps(const Geom& g, int prec) {
+  return prec == 1 && g.N < 80 ? 0 : std::min(8 + g.N / (4 * g.n2), 2 + g.N / 8);
+}
+
+// Milliseconds of a step, of the LU of the batch and of the complex128 LU of a few of its points (solve_fp64), within
+// some 20%: a latency of N times 4.75 us (N = 136) to 10 us (N >= 1080), the flops at the LU's rate.
+struct SolveCost {
+  double product, step, lu, latency, per_point;
+  SolveCost(const Geom& g, int nb, int prec, bool vq) {
+    const double N = g.N, rate = std::min(47e9, 6e7 * N);  // flops per ms in complex128
+    product = 16 * N * N * g.n2 * nb / 55e9;
+    step = (vq ? 0.055 : 0.02) + product;
+    latency = 1e-3 * N * std::min(10.0, 4 + N / 180);
+    per_point = 16 / 3.0 * N * N * N / rate;
+    lu = prec == 0 ? latency + nb * per_point : 0.75 * latency + nb * per_point / 1.9 + 2 * step;
+  }
+  double singles(int n) const { return (n + 31) / 32 * latency + n * per_point; }
+};
 
 // Workspace of solve_fp64, sized for the largest box (c->g): one point, or with `full` at most 4 GB of complex128
 // matrices (two per point) and 32 points; where memory does not reach, half as many, and so on.
@@ -426,17 +447,24 @@ namespace adga_host {
 // instability).
 //
 // The rule: the residuals' ratio gives each matrix's contraction rho (the first one, |T B| / |B|, and the
-// later |r'| / |r| where those are worse), hence the steps ln(tol / r) / ln(rho) it still needs; the LU is
-// taken (false, Y undefined) as soon as more than one point in eight needs over series_steps() of them in
-// all - for a large batch from three products on its first 8 points, so that a batch that does not contract
-// costs next to nothing, and for a small one from its first one or two.  The steps predicted are queued
-// together: a few waits per batch.  They go on to `tol`, or until the residual stops falling; a matrix whose
-// residual then is above `accept` puts its point into `left`.  `steps`: those taken.
-bool series_solve(adga_ctx* c, int nb, double tol, double accept, const z64* B, z64* Y, std::vector<double>& relh,
+// later |r'| / |r| where those are worse), hence the steps ln(tol / r) / ln(rho) it still needs; a point that
+// needs over series_steps() more of them is slow.  What counts is what is still to do, not what is done: a point
+// that needs a few steps more than foreseen gets them, where the LU would cost many.  The LU is taken (false, Y
+// undefined) as soon as the other points' steps and the single LUs of the slow ones cost more than it does
+// (41 points of N = 540: a step 0.04 ms, the complex64 LU of the batch 3.6, the complex128 LU of one
+// point 3.8), or one point in eight is slow, or one is and `singles` is not allowed - for a batch of expensive products from three
+// of them on its first 8 points, so that a batch that does not contract costs next to nothing, and for the others
+// from the first one or two.  The steps predicted are queued together: a few waits per batch.  They go on to
+// `tol`, or until the residual stops falling; a matrix whose residual then is above `accept`
+// puts its point into `left` (none without `singles`).  `steps`: those taken.
+bool series_solve(adga_ctx* c, int nb, const SeriesGoal& goal, const z64* B, z64* Y, std::vector<double>& relh,
                   std::vector<int>& left, int* steps) {
   const Geom& g = c->gw;
   hipStream_t s = c->stream;
-  const int kmax = series_steps(g);
+  const double tol = goal.tol, accept = goal.accept;
+  const int kmax = series_steps(g, goal.prec);
+  if (kmax < 1) return false;
+  const SolveCost cost(g, nb, goal.prec, c->vq != nullptr);
   const adga::VqTerm vt{c->W, c->opgd, c->vqQ};
   const adga::VqTerm* vtp = c->vq ? &vt : nullptr;
   std::vector<double> rho(2 * nb, 0.0), prev;
@@ -466,26 +494,32 @@ bool series_solve(adga_ctx* c, int nb, double tol, double accept, const z64* B, 
       need[m] = (int)std::min(n, (double)kmax + 1);
     }
   };
-  auto slow = [&](int k) {  // points among the first k that need more than kmax steps in all
+  // over kmax more steps, or over twice as many in all: a prediction that keeps growing
+  auto is_slow = [&](int m) { return need[m] > kmax || done + need[m] > 2 * kmax; };
+  auto slow = [&](int k) {  // points among the first k
     int n = 0;
-    for (int b = 0; b < k; ++b) n += done + std::max(need[2 * b], need[2 * b + 1]) > kmax;
+    for (int b = 0; b < k; ++b) n += is_slow(2 * b) || is_slow(2 * b + 1);
     return n;
   };
   left.clear();
   if (steps) *steps = 0;
   adga::launch_absmax_rhs(g, nb, B, c->nrm, s);
+  // a look at a few points pays where a product on all takes longer than three waits (512 points of N = 40: iterated
+  // 0.36 ms, 0.46 with the look; given up for the LU 0.63, 0.61 with the look, 0.56 untried)
   constexpr int LOOK = 8;
-  if (nb >= 8 * LOOK) {
+  if (nb >= 8 * LOOK && cost.product > 0.1) {
     advance(LOOK, adga::RESID_START, 1);
     for (int k = 0; k < 2 && 2 * slow(LOOK) <= LOOK; ++k) advance(LOOK, adga::RESID_STEP, 1);
     if (2 * slow(LOOK) > LOOK) return false;
   }
   advance(nb, adga::RESID_START, 1);
   for (;;) {
-    if (8 * slow(nb) > nb) return false;
+    const int n = slow(nb);
     int k = 0;
     for (int m = 0; m < 2 * nb; ++m)
-      if (done + need[m] <= kmax) k = std::max(k, need[m]);
+      if (!is_slow(m)) k = std::max(k, need[m]);
+    // the costs are known within some 20%: in doubt the points are kept apart
+    if (n > 0 && (!goal.singles || 8 * n > nb || k * cost.step + cost.singles(n) > 1.25 * cost.lu)) return false;
     if (k == 0) break;
     if (done == 1 && nb < 8 * LOOK) k = std::min(k, 1);  // a second look at the contraction first
     advance(nb, adga::RESID_STEP, k);
@@ -493,7 +527,7 @@ bool series_solve(adga_ctx* c, int nb, double tol, double accept, const z64* B, 
   }
   for (int b = 0; b < nb; ++b)
     if (!(relh[2 * b] <= accept && relh[2 * b + 1] <= accept)) left.push_back(b);
-  if (8 * left.size() > (size_t)nb) return false;
+  if (!left.empty() && (!goal.singles || 8 * left.size() > (size_t)nb)) return false;
   // the last residual is at hand: one more step, whose residual is below the one tested by the contraction
   if (adga::resid_step_pending(vtp)) adga::launch_add(2L * nb * g.N * g.n2, c->R, Y, s);
   return true;
@@ -828,9 +862,10 @@ int run_points_impl(adga_ctx* c, int npts, const int* iq, int precision, double*
       // (4e-7 at N = 1080); one below the round-off of a residual is left to the LU and its limits
       const double tol = prec == 0 ? SERIES_TOL64 : std::min(c->refine_tol, 1e-6);
       int steps = 0;
-      bool series = lu_ok && c->series && tol >= SERIES_TOL64 && series_solve(c, nb, tol, prec == 0 ? SERIES_ACCEPT64 : tol, c->Bp, c->Y, relh, left,
-                                             &steps);
-      if (series && !left.empty() && (tan || !c->fallback)) series = false;  // these need every point's factors
+      // the derivatives and the option "fallback" off need the factors of every point or of none
+      const SeriesGoal goal{prec, tol, prec == 0 ? SERIES_ACCEPT64 : tol, !tan && c->fallback};
+      const bool series =
+          lu_ok && c->series && tol >= SERIES_TOL64 && series_solve(c, nb, goal, c->Bp, c->Y, relh, left, &steps);
       if (series) {
         CK(hipEventRecord(ev[2], s));
         for (int b : left) resolved[2 * b] = resolved[2 * b + 1] = 1;

@@ -258,11 +258,18 @@ inline int op_finish(adga_ctx* c, bool launched, const char* what) {
 // (factored: the batch's complex128 factors are in c->M; else its forward solve was the fixed-point iteration)
 void tangent_batch(adga_ctx* c, int nb, int p0, int npts, const std::vector<int>& keep, int nfailed,
                    const TangentOut& out, bool factored);
-// M Y = B for every matrix of a batch by fixed-point iteration in FP64; false where the LU is to be taken
-bool series_solve(adga_ctx* c, int nb, double tol, double accept, const z64* B, z64* Y, std::vector<double>& relh,
-                  std::vector<int>& left, int* steps = nullptr);
 // the FP64 mode's relative residual: the aim, and what a residual at its round-off may be
 constexpr double SERIES_TOL64 = 1e-15, SERIES_ACCEPT64 = 1e-14;
+// of the fixed-point iteration: the LU it competes with (0 complex128, 1 complex64 and refinement), the relative
+// residual it aims at and the one it may end with, and whether single points may be left to an LU of their own
+struct SeriesGoal {
+  int prec;
+  double tol, accept;
+  bool singles;
+};
+// M Y = B for every matrix of a batch by fixed-point iteration in FP64; false where the LU is to be taken
+bool series_solve(adga_ctx* c, int nb, const SeriesGoal& goal, const z64* B, z64* Y, std::vector<double>& relh,
+                  std::vector<int>& left, int* steps = nullptr);
 // the LU workspace of a batch (M, inv, piv, info, act of the context); false: not enough memory (api.cpp)
 bool ensure_lu(adga_ctx* c, int nb);
 // the batch's M in complex128, factored, in the workspace; false: BSE size outside the LU kernel's range

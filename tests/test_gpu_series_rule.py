@@ -31,3 +31,31 @@ def test_gpu_series_goes_on_above_round_off(noise, tol):
     st = _run(_workload(1, (4, 4, 4), 200, noise), 64, "refined", refine_tol=tol)[1]
     assert st["n_lu_launches"] == 0 and st["n_fp64_resolved"] == 0
     assert st["refine_resid"] <= tol
+
+
+@pytest.mark.parametrize("precision,noise", [("fp64", 0.4), ("fp64", 0.45), ("refined", 0.5)])
+def test_gpu_series_gets_the_last_steps(precision, noise):
+    """41 points of N = 540, where a step costs a hundredth of any LU: points that need a few steps more than foreseen
+    get them; neither they nor the batch are factored after some twenty steps."""
+    st = _run(_workload(3, (4, 4, 3), 30, noise), 41, precision)[1]
+    assert st["n_lu_launches"] == 0 and st["n_fp64_resolved"] == 0
+    assert st["refine_resid"] <= (1e-14 if precision == "fp64" else 1e-12)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "refined"])
+def test_gpu_series_slow_point_in_a_small_batch(precision):
+    """V(q) strong at one of 48 points: the LU of that point alone costs nearly what the LU of all does, so the batch
+    is factored at the first sign of it."""
+
+    def v_q(inp):
+        inp.v_q[:, :, 40] = 60.0 * np.eye(4)
+
+    st = _run(_workload(2, (4, 4, 3), 17, 1e-3, vq=0.02), 48, precision, change=v_q)[1]
+    assert st["n_lu_launches"] == 1
+
+
+def test_gpu_series_leaves_the_smallest_refined_systems_to_the_lu():
+    """N = 40: a complex64 LU costs about three steps."""
+    wl = _workload(1, (8, 8, 8), 20, 0.01)
+    assert _run(wl, 512, "refined")[1]["n_lu_launches"] == 1
+    assert _run(wl, 512, "fp64")[1]["n_lu_launches"] == 0
