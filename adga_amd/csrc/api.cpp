@@ -447,7 +447,7 @@ namespace adga_host {
 // instability).
 //
 // The rule: the residuals' ratio gives each matrix's contraction rho (the first one, |T B| / |B|, and the
-// later |r'| / |r| where those are worse), hence the steps ln(tol / r) / ln(rho) it still needs; a point that
+// later |r'| / |r| where those are worse), hence the steps ln(aim / r) / ln(rho) it still needs; a point that
 // needs over series_steps() more of them is slow.  What counts is what is still to do, not what is done: a point
 // that needs a few steps more than foreseen gets them, where the LU would cost many.  The LU is taken (false, Y
 // undefined) as soon as the other points' steps and the single LUs of the slow ones cost more than it does
@@ -455,23 +455,23 @@ namespace adga_host {
 // point 3.8), or one point in eight is slow, or one is and `singles` is not allowed - for a batch of expensive products from three
 // of them on its first 8 points, so that a batch that does not contract costs next to nothing, and for the others
 // from the first one or two.  The steps predicted are queued together: a few waits per batch.  They go on to
-// `tol`, or until the residual stops falling; a matrix whose residual then is above `accept`
+// the goal's aim, or until the residual stops falling; a matrix whose residual then is above `accept`
 // puts its point into `left` (none without `singles`).  `steps`: those taken.
 bool series_solve(adga_ctx* c, int nb, const SeriesGoal& goal, const z64* B, z64* Y, std::vector<double>& relh,
                   std::vector<int>& left, int* steps) {
   const Geom& g = c->gw;
   hipStream_t s = c->stream;
-  const double tol = goal.tol, accept = goal.accept;
+  const double accept = goal.accept;
   const int kmax = series_steps(g, goal.prec);
   if (kmax < 1) return false;
   const SolveCost cost(g, nb, goal.prec, c->vq != nullptr);
   const adga::VqTerm vt{c->W, c->opgd, c->vqQ};
   const adga::VqTerm* vtp = c->vq ? &vt : nullptr;
   std::vector<double> rho(2 * nb, 0.0), prev;
-  std::vector<int> need(2 * nb);
+  std::vector<int> need(2 * nb), slow_need(2 * nb);  // steps to the aim, to the tolerance
   int done = 0;  // residuals of the present batch
   // the residuals of the first k points after `mode`, `count` - 1 more steps, and each matrix's rho and need
-  // (0: converged, or not falling; kmax + 1: not contracting)
+  // (0: converged, or not falling; above kmax: not contracting)
   auto advance = [&](int k, adga::ResidMode mode, int count) {
     const bool start = mode == adga::RESID_START;
     if (start) done = 0;
@@ -486,16 +486,21 @@ bool series_solve(adga_ctx* c, int nb, const SeriesGoal& goal, const z64* B, z64
     for (int m = 0; m < 2 * k; ++m) {
       const double r = relh[m], fell = start ? r : std::pow(r / prev[m], 1.0 / count);
       if (start) rho[m] = fell;
-      need[m] = 0;
-      if (r <= tol) continue;
+      need[m] = slow_need[m] = 0;
+      const double aim = goal.aim(rho[m]);
+      if (r <= aim) continue;
       if (!start && r <= 8 * SERIES_ACCEPT64 && !(fell < 0.5)) continue;  // at round-off
       rho[m] = std::max(rho[m], fell);
-      const double n = rho[m] < 1.0 && std::isfinite(r) ? std::ceil(std::log(tol / r) / std::log(rho[m])) : INFINITY;
-      need[m] = (int)std::min(n, (double)kmax + 1);
+      auto steps_to = [&](double goal_r) {
+        const double n = rho[m] < 1.0 && std::isfinite(r) ? std::ceil(std::log(goal_r / r) / std::log(rho[m])) : INFINITY;
+        return (int)std::min(std::max(n, 0.0), 2.0 * kmax + 1);
+      };
+      need[m] = steps_to(aim);
+      slow_need[m] = steps_to(goal.tol);
     }
   };
-  // over kmax more steps, or over twice as many in all: a prediction that keeps growing
-  auto is_slow = [&](int m) { return need[m] > kmax || done + need[m] > 2 * kmax; };
+  // over kmax more steps to the tolerance, or over twice as many in all: a prediction that keeps growing
+  auto is_slow = [&](int m) { return slow_need[m] > kmax || done + slow_need[m] > 2 * kmax; };
   auto slow = [&](int k) {  // points among the first k
     int n = 0;
     for (int b = 0; b < k; ++b) n += is_slow(2 * b) || is_slow(2 * b + 1);

@@ -59,3 +59,20 @@ def test_gpu_series_leaves_the_smallest_refined_systems_to_the_lu():
     wl = _workload(1, (8, 8, 8), 20, 0.01)
     assert _run(wl, 512, "refined")[1]["n_lu_launches"] == 1
     assert _run(wl, 512, "fp64")[1]["n_lu_launches"] == 0
+
+
+@pytest.mark.parametrize("n,nk,iwf,npts,noise", [(1, (4, 4, 4), 200, 64, 0.4), (1, (4, 4, 4), 200, 64, 0.5),
+                                                 (3, (4, 4, 3), 30, 41, 0.4), (3, (4, 4, 4), 60, 16, 0.5)])
+def test_gpu_series_refined_accuracy_at_slow_contraction(n, nk, iwf, npts, noise):
+    """At a contraction rho of 0.3 to 0.5 a step the error after the last step is r rho / (1 - rho), which stays within
+    a tenth of the tolerance (1.5 for the estimate of rho from the number of products), and chi within that of the
+    FP64 LU's."""
+    wl = _workload(n, nk, iwf, noise)
+    r, st = _run(wl, npts, "refined")
+    assert st["n_lu_launches"] == 0 and st["n_fp64_resolved"] == 0
+    res = st["refine_resid"]
+    rho = res ** (1.0 / st["n_gemm_dominant"])
+    assert res * rho / (1 - rho) < 1.5e-13, (res, rho)
+    ref = _run(wl, npts, "fp64", series=0)[0]
+    for k in ("chi_d", "chi_m"):
+        assert np.abs(r[k] - ref[k]).max() < 1e-13 * np.abs(ref[k]).max()
