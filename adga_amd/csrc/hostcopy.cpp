@@ -3,7 +3,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
-#include <system_error>
+#include <exception>
 #include <thread>
 
 namespace adga_host {
@@ -66,8 +66,9 @@ hipError_t HostCopy::to_host(void* dst, const void* src, size_t bytes, hipStream
   int started = 0;
   try {
     for (; started < THREADS; ++started) pool[started] = std::thread(work, started);
-  } catch (const std::system_error&) {
-    // no more threads: this one does the rest of the shares
+  } catch (const std::exception&) {
+    // no more threads (std::system_error) or no memory for one (std::bad_alloc; past here it would end the process,
+    // with threads not joined): this one does the rest of the shares
   }
   for (int t = started; t < THREADS; ++t) work(t);
   for (int t = 0; t < started; ++t) pool[t].join();
