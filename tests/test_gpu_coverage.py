@@ -1,0 +1,56 @@
+"""The residual product's 64 x 64 tiles, which need more points than the smallest workloads."""
+import numpy as np
+import pytest
+
+from conftest import rel_err
+from adga_amd import synth
+from test_gpu_series import _workload
+
+pytestmark = pytest.mark.gpu
+
+
+def _tiles(rows, cols, channels):
+    """64 x 64 tiles of a residual product; from 2048 on they are taken, below 32 x 32 ones"""
+    return channels * -(-rows // 64) * -(-cols // 64)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "refined"])
+def test_gpu_large_tiles_equal_lu(precision):
+    """N = 666, 720 points: 64 x 64 tiles with remainders of 26 rows, 16 columns and 10 in K, against the LU (the
+    bounds of the smaller shapes' test: 1e-12 in FP64, 1e-10 refined)."""
+    from adga_amd import api
+    wl = _workload(3, (9, 9, 9), 37, 1e-3)
+    assert wl.maxdim == 666 and _tiles(666, 720 * 9, 2) >= 2048
+    inp = synth.build_inputs(wl)
+    x = [synth.chi_loc(inp, 1, c) for c in ("dens", "magn")]
+    res = []
+    for series in (1, 0):
+        print(f"64 x 64 tiles {precision} series={series}", flush=True)
+        with api.Context(inp, series=series, batch=720) as ctx:
+            ctx.set_local_omega(1, *x)
+            r = ctx.run_points(np.arange(1, 721, dtype=np.int32), precision)
+            assert (r["status"] == 0).all() and ctx.stats()["n_lu_launches"] == 1 - series
+            res.append([r["chi_d"], r["chi_m"], ctx.get_sigma()[0]])
+    for a, b in zip(*res):
+        assert rel_err(a, b) < (1e-12 if precision == "fp64" else 1e-10)
+
+
+def test_gpu_large_tiles_equal_small_tiles():
+    """1700 points of N = 1080 at once and in batches of 100: every product of the batch, gamma^q's upper half of the
+    rows included, on 64 x 64 and on 32 x 32 tiles.  Equal but for the rounding of sums in another order: 1e-12."""
+    from adga_amd import api
+    assert _tiles(540, 1700 * 9, 1) >= 2048 and _tiles(1080, 100 * 9, 2) < 2048
+    wl = _workload(3, (12, 12, 12), 60, 1e-3)
+    inp = synth.build_inputs(wl)
+    x = [synth.chi_loc(inp, 1, c) for c in ("dens", "magn")]
+    iq = np.arange(1, 1701, dtype=np.int32)
+    res = []
+    for batch in (1700, 100):
+        print(f"1700 points in batches of {batch}", flush=True)
+        with api.Context(inp, batch=batch) as ctx:
+            ctx.set_local_omega(1, *x)
+            r = ctx.run_points(iq, "fp64")
+            assert (r["status"] == 0).all() and ctx.stats()["n_lu_launches"] == 0
+            res.append([r["chi_d"], r["chi_m"], ctx.get_sigma()[0]])
+    for a, b in zip(*res):
+        assert rel_err(a, b) < 1e-12
