@@ -1,4 +1,5 @@
-"""The residual product's 64 x 64 tiles, which need more points than the smallest workloads."""
+"""The residual product's 64 x 64 tiles and downloads of several chunks per host thread, which need more than the smallest
+workloads."""
 import numpy as np
 import pytest
 
@@ -54,3 +55,23 @@ def test_gpu_large_tiles_equal_small_tiles():
             res.append([r["chi_d"], r["chi_m"], ctx.get_sigma()[0]])
     for a, b in zip(*res):
         assert rel_err(a, b) < 1e-12
+
+
+@pytest.mark.parametrize("nk,iwf", [((16, 16, 17), 32), ((17, 19, 23), 64)], ids=["17.8MB", "60.9MB"])
+def test_gpu_download_in_many_chunks(nk, iwf):
+    """Self-energies of 8.5 and 29 chunks of 2 MB for the eight host threads: a partial last chunk, an uneven split, and
+    slots used again; equal on a second read, and their k sum is the context's own."""
+    from adga_amd import api
+    inp = synth.build_inputs(_workload(2, nk, iwf, 1e-3))
+    print(f"download {nk}", flush=True)
+    with api.Context(inp) as ctx:
+        ctx.set_local_omega(1, *[synth.chi_loc(inp, 1, c) for c in ("dens", "magn")])
+        ctx.run_points(np.array([1, 6, 78], dtype=np.int32), "fp64")
+        a = ctx.get_sigma()[0]
+        b = ctx.get_sigma()[0]
+        loc = ctx.get_sigma_g_loc()[0]
+    assert a.nbytes > 16 << 20 and a.nbytes % (2 << 20) != 0 and np.array_equal(a, b)
+    mean = a.mean(axis=3)
+    for i in range(2):
+        mean[i, i] += inp.siw[inp.iwmax - iwf:inp.iwmax + iwf, i]
+    assert rel_err(loc, mean) < 1e-13
