@@ -1,5 +1,5 @@
-"""The residual product's 64 x 64 tiles and downloads of several chunks per host thread, which need more than the smallest
-workloads."""
+"""Shapes that need more than the smallest workloads: the residual product's 64 x 64 tiles, downloads of several chunks
+per host thread and several one-particle frequencies per workgroup."""
 import numpy as np
 import pytest
 
@@ -75,3 +75,23 @@ def test_gpu_download_in_many_chunks(nk, iwf):
     for i in range(2):
         mean[i, i] += inp.siw[inp.iwmax - iwf:inp.iwmax + iwf, i]
     assert rel_err(loc, mean) < 1e-13
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 4])
+@pytest.mark.parametrize("iwmax", [1024, 1025, 1026, 1027])
+def test_gpu_one_particle_sums_of_many_frequencies(n, iwmax):
+    """get_giw with four frequencies to a workgroup (n <= 3, from 1024 on) and get_sigma_g_loc with two outside the
+    box, last groups of every size, against the oracle: 1e-12 as for the routines' other tests."""
+    import adga_oracle
+    from adga_amd import api
+    nk, iwf = (3, 2, 2), 4
+    wl = synth.Workload("onep", n, nk, iwf, 0, 10.0, 3.0, 0.4, "sc1" if n == 1 else "rand5", t=0.2, seed=n, iwmax=iwmax)
+    inp = synth.build_inputs(wl)
+    rng = np.random.default_rng(iwmax)
+    ss = 0.2 * (rng.normal(size=(n, n, wl.nf, 12)) + 1j * rng.normal(size=(n, n, wl.nf, 12)))
+    print(f"one-particle sums n={n} iwmax={iwmax}", flush=True)
+    with api.Context(inp) as ctx:
+        assert rel_err(ctx.get_giw(), adga_oracle.get_giw(inp)) < 1e-12
+        sl, gl = ctx.get_sigma_g_loc(ss)
+    osl, ogl = adga_oracle.get_sigma_g_loc(inp, ss)
+    assert rel_err(sl, osl) < 1e-12 and rel_err(gl, ogl) < 1e-12
