@@ -1,5 +1,6 @@
-"""Shapes that need more than the smallest workloads: the residual product's 64 x 64 tiles, downloads of several chunks
-per host thread and several one-particle frequencies per workgroup."""
+"""Shapes and branches that need more than the smallest workloads: the residual product's 64 x 64 tiles, downloads of
+several chunks per host thread, several one-particle frequencies per workgroup, and derivatives whose solve does not
+converge by iteration where the forward one does."""
 import numpy as np
 import pytest
 
@@ -95,3 +96,45 @@ def test_gpu_one_particle_sums_of_many_frequencies(n, iwmax):
         sl, gl = ctx.get_sigma_g_loc(ss)
     osl, ogl = adga_oracle.get_sigma_g_loc(inp, ss)
     assert rel_err(sl, osl) < 1e-12 and rel_err(gl, ogl) < 1e-12
+
+
+def test_gpu_derivative_solves_that_need_the_lu():
+    """N = 360 at the iteration's limit: the forward solve and two directions iterate (17 to 19 products each), the third
+    direction's right-hand side does not, and its LU factors are formed after the forward pass; with the directions in
+    the opposite order they are formed for the first and serve all three.  Against the LU throughout: 1e-12."""
+    import dataclasses
+    from adga_amd import api
+    inp = synth.build_inputs(_workload(3, (4, 4, 3), 20, 0.225))
+    tan = synth.tangents(inp)
+    x = [synth.chi_loc(inp, 1, c) for c in ("dens", "magn")]
+    d = synth.dchi_loc(inp, tan, 1)
+    v = np.random.default_rng(3).standard_normal(d.shape[:2] + (1,))
+    d = d + 0.03 * (v + v.transpose(1, 0, 2))
+    iq = np.arange(1, 49, dtype=np.int32)
+    fields = ("dhk", "dsiw", "dgiw", "dmu", "du", "du_tilde")
+    for order in (slice(None), slice(None, None, -1)):
+        t = dataclasses.replace(tan, **{f: np.ascontiguousarray(getattr(tan, f)[..., order]) for f in fields})
+        dx = np.asfortranarray(d[..., order])
+        out, products = [], []
+        for series in (1, 0):
+            print(f"derivatives at the limit, series={series} order {order}", flush=True)
+            with api.Context(inp, batch=48, series=series) as ctx:
+                ctx.set_tangents(t)
+                ctx.set_local_omega(1, *x)
+                ctx.set_local_omega_tangent(dx, dx)
+                ctx.run_points(iq, "fp64")
+                products.append(ctx.stats()["n_gemm_dominant"])
+                ctx.reset_sigma()
+                r = ctx.run_points_tangent(iq)
+                st = ctx.stats()
+                products.append(st["n_gemm_dominant"])
+                assert (r["status"] == 0).all() and st["n_lu_launches"] == 1 - series
+                out.append((r["chi_d"], r["dchi_d"], r["dchi_m"], ctx.get_sigma()[0], ctx.get_sigma_tangent()))
+        forward, total = products[:2]
+        each = forward - 4
+        if order == slice(None):
+            assert forward + each <= total < forward + 3 * each, (forward, total)
+        else:
+            assert total < forward + each, (forward, total)
+        for a, b in zip(*out):
+            assert rel_err(a, b) < 1e-12
