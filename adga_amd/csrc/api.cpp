@@ -495,7 +495,7 @@ bool series_solve(adga_ctx* c, int nb, const SeriesGoal& goal, const z64* B, z64
         const double n = rho[m] < 1.0 && std::isfinite(r) ? std::ceil(std::log(goal_r / r) / std::log(rho[m])) : INFINITY;
         return (int)std::min(std::max(n, 0.0), 2.0 * kmax + 1);
       };
-      need[m] = steps_to(aim);
+      need[m] = r <= goal.tol ? std::min(4, steps_to(aim)) : steps_to(aim);  // rho may be too large: looked at again
       slow_need[m] = steps_to(goal.tol);
     }
   };
