@@ -446,17 +446,17 @@ namespace adga_host {
 // the norm that stops it is the residual itself.  It converges where T contracts (the BSE far from an
 // instability).
 //
-// The rule: the residuals' ratio gives each matrix's contraction rho (the first one, |T B| / |B|, and the
-// later |r'| / |r| where those are worse), hence the steps ln(aim / r) / ln(rho) it still needs; a point that
-// needs over series_steps() more of them is slow.  What counts is what is still to do, not what is done: a point
-// that needs a few steps more than foreseen gets them, where the LU would cost many.  The LU is taken (false, Y
-// undefined) as soon as the other points' steps and the single LUs of the slow ones cost more than it does
-// (41 points of N = 540: a step 0.04 ms, the complex64 LU of the batch 3.6, the complex128 LU of one
-// point 3.8), or one point in eight is slow, or one is and `singles` is not allowed - for a batch of expensive products from three
-// of them on its first 8 points, so that a batch that does not contract costs next to nothing, and for the others
-// from the first one or two.  The steps predicted are queued together: a few waits per batch.  They go on to
-// the goal's aim, or until the residual stops falling; a matrix whose residual then is above `accept`
-// puts its point into `left` (none without `singles`).  `steps`: those taken.
+// The rule: the residuals' ratio gives each matrix's contraction rho (the first one, |T B| / |B|, and the later
+// |r'| / |r| where those are worse), hence the steps ln(aim / r) / ln(rho) it still needs; a point that needs over
+// series_steps() more of them is slow.  What counts is what is still to do, not what is done: a point that needs a
+// few steps more than foreseen gets them, where the LU would cost many.  The LU is taken (false, Y undefined) as
+// soon as the other points' steps and the single LUs of the slow ones cost more than it does (41 points of N =
+// 540: a step 0.04 ms, the complex64 LU of the batch 3.6, the complex128 LU of one point 3.8), or one point in
+// eight is slow, or one is and `singles` is not allowed - for a batch of expensive products from three of them on
+// 8 of its points, so that a batch that does not contract costs next to nothing, and for the others from the first
+// one or two.  The steps predicted are queued together: a few waits per batch.  They go on to the goal's aim, or
+// until the residual stops falling; a matrix whose residual then is above `accept` puts its point into `left`
+// (none without `singles`).  `steps`: those taken.
 bool series_solve(adga_ctx* c, int nb, const SeriesGoal& goal, const z64* B, z64* Y, std::vector<double>& relh,
                   std::vector<int>& left, int* steps) {
   const Geom& g = c->gw;
@@ -470,14 +470,20 @@ bool series_solve(adga_ctx* c, int nb, const SeriesGoal& goal, const z64* B, z64
   std::vector<double> rho(2 * nb, 0.0), prev;
   std::vector<int> need(2 * nb), slow_need(2 * nb);  // steps to the aim, to the tolerance
   int done = 0;  // residuals of the present batch
-  // the residuals of the first k points after `mode`, `count` - 1 more steps, and each matrix's rho and need
+  // the points' systems: the batch's, or copies of a few of them
+  struct Systems {
+    const z64 *S, *B;
+    const adga::VqTerm* vq;
+  };
+  const Systems all{c->S, B, vtp};
+  // the residuals of k points after `mode`, `count` - 1 more steps, and each matrix's rho and need
   // (0: converged, or not falling; above kmax: not contracting)
-  auto advance = [&](int k, adga::ResidMode mode, int count) {
+  auto advance = [&](const Systems& of, int k, adga::ResidMode mode, int count) {
     const bool start = mode == adga::RESID_START;
     if (start) done = 0;
     prev.assign(relh.begin(), relh.begin() + 2 * k);
     for (int j = 0; j < count; ++j)
-      adga::launch_residual(g, k, c->S, c->cd, c->cm, B, Y, c->Z, c->R, c->nrm, s, vtp,
+      adga::launch_residual(g, k, of.S, c->cd, c->cm, of.B, Y, c->Z, c->R, c->nrm, s, of.vq,
                             j == 0 ? mode : adga::RESID_STEP, k == nb && !(start && j == 0) ? &c->lut : nullptr,
                             j + 1 == count);  // only the last one's norms are read
     CK(hipMemcpyAsync(relh.data(), c->nrm.rel, sizeof(double) * 2 * k, hipMemcpyDeviceToHost, s));
@@ -508,16 +514,29 @@ bool series_solve(adga_ctx* c, int nb, const SeriesGoal& goal, const z64* B, z64
   };
   left.clear();
   if (steps) *steps = 0;
-  adga::launch_absmax_rhs(g, nb, B, c->nrm, s);
   // a look at a few points pays where a product on all takes longer than three waits (512 points of N = 40: iterated
   // 0.36 ms, 0.46 with the look; given up for the LU 0.63, 0.61 with the look, 0.56 untried)
   constexpr int LOOK = 8;
   if (nb >= 8 * LOOK && cost.product > 0.1) {
-    advance(LOOK, adga::RESID_START, 1);
-    for (int k = 0; k < 2 && 2 * slow(LOOK) <= LOOK; ++k) advance(LOOK, adga::RESID_STEP, 1);
+    // spread over the batch: a q list begins in a neighbourhood of Gamma.  Their systems are copied behind the first
+    // LOOK solutions of Y, not in use yet.
+    const long blen = 2L * g.N * g.n2, slen = (long)g.nf * g.n4, wlen = (long)g.N * g.n2;
+    z64 *Bs = Y + LOOK * blen, *Ss = Bs + LOOK * blen, *Ws = Ss + LOOK * slen;
+    int sel[LOOK];
+    for (int i = 0; i < LOOK; ++i) sel[i] = (int)((2L * i + 1) * nb / (2 * LOOK));
+    CK(hipMemcpyAsync(c->keep, sel, sizeof sel, hipMemcpyHostToDevice, s));
+    adga::launch_gather(LOOK, blen, c->keep, B, Bs, false, s);
+    adga::launch_gather(LOOK, slen, c->keep, c->S, Ss, false, s);
+    if (c->vq) adga::launch_gather(LOOK, wlen, c->keep, c->W, Ws, false, s);
+    const adga::VqTerm vs{Ws, c->opgd, c->vqQ};
+    const Systems few{Ss, Bs, c->vq ? &vs : nullptr};
+    adga::launch_absmax_rhs(g, LOOK, Bs, c->nrm, s);
+    advance(few, LOOK, adga::RESID_START, 1);
+    for (int k = 0; k < 2 && 2 * slow(LOOK) <= LOOK; ++k) advance(few, LOOK, adga::RESID_STEP, 1);
     if (2 * slow(LOOK) > LOOK) return false;
   }
-  advance(nb, adga::RESID_START, 1);
+  adga::launch_absmax_rhs(g, nb, B, c->nrm, s);
+  advance(all, nb, adga::RESID_START, 1);
   for (;;) {
     const int n = slow(nb);
     int k = 0;
@@ -527,7 +546,7 @@ bool series_solve(adga_ctx* c, int nb, const SeriesGoal& goal, const z64* B, z64
     if (n > 0 && (!goal.singles || 8 * n > nb || k * cost.step + cost.singles(n) > 1.25 * cost.lu)) return false;
     if (k == 0) break;
     if (done == 1 && nb < 8 * LOOK) k = std::min(k, 1);  // a second look at the contraction first
-    advance(nb, adga::RESID_STEP, k);
+    advance(all, nb, adga::RESID_STEP, k);
     if (steps) *steps = done - 1;
   }
   for (int b = 0; b < nb; ++b)

@@ -76,3 +76,20 @@ def test_gpu_series_refined_accuracy_at_slow_contraction(n, nk, iwf, npts, noise
     ref = _run(wl, npts, "fp64", series=0)[0]
     for k in ("chi_d", "chi_m"):
         assert np.abs(r[k] - ref[k]).max() < 1e-13 * np.abs(ref[k]).max()
+
+
+@pytest.mark.parametrize("precision", ["fp64", "refined"])
+def test_gpu_series_looks_at_points_all_over_the_batch(precision):
+    """V(q) strong at the first eight of 500 points of N = 360, as a neighbourhood of Gamma would have it: they are
+    solved by themselves, the rest is iterated."""
+
+    def v_q(inp):
+        inp.v_q[:, :, :8] = 60.0 * np.eye(9)[:, :, None]
+
+    r, st = _run(_workload(3, (8, 8, 8), 20, 1e-3, vq=0.02), 500, precision, change=v_q)
+    assert st["n_lu_launches"] == 0
+    if precision == "refined":
+        assert st["n_fp64_resolved"] == 16
+    ref = _run(_workload(3, (8, 8, 8), 20, 1e-3, vq=0.02), 500, precision, change=v_q, series=0)[0]
+    for k in ("chi_d", "chi_m"):
+        assert np.abs(r[k] - ref[k]).max() < (1e-12 if precision == "fp64" else 1e-10) * np.abs(ref[k]).max()
