@@ -74,11 +74,13 @@ int adga_ctx_create(const adga_dims *dims, const int *q_data, const int *k_data_
  * residual max|r|/max|b| every BSE solve must reach, default 1e-12), "refine_maxit" (default 12;
  * a matrix that has not converged by then, or whose residual a correction did not halve, or whose
  * complex64 LU met a zero pivot, is solved again in complex128 unless "fallback" is 0; its final
- * status then depends only on the complex128 solve), "series" (1, the default: the BSE systems of a batch, eta (1 - T) = B, are solved by the
- * fixed-point iteration eta <- B + eta T in FP64 where T contracts, in the FP64 mode to the round-off of the
- * residual, 1e-15 .. 1e-14, in the refined mode to "refine_tol"; batches that do not contract, or would need
- * more steps than the LU costs, take the LU, and single points that do not converge the complex128 LU; 0: the
- * LU always), "do_eom" (1: the default; 0: no
+ * status then depends only on the complex128 solve; it bounds the complex64 corrections only), "series" (1, the
+ * default: the BSE systems of a batch, eta (1 - T) = B, are solved by the fixed-point iteration eta <- B + eta T
+ * in FP64 where T contracts, in the FP64 mode to the round-off of the residual, 1e-15 .. 1e-14, in the refined
+ * mode to "refine_tol" and an error of a tenth of it; batches that do not contract, or would need more steps than
+ * the LU costs, take the LU, and single points that do not converge the complex128 LU.  A point's steps and its
+ * way then depend on the batch it is in, so that its results agree between batches to the accuracy of the mode,
+ * not to the bit; 0: the LU always, with the same bits in every batch where "bubble" is 0 or 1), "do_eom" (1: the default; 0: no
  * equation of motion, as the reference's do_eom = .false. for a q path),
  * "bubble" (0: direct k sum per point; 1: all q of the current omega at once by
  * k-grid DFT, cached per omega; 2: DFT when a batch has enough points (24 with three or five orbitals on

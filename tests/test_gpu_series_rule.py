@@ -93,3 +93,30 @@ def test_gpu_series_looks_at_points_all_over_the_batch(precision):
     ref = _run(_workload(3, (8, 8, 8), 20, 1e-3, vq=0.02), 500, precision, change=v_q, series=0)[0]
     for k in ("chi_d", "chi_m"):
         assert np.abs(r[k] - ref[k]).max() < (1e-12 if precision == "fp64" else 1e-10) * np.abs(ref[k]).max()
+
+
+@pytest.mark.parametrize("precision", ["fp64", "refined"])
+@pytest.mark.parametrize("noise", [1e-3, 0.03, 0.5])
+def test_gpu_batch_dependence(precision, noise):
+    """The same points in batches of 100, 13 and 1, the bubble formed one way: by the LU each point has the same bits.
+    By the iteration a matrix takes the steps of its batch's slowest, and whether a batch is iterated depends on its
+    points: they agree to the accuracy of each mode (1e-12 in FP64, a refined solve's 1e-11)."""
+    from adga_amd import api
+    inp = synth.build_inputs(_workload(3, (5, 5, 4), 20, noise))
+    x = [synth.chi_loc(inp, 1, c) for c in ("dens", "magn")]
+    for series in (0, 1):
+        ref = None
+        for batch in (100, 13, 1):
+            print(f"batches of {batch} noise={noise} {precision} series={series}", flush=True)
+            with api.Context(inp, batch=batch, bubble=0, series=series) as ctx:
+                ctx.set_local_omega(1, *x)
+                r = ctx.run_points(np.arange(1, 101, dtype=np.int32), precision)
+                out = [r["chi_d"], r["chi_m"], ctx.get_sigma()[0]]
+            assert (r["status"] == 0).all()
+            ref = ref or out
+            for a, b in zip(out, ref):
+                if series == 0:
+                    assert np.array_equal(a, b)
+                else:
+                    err = np.abs(a - b).max() / np.abs(b).max()
+                    assert err < (1e-12 if precision == "fp64" else 1e-11)
