@@ -24,7 +24,7 @@ void alloc_norm(adga::ResidNorm& n, size_t nmat) {
 void free_batch(adga_ctx* c) {
   dfree(c->chi0q); dfree(c->S); dfree(c->gamq); dfree(c->Bp); dfree(c->Y); dfree(c->Z); dfree(c->R);
   dfree(c->mt); dfree(c->chi_out); dfree(c->bub_out); free_norm(c->nrm);
-  dfree(c->qidx); dfree(c->keep);
+  dfree(c->qidx); dfree(c->keep); dfree(c->look);
   c->cap = 0;
 }
 
@@ -60,6 +60,7 @@ void ensure_batch(adga_ctx* c, int nb) {
   alloc_norm(c->nrm, 2 * nb);
   dalloc(&c->qidx, nb);
   dalloc(&c->keep, nb);
+  dalloc(&c->look, SERIES_LOOK);
   c->cap = nb;
 }
 
@@ -498,7 +499,8 @@ bool series_solve(adga_ctx* c, int nb, const SeriesGoal& goal, const z64* B, z64
       if (!start && r <= 8 * SERIES_ACCEPT64 && !(fell < 0.5)) continue;  // at round-off
       rho[m] = std::max(rho[m], fell);
       auto steps_to = [&](double goal_r) {
-        const double n = rho[m] < 1.0 && std::isfinite(r) ? std::ceil(std::log(goal_r / r) / std::log(rho[m])) : INFINITY;
+        const bool falls = rho[m] < 1.0 && std::isfinite(r);
+        const double n = falls ? std::ceil(std::log(goal_r / r) / std::log(rho[m])) : INFINITY;
         return (int)std::min(std::max(n, 0.0), 2.0 * kmax + 1);
       };
       need[m] = r <= goal.tol ? std::min(4, steps_to(aim)) : steps_to(aim);  // rho may be too large: looked at again
@@ -516,7 +518,7 @@ bool series_solve(adga_ctx* c, int nb, const SeriesGoal& goal, const z64* B, z64
   if (steps) *steps = 0;
   // a look at a few points pays where a product on all takes longer than three waits (512 points of N = 40: iterated
   // 0.36 ms, 0.46 with the look; given up for the LU 0.63, 0.61 with the look, 0.56 untried)
-  constexpr int LOOK = 8;
+  constexpr int LOOK = SERIES_LOOK;
   if (nb >= 8 * LOOK && cost.product > 0.1) {
     // spread over the batch: a q list begins in a neighbourhood of Gamma.  Their systems are copied behind the first
     // LOOK solutions of Y, not in use yet.
@@ -524,10 +526,10 @@ bool series_solve(adga_ctx* c, int nb, const SeriesGoal& goal, const z64* B, z64
     z64 *Bs = Y + LOOK * blen, *Ss = Bs + LOOK * blen, *Ws = Ss + LOOK * slen;
     int sel[LOOK];
     for (int i = 0; i < LOOK; ++i) sel[i] = (int)((2L * i + 1) * nb / (2 * LOOK));
-    CK(hipMemcpyAsync(c->keep, sel, sizeof sel, hipMemcpyHostToDevice, s));
-    adga::launch_gather(LOOK, blen, c->keep, B, Bs, false, s);
-    adga::launch_gather(LOOK, slen, c->keep, c->S, Ss, false, s);
-    if (c->vq) adga::launch_gather(LOOK, wlen, c->keep, c->W, Ws, false, s);
+    CK(hipMemcpyAsync(c->look, sel, sizeof sel, hipMemcpyHostToDevice, s));
+    adga::launch_gather(LOOK, blen, c->look, B, Bs, false, s);
+    adga::launch_gather(LOOK, slen, c->look, c->S, Ss, false, s);
+    if (c->vq) adga::launch_gather(LOOK, wlen, c->look, c->W, Ws, false, s);
     const adga::VqTerm vs{Ws, c->opgd, c->vqQ};
     const Systems few{Ss, Bs, c->vq ? &vs : nullptr};
     adga::launch_absmax_rhs(g, LOOK, Bs, c->nrm, s);

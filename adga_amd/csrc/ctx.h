@@ -82,7 +82,7 @@ struct adga_ctx {
   z64 *chi0q = nullptr, *S = nullptr, *gamq = nullptr, *Bp = nullptr, *Y = nullptr, *Z = nullptr, *R = nullptr,
       *mt = nullptr, *chi_out = nullptr, *bub_out = nullptr;
   adga::ResidNorm nrm{};  // residual norms of the batch's matrices
-  int* qidx = nullptr;
+  int *qidx = nullptr, *look = nullptr;  // q index of each point; points of the iteration's first look
   // LU workspace, allocated by the first batch that factors (lu_cap points)
   int lu_cap = 0;
   void* M = nullptr;
@@ -98,7 +98,7 @@ struct adga_ctx {
   // accumulated self-energies
   z64 *sig_nl = nullptr, *sig_dmft = nullptr, *sig_hf = nullptr;
   // k-grid convolutions: twiddles, Ghat table, per-omega bubble cache, pending EOM of one omega
-  int bubble_mode = 2;  // 0 direct, 1 DFT, 2 DFT when the batch has >= 64 points or the cache is valid
+  int bubble_mode = 2;  // 0 direct, 1 DFT, 2 DFT when the batch has bubble_dft_points() or the cache is valid
   int eom_mode = 1;     // 0 direct, 1 DFT (accumulated per omega, flushed on omega change / get_sigma)
   bool do_eom = true;   // option "do_eom": the reference's do_eom (off for a q path, main.F90:341-347)
   z64 *tw = nullptr, *ghat = nullptr, *bub_p = nullptr, *bub_all = nullptr, *macc = nullptr, *mwork = nullptr;
@@ -260,6 +260,7 @@ void tangent_batch(adga_ctx* c, int nb, int p0, int npts, const std::vector<int>
                    const TangentOut& out, bool factored);
 // the FP64 mode's relative residual: the aim, and what a residual at its round-off may be
 constexpr double SERIES_TOL64 = 1e-15, SERIES_ACCEPT64 = 1e-14;
+constexpr int SERIES_LOOK = 8;  // points of the first look at a batch
 // of the fixed-point iteration: the LU it competes with (0 complex128, 1 complex64 and refinement), the relative
 // residual it aims at and the one it may end with, and whether single points may be left to an LU of their own
 struct SeriesGoal {
