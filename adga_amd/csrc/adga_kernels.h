@@ -145,7 +145,8 @@ bool launch_gkiw(const Geom& g, int k, int iw, const z64* hk, const z64* siw, co
 void launch_chi_qw(const Geom& g, const z64* X, const z64* Y, z64* chi, hipStream_t s);
 void launch_ndmft(const Geom& g, const z64* giw, z64* nd, hipStream_t s);
 void launch_add_siw(const Geom& g, int nk, const z64* siw, z64* ss, hipStream_t s);
-// m_tot at the rows eom_row0 .. N - 1; with vq non-null: V(q_b) = vq + qpos[b] n4 enters the density eta term and -V gamma^w_d / (beta nqp) is added
+// m_tot at the rows eom_row0 .. N - 1; with vq non-null: V(q_b) = vq + qpos[b] n4 enters the density eta term and
+// -V gamma^w_d / (beta nqp) is added
 void launch_mtot(const Geom& g, int npts, const z64* u, const z64* ut, const z64* eta, const z64* gamq, z64* mt,
                  hipStream_t s, const int* qpos = nullptr, const z64* vq = nullptr, const z64* gamd = nullptr,
                  bool accumulate = false);

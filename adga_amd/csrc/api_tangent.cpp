@@ -1,9 +1,10 @@
 // Derivatives of the hot path along caller-given directions of its inputs (the tangent-linear form of
 // bubble -> BSE -> chi / Sigma): the C-ABI entry points adga_set_tangents, adga_set_local_omega_tangent,
 // adga_run_points_tangent (api.cpp) and adga_get_sigma_tangent, and the per-batch work they share.  The
-// derivative of a batch reuses the batch's forward data (S, C, gamma, eta, m_tot and the complex128 LU
-// factors): each direction costs two bubble passes (product rule: the bubble is formed again, not
-// stored), a right-hand side and a solve with the existing factors, chi's contraction and two EOM passes.
+// derivative of a batch reuses the batch's forward data (S, C, gamma, eta, m_tot and, where the forward solve
+// was an LU, its complex128 factors): each direction costs two bubble passes (product rule: the bubble is
+// formed again, not stored), a right-hand side and its solve, by iteration where the forward one iterated and
+// with the factors elsewhere, chi's contraction and two EOM passes.
 #include <cstring>
 #include <numeric>
 
@@ -106,7 +107,8 @@ void tangent_batch(adga_ctx* c, int nb, int p0, int npts, const std::vector<int>
     if (!factored) {
       relh.assign(nmat, 0.0);
       infoh.assign(nmat, 0);
-      const bool iterated = c->series && series_solve(c, nb, {0, SERIES_TOL64, SERIES_ACCEPT64, false}, c->t_B, c->t_dY, relh, left);
+      const SeriesGoal goal{0, SERIES_TOL64, SERIES_ACCEPT64, false};
+      const bool iterated = c->series && series_solve(c, nb, goal, c->t_B, c->t_dY, relh, left);
       if (!iterated && ensure_lu(c, nb)) {
         if (!factor_fp64(c, nb)) throw HipError{hipErrorInvalidValue, "tangent solve: BSE size outside the LU's range"};
         factored = true;

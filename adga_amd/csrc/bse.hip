@@ -6,11 +6,13 @@
 // C = chi0^w F_r, inverts it, and forms eta = (1+gamma^w)(A^-1 - 1).  Here the
 // same eta is obtained without an explicit inverse and without the cancellation
 // in A^-1 - 1: eta A = (1+gamma^w)(1 - A) = (1+gamma^w) blockdiag(S) C is solved
-// as A^T eta^T = B by LU with partial pivoting of M = A^T, with the n^2
-// right-hand sides appended as extra columns of M so the forward elimination
-// happens inside the factorisation.  B and every residual are formed in FP64
-// from the unrounded S and C, so the residual is on the scale of eta itself.
-// M is stored row-major per matrix (row r, column c at r*ldm + c).
+// as M Y = B with M = A^T, Y = eta^T: by fixed-point iteration on the residual
+// products below where 1 - M contracts (M is then never formed), else by LU with
+// partial pivoting of M, stored row-major per matrix (row r, column c at
+// r*ldm + c); the n^2 right-hand sides are extra columns of M where they do not
+// fit the solve's LDS at once, so that their forward elimination happens inside
+// the factorisation.  B and every residual are formed in FP64 from the unrounded
+// S and C, so the residual is on the scale of eta itself.
 #include <type_traits>
 
 #include "adga_kernels.h"
@@ -613,11 +615,13 @@ k_resid_gemm(Geom g, int npts, int ch0, int nch, const z64* __restrict__ cd, con
   }
 }
 
-// Out = C_ch^T Z_ch (+ B - Y when B is given, + Out itself when accumulate), rows r0 .. N - 1.  64 x 64 tiles from four rounds
-// of the chip's 512 such workgroups on; below, 32 x 32 tiles lose less to the last round and to few
-// workgroups (64 x 64 against 32 x 32, columns of both channels: N = 1080, 27000 columns 3.37 / 3.64 ms;
-// N = 4000, 2400 columns 3.89 / 4.25; below the line, timed before the staging moved between the MFMAs:
-// N = 2000, 3200 columns 1.44 / 1.39; N = 540, 738 columns 89 / 50 us; N = 40, 1024 columns 15 / 8).
+// Out = C_ch^T Z_ch (+ B - Y when B is given, + Out itself when accumulate), rows r0 .. N - 1.  64 x 64 tiles from
+// four rounds of the chip's 512 such workgroups on; below, 32 x 32 tiles lose less to the last round and to few
+// workgroups.  64 x 64 against 32 x 32, us, columns of both channels: N = 400, 1024 columns (112 tiles of 64 x 64)
+// 61 / 35; N = 136, 2408 (114) 34 / 20; N = 540, 9000 (1278) 353 / 312; N = 720, 9000 (1704) 591 / 549; N = 2000, 4500
+// (2304) 1899 / 1917; N = 4000, 2400 (2394) 3713 / 4227; N = 960, 12800 (3000) 1166 / 1289.  Between 1200 and 2048
+// tiles either wins with how full the last round is: N = 960, 6400 (1500) 589 / 649; N = 2000, 3200 (1600) 1396 / 1355;
+// N = 1080, 7200 (1938) 869 / 930.
 void resid_gemm(const Geom& g, int npts, int ch0, int nch, const z64* cd, const z64* cm, const z64* Z, z64* Out,
                 const z64* B, const z64* Y, hipStream_t s, bool accumulate, unsigned long long* rmax, int r0,
                 bool update) {

@@ -163,9 +163,9 @@ bool launch_dchi_mm(const Geom& g, int npts, const z64* chi0q, const z64* dchi0q
                    dchi_out, dbub_out, s);
 }
 
-// The same for n <= 2, whose n2 values fill little of a matrix fragment, with one workgroup per point: thread (k slice, channel, row s) accumulates row s of
-// chi_ch over its slice of x = d*n2 + i3 (the n2 values of chi0^q at one x are read by every thread of the
-// slice), the slices are summed through LDS, and threads 0 .. n4-1 form bubble_nl (summed over d in order).
+// The same for n <= 2, whose n2 values fill little of a matrix fragment, with one workgroup per point: thread (k
+// slice, channel, row s) accumulates row s of chi_ch over its slice of x = d*n2 + i3 (the n2 values of chi0^q at one
+// x are read by every thread of the slice), the slices are summed through LDS, and threads 0 .. n4-1 form bubble_nl (summed over d in order).
 template <int N2>
 __global__ void __launch_bounds__(256) k_chi_wg(Geom g, const z64* __restrict__ chi0q, const z64* __restrict__ chi0w,
                                                 const z64* __restrict__ gam_d, const z64* __restrict__ gam_m,

@@ -52,7 +52,8 @@ __device__ __forceinline__ int min_row(unsigned long long mask, int row) {
 }
 
 // The w <= GJ_W columns from c0 on, given as the columns of Pn and left as the columns of G, and the multipliers of
-// step j as column j of F (n values each, so that consecutive lanes take consecutive rows), in the registers of one workgroup, thread t holding rows t + i NT.  One
+// step j as column j of F (n values each, so that consecutive lanes take consecutive rows), in the registers of one
+// workgroup, thread t holding rows t + i NT.  One
 // barrier per column: each wave publishes its best candidate with the row's values.  The column of step j is always
 // register 0: each step writes the updated column c to register c - 1 and the finished one to the last, so that
 // GJ_W steps leave them in order and one loop body serves all (unrolled, the body's 16 copies ran at the rate of
@@ -425,7 +426,7 @@ z64* launch_gj_inverse(int n, z64* A, z64* B, z64* C, z64* G, int* piv, int* pos
     return B;
   }
   z64 *Pn = G + (size_t)n * GJ_W, *F = Pn + (size_t)n * GJ_W, *src = A;
-  unsigned long long* rmax = reinterpret_cast<unsigned long long*>(F + (size_t)n * GJ_W);
+  auto* rmax = reinterpret_cast<unsigned long long*>(F + (size_t)n * GJ_W);
   const int nt = (n + 31) / 32;
   hipLaunchKernelGGL(k_gj_first, dim3((n * GJ_W + 255) / 256), dim3(256), 0, s, n, std::min(GJ_W, n), A, Pn, rmax);
   for (int c0 = 0; c0 < n; c0 += GJ_W) {

@@ -7,8 +7,9 @@
 //   EOM     s(k) = sum_q f(q) g(k - q)    f = m_tot(q)_{...},  g = G(., nu - omega)_jk'
 //                = 1/nkp sum_R F(R) G(R) e^{+ikR}
 // with the forward transform X(R) = sum_k x(k) e^{-ikR}, e^{-ikR} = prod_axes e^{-2 pi i k_a R_a / n_a}.
-// The transform is applied one axis at a time (a 3D DFT is three batched products with the
-// n_a x n_a twiddle matrix); each pass is bound by HBM streaming of the batch of fields.
+// The transform is separable: one axis after the other, a whole field's three axes in LDS where it fits
+// (k_dft3_lds), elsewhere one pass over HBM per axis (a batched product with the n_a x n_a twiddle matrix),
+// bound by streaming the batch of fields.
 // A field is one contiguous grid (kz fastest, like k_index_3, kq_tools.f90:119-125).
 #include <algorithm>
 

@@ -85,8 +85,9 @@ int adga_ctx_create(const adga_dims *dims, const int *q_data, const int *k_data_
  * "bubble" (0: direct k sum per point; 1: all q of the current omega at once by
  * k-grid DFT, cached per omega; 2: DFT when a batch has enough points (24 with three or five orbitals on
  * a grid whose axes have at most 24 points and whose padded field fits the LDS, nkpx nkpy (nkpz | 1) <= 10240;
- * 64 otherwise) or the cache is valid, and the tables of every q fit the memory, the default), "eom" (0: direct sum per batch; 1: m_tot accumulated on the q grid and convolved with
- * G by k-grid DFT when omega changes or the self-energy is read, the default), "lu_streams" (1: each
+ * 64 otherwise) or the cache is valid, and the tables of every q fit the memory, the default), "eom" (0: direct
+ * sum per batch; 1: m_tot accumulated on the q grid and convolved with G by k-grid DFT when omega changes or the
+ * self-energy is read, the default), "lu_streams" (1: each
  * batch's LU on one stream; 2 .. 4: the batch split into that many parts on as many streams, each one
  * operation behind the previous, the large Schur updates on the whole batch; 0, the default: chosen per
  * device and batch shape (precision, BSE size, matrices in the batch): the shape's first three
@@ -326,7 +327,8 @@ int adga_get_ndga(adga_ctx *ctx, const double *sigma_sum, double *n_dga_k, doubl
 
 /*
  * Statistics of the last adga_run_points call (nout <= 16 values): out[0] = max refinement
- * iterations (complex64 corrections, or the fixed-point iteration's steps beyond its first), out[1] = max final relative residual of the points that succeeded, out[2..8] =
+ * iterations (complex64 corrections, or the fixed-point iteration's steps beyond its first), out[1] = max final
+ * relative residual of the points that succeeded (the iteration takes one more step after it), out[2..8] =
  * milliseconds spent in the reference's stage buckets Local, Chi0, Gammas, Inversion, Eta rest, EOM,
  * Chi (src/main.F90:484-783), out[9] = milliseconds of the batched LU factorisations, out[10] =
  * their number (0 where no batch was factored), out[11..13] = milliseconds, algorithmic flops and launches
