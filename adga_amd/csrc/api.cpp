@@ -253,14 +253,11 @@ bool bubble_by_dft(const adga_ctx* c, int nb, bool hit) {
 }  // namespace adga_host
 
 namespace {
-// Steps of the fixed-point iteration (series_solve) that cost no more than the LU of the same batch, in complex128
-// (prec 0) or in complex64 with its refinement (1).  Measured, in steps, the LU costs (N = 40, 512 points) 10 / 3,
+// Steps of the fixed-point iteration (series_solve) that cost no more than the LU of the same batch.  Measured, in
+// steps, the LU costs in complex128 / in complex64 with its refinement (N = 40, 512 points) 10 / 3,
 // (136, 301) 40 / 22, (200, 512) 75 / 37, (540, 41) 100 / 75, (540, 500) 50 / 30, (960, 200) 48 / 40, (1080, 500)
-// 75 / 42, (2000, 64) 50 / 33, (4000, 16) 110 / 60.  None for the smallest in the refined mode: 512 points of N = 40
-// take 0.41 to 0.44 ms by the iteration, 0.43 by the LU and 0.48 by the LU after a look at the contraction.
-int series_steps(const Geom& g, int prec) {
-  return prec == 1 && g.N < 80 ? 0 : std::min(8 + g.N / (4 * g.n2), 2 + g.N / 8);
-}
+// 75 / 42, (2000, 64) 50 / 33, (4000, 16) 110 / 60.
+int series_steps(const Geom& g) { return std::min(8 + g.N / (4 * g.n2), 2 + g.N / 8); }
 
 // Milliseconds of a step, of the LU of the batch and of the complex128 LU of a few of its points (solve_fp64), within
 // some 20%: a latency of N times 4.75 us (N = 136) to 10 us (N >= 1080), the flops at the LU's rate.
@@ -463,8 +460,7 @@ bool series_solve(adga_ctx* c, int nb, const SeriesGoal& goal, const z64* B, z64
   const Geom& g = c->gw;
   hipStream_t s = c->stream;
   const double accept = goal.accept;
-  const int kmax = series_steps(g, goal.prec);
-  if (kmax < 1) return false;
+  const int kmax = series_steps(g);
   const SolveCost cost(g, nb, goal.prec, c->vq != nullptr);
   const adga::VqTerm vt{c->W, c->opgd, c->vqQ};
   const adga::VqTerm* vtp = c->vq ? &vt : nullptr;

@@ -59,8 +59,8 @@ __device__ __forceinline__ int min_row(unsigned long long mask, int row) {
 // GJ_W steps leave them in order and one loop body serves all (unrolled, the body's 16 copies ran at the rate of
 // instruction misses: 126 us per panel at n = 1080).  pos[r]: the column row r was the pivot of, -1 before.
 //
-// Bound by FP64 issue on one CU and the latency of barrier, search and reciprocal: 46 us per panel at n = 1080
-// (62 us with A and G row-major and the pivot row read from LDS by every thread).
+// Bound by FP64 issue on one CU and the latency of barrier, search and reciprocal: 49 us per panel at n = 1080, 3 of
+// them for F (62 us with A and G row-major and the pivot row read from LDS by every thread).
 template <int RPT, int NT>
 __global__ void __launch_bounds__(NT) k_gj_panel(int n, int c0, int w, const z64* __restrict__ Pn,
                                                  z64* __restrict__ G, z64* __restrict__ F, int* __restrict__ piv,
@@ -201,7 +201,7 @@ __global__ void __launch_bounds__(256) k_gj_first(int n, int w, const z64* __res
 // x_j = in(p_j, c) - sum_{k<j} F(p_j, k) x_k, and p_j itself enters the sum from its own step on.  One wave per
 // workgroup and 32 x 32 tile, the recursion of its 32 columns on as many lanes (both halves of the wave alike), the
 // products' operands from L2 and LDS (inner size 16: four k of each MFMA, four MFMAs).  Bound by latency: every tile
-// is in flight at once.
+// is in flight at once (n = 1080: 25 us, 21 with the product by G, whose error grows with the pivot block).
 __global__ void __launch_bounds__(64) k_gj_update(int n, int c0, int w, const z64* __restrict__ in,
                                                   const z64* __restrict__ G, const z64* __restrict__ F,
                                                   const int* __restrict__ piv, const int* __restrict__ pos,

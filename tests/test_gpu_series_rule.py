@@ -54,13 +54,6 @@ def test_gpu_series_slow_point_in_a_small_batch(precision):
     assert st["n_lu_launches"] == 1
 
 
-def test_gpu_series_leaves_the_smallest_refined_systems_to_the_lu():
-    """N = 40: a complex64 LU costs about three steps."""
-    wl = _workload(1, (8, 8, 8), 20, 0.01)
-    assert _run(wl, 512, "refined")[1]["n_lu_launches"] == 1
-    assert _run(wl, 512, "fp64")[1]["n_lu_launches"] == 0
-
-
 @pytest.mark.parametrize("n,nk,iwf,npts,noise", [(1, (4, 4, 4), 200, 64, 0.4), (1, (4, 4, 4), 200, 64, 0.5),
                                                  (3, (4, 4, 3), 30, 41, 0.4), (3, (4, 4, 4), 60, 16, 0.5)])
 def test_gpu_series_refined_accuracy_at_slow_contraction(n, nk, iwf, npts, noise):
