@@ -266,12 +266,17 @@ struct SolveCost {
   SolveCost(const Geom& g, int nb, int prec, bool vq) {
     const double N = g.N, rate = std::min(47e9, 6e7 * N);  // flops per ms in complex128
     product = 16 * N * N * g.n2 * nb / 55e9;
-    step = (vq ? 0.055 : 0.02) + product;
+    step = 0.016 + 0.0018 * g.n2 + (vq ? 0.035 : 0.0) + product;
     latency = 1e-3 * N * std::min(10.0, 4 + N / 180);
     per_point = 16 / 3.0 * N * N * N / rate;
     lu = prec == 0 ? latency + nb * per_point : 0.75 * latency + nb * per_point / 1.9 + 2 * step;
   }
   double singles(int n) const { return (n + 31) / 32 * latency + n * per_point; }
+  // steps of each of `solves` iterations that cost no more than one factorisation and as many solves with it, which
+  // read the factors once each; with 50% to spare, as series_steps() has on the whole
+  int shared_steps(const Geom& g, int nb, int solves) const {
+    return (int)(1.5 * (lu / solves + 32.0 * nb * g.N * g.N / 3e9) / step);
+  }
 };
 
 // Workspace of solve_fp64, sized for the largest box (c->g): one point, or with `full` at most 4 GB of complex128
@@ -460,8 +465,10 @@ bool series_solve(adga_ctx* c, int nb, const SeriesGoal& goal, const z64* B, z64
   const Geom& g = c->gw;
   hipStream_t s = c->stream;
   const double accept = goal.accept;
-  const int kmax = series_steps(g);
   const SolveCost cost(g, nb, goal.prec, c->vq != nullptr);
+  const int most = series_steps(g);
+  const int kmax = goal.solves > 1 ? std::min(most, cost.shared_steps(g, nb, goal.solves)) : most;
+  if (kmax < 1) return false;
   const adga::VqTerm vt{c->W, c->opgd, c->vqQ};
   const adga::VqTerm* vtp = c->vq ? &vt : nullptr;
   std::vector<double> rho(2 * nb, 0.0), prev;
@@ -885,7 +892,7 @@ int run_points_impl(adga_ctx* c, int npts, const int* iq, int precision, double*
       const double tol = prec == 0 ? SERIES_TOL64 : std::min(c->refine_tol, 1e-6);
       int steps = 0;
       // the derivatives and the option "fallback" off need the factors of every point or of none
-      const SeriesGoal goal{prec, tol, prec == 0 ? SERIES_ACCEPT64 : tol, !tan && c->fallback};
+      const SeriesGoal goal{prec, tol, prec == 0 ? SERIES_ACCEPT64 : tol, !tan && c->fallback, tan ? 1 + c->ndir : 1};
       const bool series =
           lu_ok && c->series && tol >= SERIES_TOL64 && series_solve(c, nb, goal, c->Bp, c->Y, relh, left, &steps);
       if (series) {

@@ -107,7 +107,7 @@ void tangent_batch(adga_ctx* c, int nb, int p0, int npts, const std::vector<int>
     if (!factored) {
       relh.assign(nmat, 0.0);
       infoh.assign(nmat, 0);
-      const SeriesGoal goal{0, SERIES_TOL64, SERIES_ACCEPT64, false};
+      const SeriesGoal goal{0, SERIES_TOL64, SERIES_ACCEPT64, false, c->ndir - dir};
       const bool iterated = c->series && series_solve(c, nb, goal, c->t_B, c->t_dY, relh, left);
       if (!iterated && ensure_lu(c, nb)) {
         if (!factor_fp64(c, nb)) throw HipError{hipErrorInvalidValue, "tangent solve: BSE size outside the LU's range"};

@@ -267,6 +267,7 @@ struct SeriesGoal {
   int prec;
   double tol, accept;
   bool singles;
+  int solves = 1;  // right-hand sides that one factorisation would serve: the forward one and each direction's
   // The residual to aim at where each step leaves rho of it.  The refined mode's solution is to be as accurate as
   // a complex64 LU leaves it, whose last correction as a rule falls far below the tolerance: the error, up to
   // r rho / (1 - rho) after the last step, stays within a tenth of it (N = 1080, rho = 0.43: chi's largest relative

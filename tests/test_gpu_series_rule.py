@@ -113,3 +113,22 @@ def test_gpu_batch_dependence(precision, noise):
                 else:
                     err = np.abs(a - b).max() / np.abs(b).max()
                     assert err < (1e-12 if precision == "fp64" else 1e-11)
+
+
+def test_gpu_derivatives_share_one_factorisation():
+    """N = 100, five orbitals: the forward solve iterates, but four solves by iteration cost more than one LU and four
+    solves with its factors."""
+    from adga_amd import api
+    wl = _workload(5, (4, 4, 4), 2, 1e-3)
+    inp = synth.build_inputs(wl)
+    tan = synth.tangents(inp)
+    iq = np.arange(1, 63, dtype=np.int32)
+    print("one factorisation for all directions", flush=True)
+    with api.Context(inp, batch=62) as ctx:
+        ctx.set_tangents(tan)
+        ctx.set_local_omega(0, *[synth.chi_loc(inp, 0, c) for c in ("dens", "magn")])
+        ctx.set_local_omega_tangent(*[synth.dchi_loc(inp, tan, 0) for _ in range(2)])
+        ctx.run_points(iq, "fp64")
+        assert ctx.stats()["n_lu_launches"] == 0
+        ctx.run_points_tangent(iq)
+        assert ctx.stats()["n_lu_launches"] == 1
